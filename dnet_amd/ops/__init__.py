@@ -148,19 +148,24 @@ def dequant_int8(w: torch.Tensor, scales: torch.Tensor, group: int,
 
 
 def _attn_splits(b: int, hkv: int, smax: int) -> int:
-    # fill ~1024 blocks (4/CU); cap so each split owns >= ~512 positions of
-    # capacity (short actual sequences leave idle splits + combine overhead)
+    """How many workgroups may share one (row, kv head)'s positions. The
+    kernel uses as many of them as the row's length is worth.
+
+    Up to 1024 workgroups (4 per CU, what fits at once): beyond, the extra
+    partials cost more than the shorter spans give (64 heads of 1000 to 8000
+    positions: 39 us at 8 or 16 splits, 42 at 64). Each split has to own 128
+    positions of the capacity (one step of its 4 waves), or 1024 where the
+    (row, head) pairs alone give every CU a workgroup: 256 pairs at 500 to
+    1000 positions 22.6 us in one piece, 26.3 in two; 8 pairs at 8000
+    positions 88 us in one piece, 15 in 32."""
     import os
     force = os.environ.get("DNET_ATTN_SPLITS")
     if force:
         return max(1, int(force))
+    base = b * hkv
+    cap = min(32, smax // (128 if base < 256 else 1024))
     splits = 1
-    cap = max(1, smax // 512)
-    # target ~2048 blocks (8/CU): measured at 2k ctx batch 32 (qwen-32b,
-    # 512 base blocks) splits=4 runs 21.5 ms/step vs 27.2 at splits=2 —
-    # serial chunks per block hurt more than combine overhead until the
-    # per-split span drops under ~512 positions (the cap)
-    while (b * hkv * splits * 2 <= 2048 and splits * 2 <= cap):
+    while base * splits * 2 <= 1024 and splits * 2 <= cap:
         splits *= 2
     return splits
 

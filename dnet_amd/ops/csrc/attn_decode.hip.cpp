@@ -2,13 +2,43 @@
 //
 //   out[b,h,:] = softmax(q[b,h,:] . K[b,kv(h),:len,:]^T * scale) @ V[b,kv(h),:len,:]
 //
-// One workgroup per (batch, kv_head): the K/V read — the memory bound — is
-// staged through LDS once and shared by all query heads of the group and all
-// 4 waves. Online softmax (flash-decode style) over 64-position chunks;
-// per-lane layout: score phase = one seq position per lane, accumulate
-// phase = D/64 output dims per lane with the softmax weight broadcast by
-// shuffle. Sequence length comes from a device tensor (`pos`) so the kernel
-// is hipGraph-replayable across decode steps without recapture.
+// The read of the cache bounds it; everything else has to stay out of the
+// way of the loads. One workgroup of 4 waves per (batch row, kv head, split)
+// and each wave on its own: it takes every 4th tile of 32 positions, keeps its
+// own online softmax and never waits for another wave before the one merge at
+// the end.
+//   * K goes from memory straight into the registers in the A layout of
+//     v_mfma_f32_16x16x32_bf16 (16 positions x 32 dims), q (the up to 16 query
+//     heads of the group) is the B operand: scores^T [position][head].
+//   * In C layout a lane holds 4 positions of one head, and over two 16-row
+//     tiles exactly the 8 positions that the B operand of the value product
+//     wants from it (the order of the contraction index is free as long as V
+//     follows it): the weights never cross lanes.
+//   * V rows pass through a wave-private LDS tile and come back transposed by
+//     ds_read_b64_tr_b16 (4 positions of one dim per lane). Pitch DV + 16
+//     halves: the 8 rows that half a wave reads at once fall into different
+//     banks.
+//   * The next tile's loads are issued as soon as the registers are free
+//     (before the softmax), 16 KB in flight per wave.
+// Softmax weights are fp32; the matrix core takes them as two bf16 parts
+// (16 significant bits), so the value product is as exact as fp32 weights
+// against bf16 values. An int8 cache is multiplied as whole numbers (exact in
+// bf16) and scaled in fp32.
+//
+// Sequence length comes from a device tensor (`pos`), so the kernel is
+// hipGraph-replayable; how many of the launched splits work is decided from
+// it on the device (at least `min_span` positions each), the others leave at
+// once.
+//
+// Measured, MI355X, D 128, with the combine, before (one thread per position
+// on packed dot products, both tiles staged for the whole workgroup) -> now:
+// 32 rows of 1500 to 8000 positions x 8 kv heads (622 MB, 4 query heads each)
+// 270 -> 126 us (5.0 TB/s); 13 rows of 900 to 4000, int8 cache (67 MB, 5
+// heads) 113 -> 25 us; 8 rows of 50 to 1900 (32 MB) 55 -> 14 us; one row of
+// 701 positions 20 -> 8 us. Error against 64 bits: that of the bf16 result
+// (int8 cache: 3.4e-3 -> 1.7e-3, its keys and values are no longer rounded to
+// bf16). At 3 waves per SIMD (168 registers) the int8 form gains a tenth over
+// 2, the bf16 one nothing; head size 192 would spill there.
 //
 // Replaces the reference's MLX scaled_dot_product_attention decode path
 // (reference: src/dnet/core/models/llama.py apply_single_layer).
@@ -16,517 +46,326 @@
 
 namespace dnet {
 
-// Row pitch in bf16 elements for a D-wide LDS tile such that the per-lane
-// column reads are bank-conflict-free (pitch in dwords must be ≡ 2 mod 4
-// and 8B-aligned; 66 dwords for D=128 → 2l mod 64 distinct per 32-lane group).
-__device__ __host__ __forceinline__ constexpr int lds_pitch(int D) {
-  return D + 4;  // bf16 elems; D=128 -> 264 B = 66 dwords; D=64 -> 136 B = 34 dwords
-}
-
-__device__ __forceinline__ float wave_allreduce_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-__device__ __forceinline__ float wave_allreduce_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
-}
-
-constexpr int kChunk = 64;
-
 using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
-using bf16x2 = __attribute__((ext_vector_type(2))) __bf16;
+using s16x4 = __attribute__((ext_vector_type(4))) short;
+using s16x8 = __attribute__((ext_vector_type(8))) short;
 using f32x4 = __attribute__((ext_vector_type(4))) float;
+using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
 
-// splits > 1: flash-decode S-partitioning — gridDim.y splits each take
-// chunks c = c0 + split, c0 + split + splits, ...; unnormalized partials
-// (acc, m, l) go to scratch [B, Hq, splits, D+2] f32 and a combine kernel
-// merges them (sink logit folded there). Raises the block count from
-// B*Hkv to B*Hkv*splits so small batches still fill 256 CUs.
-template <int D, int DV, bool Q8>
-__global__ void attn_decode_kernel(const short* __restrict__ q,
-                                   const void* __restrict__ kc,
-                                   const void* __restrict__ vc,
-                                   const short* __restrict__ kscale,
-                                   const short* __restrict__ vscale,
-                                   const int* __restrict__ pos,
-                                   short* __restrict__ out, const int Hq,
-                                   const int Hkv, const int Smax,
-                                   const float scale, const int ldq,
-                                   const int window,
-                                   const short* __restrict__ sinks,
-                                   float* __restrict__ partials,
-                                   const int splits) {
-  constexpr int P = lds_pitch(D);
-  constexpr int PV = lds_pitch(DV);
-  constexpr int DPL = DV / kWave;  // output dims per lane (1 or 2)
-  const int b = blockIdx.x / Hkv;
-  const int hkv = blockIdx.x % Hkv;
-  const int G = Hq / Hkv;  // query heads per kv head
-  const int wid = threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
+constexpr int kTile = 32;   // positions of a wave's step
 
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  short* k_lds = reinterpret_cast<short*>(smem);               // [kChunk][P]
-  short* v_lds = k_lds + kChunk * P;                           // [kChunk][PV]
-  short* q_lds = v_lds + kChunk * PV;                          // [G][D]
-  float* p_lds = reinterpret_cast<float*>(q_lds + ((G * D + 7) & ~7));
-  // p_lds: [4 waves][kChunk] exp'd scores — LDS broadcast reads replace
-  // the per-iteration __shfl (long dependency chain). (An f32 V tile
-  // was measured: the +17 KB LDS costs a block/CU of occupancy and
-  // LOSES 13% at 2k ctx — V stays bf16.)
+// how many splits share a row's positions (same rule in the combine)
+__device__ __forceinline__ int active_splits(int span, int splits,
+                                             int min_span) {
+  return max(1, min(splits, (span + min_span - 1) / min_span));
+}
 
-  const int len = pos[b];
-  const int start = (window > 0) ? max(0, len - window) : 0;  // sliding
-  const int64_t kvbase = ((int64_t)b * Hkv + hkv) * Smax * D;
-  const int64_t vbase = ((int64_t)b * Hkv + hkv) * Smax * DV;
-
-  // Stage this group's q rows.
-  for (int i = threadIdx.x; i < G * D / 8; i += blockDim.x) {
-    const int g = i / (D / 8);
-    reinterpret_cast<short8*>(q_lds)[i] =
-        reinterpret_cast<const short8*>(q + (int64_t)b * ldq + (hkv * G + g) * D)[i % (D / 8)];
+// 8 int8 codes -> bf16 (exact)
+__device__ __forceinline__ bf16x8 codes8(const int lo, const int hi) {
+  bf16x8 b;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    b[j] = (__bf16)(float)(signed char)(lo >> (8 * j));
+    b[4 + j] = (__bf16)(float)(signed char)(hi >> (8 * j));
   }
+  return b;
+}
 
-  // Per-wave head list: g = wid, wid+4, ... (max 4 heads per wave).
-  float m[4], l[4], acc[4][DPL];
-  const int nh = (G - wid + 3) / 4;
+// p -> hi + lo, each bf16
+__device__ __forceinline__ void split8(const float* p, bf16x8& hi, bf16x8& lo) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    m[i] = -1e30f;
-    l[i] = 0.f;
-#pragma unroll
-    for (int j = 0; j < DPL; ++j) acc[i][j] = 0.f;
-  }
-  __syncthreads();
-
-  const int nchunks = (len + kChunk - 1) / kChunk;
-  const int split = blockIdx.y;
-  for (int c = start / kChunk + split; c < nchunks; c += splits) {
-    const int s0 = c * kChunk;
-    const int valid = min(kChunk, len - s0);
-    // Stage K and V chunk into bf16 LDS; Q8 caches dequantize while staging
-    // (HBM reads stay int8 — half the KV bandwidth).
-    for (int i = threadIdx.x; i < kChunk * D / 8; i += blockDim.x) {
-      const int row = i / (D / 8);
-      const int col = (i % (D / 8)) * 8;
-      short8 kv8;
-      if (row < valid) {
-        if (Q8) {
-          constexpr int NG = D / 64;
-          const int64_t rb = kvbase / D * (int64_t)NG
-                             + (int64_t)(s0 + row) * NG + col / 64;
-          const float ks = bits2f(kscale[rb]);
-          const int2 kq = *reinterpret_cast<const int2*>(
-              (const int8_t*)kc + kvbase + (int64_t)(s0 + row) * D + col);
-          const int8_t* kb = reinterpret_cast<const int8_t*>(&kq);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) kv8.x[j] = f2bits((float)kb[j] * ks);
-        } else {
-          kv8 = *reinterpret_cast<const short8*>(
-              (const short*)kc + kvbase + (int64_t)(s0 + row) * D + col);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) kv8.x[j] = 0;
-      }
-      *reinterpret_cast<short8*>(&k_lds[row * P + col]) = kv8;
-    }
-    for (int i = threadIdx.x; i < kChunk * DV / 8; i += blockDim.x) {
-      const int row = i / (DV / 8);
-      const int col = (i % (DV / 8)) * 8;
-      short8 vv8;
-      if (row < valid) {
-        if (Q8) {
-          constexpr int NGV = DV / 64;
-          const int64_t rb = vbase / DV * (int64_t)NGV
-                             + (int64_t)(s0 + row) * NGV + col / 64;
-          const float vs = bits2f(vscale[rb]);
-          const int2 vq = *reinterpret_cast<const int2*>(
-              (const int8_t*)vc + vbase + (int64_t)(s0 + row) * DV + col);
-          const int8_t* vb = reinterpret_cast<const int8_t*>(&vq);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) vv8.x[j] = f2bits((float)vb[j] * vs);
-        } else {
-          vv8 = *reinterpret_cast<const short8*>(
-              (const short*)vc + vbase + (int64_t)(s0 + row) * DV + col);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) vv8.x[j] = 0;
-      }
-      *reinterpret_cast<short8*>(&v_lds[row * PV + col]) = vv8;
-    }
-    __syncthreads();
-
-    for (int hi = 0; hi < nh; ++hi) {
-      const int g = wid + hi * 4;
-      // Score for position s = lane (packed bf16 dot2: one VALU per
-      // 2 dims instead of 2 converts + 2 fmas).
-      float s_val = 0.f;
-      const short* krow = &k_lds[lane * P];
-      const short* qrow = &q_lds[g * D];
-      for (int d = 0; d < D; d += 4) {
-        const short4v kq = *reinterpret_cast<const short4v*>(&krow[d]);
-        const short4v qq = *reinterpret_cast<const short4v*>(&qrow[d]);
-        s_val = __builtin_amdgcn_fdot2_f32_bf16(
-            *reinterpret_cast<const bf16x2*>(&kq.x[0]),
-            *reinterpret_cast<const bf16x2*>(&qq.x[0]), s_val, false);
-        s_val = __builtin_amdgcn_fdot2_f32_bf16(
-            *reinterpret_cast<const bf16x2*>(&kq.x[2]),
-            *reinterpret_cast<const bf16x2*>(&qq.x[2]), s_val, false);
-      }
-      s_val *= scale;
-      const bool in_win = (lane < valid) && (s0 + lane >= start);
-      if (!in_win) s_val = -1e30f;
-      // Online softmax update.
-      const float cmax = wave_allreduce_max(s_val);
-      const float mn = fmaxf(m[hi], cmax);
-      const float alpha = __expf(m[hi] - mn);
-      const float p = in_win ? __expf(s_val - mn) : 0.f;
-      l[hi] = l[hi] * alpha + wave_allreduce_sum(p);
-      m[hi] = mn;
-#pragma unroll
-      for (int j = 0; j < DPL; ++j) acc[hi][j] *= alpha;
-      // Accumulate P @ V: lane owns dims d = DPL*lane + j; p comes
-      // from a per-wave LDS slab (broadcast reads — no serial __shfl
-      // dependency chain)
-      p_lds[wid * kChunk + lane] = p;
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // wave-local
-      for (int s = 0; s < valid; ++s) {
-        const float ps = p_lds[wid * kChunk + s];
-        const short* vrow = &v_lds[s * PV + DPL * lane];
-#pragma unroll
-        for (int j = 0; j < DPL; ++j)
-          acc[hi][j] = fmaf(ps, bits2f(vrow[j]), acc[hi][j]);
-      }
-    }
-    __syncthreads();
-  }
-
-  if (partials != nullptr) {
-    // write unnormalized partials; the combine kernel (or a cross-rank
-    // context-parallel combine) normalizes + folds sinks
-    for (int hi = 0; hi < nh; ++hi) {
-      const int g = wid + hi * 4;
-      float* prow = partials
-          + (((int64_t)b * Hq + hkv * G + g) * splits + split) * (DV + 2);
-#pragma unroll
-      for (int j = 0; j < DPL; ++j) prow[DPL * lane + j] = acc[hi][j];
-      if (lane == 0) {
-        prow[DV] = m[hi];
-        prow[DV + 1] = l[hi];
-      }
-    }
-    return;
-  }
-  for (int hi = 0; hi < nh; ++hi) {
-    const int g = wid + hi * 4;
-    float inv;
-    if (sinks != nullptr) {
-      // gpt-oss attention sink: one extra learned softmax logit per q head
-      // whose probability mass is dropped from the output.
-      const float sk = bits2f(sinks[hkv * G + g]);
-      const float mx = fmaxf(m[hi], sk);
-      const float num = __expf(m[hi] - mx);
-      const float denom = l[hi] * num + __expf(sk - mx);
-      inv = (denom > 0.f) ? num / denom : 0.f;
-    } else {
-      inv = (l[hi] > 0.f) ? 1.f / l[hi] : 0.f;
-    }
-    short* orow = out + ((int64_t)b * Hq + hkv * G + g) * DV + DPL * lane;
-#pragma unroll
-    for (int j = 0; j < DPL; ++j) orow[j] = f2bits(acc[hi][j] * inv);
+  for (int j = 0; j < 8; ++j) {
+    const __bf16 h = (__bf16)p[j];
+    hi[j] = h;
+    lo[j] = (__bf16)(p[j] - (float)h);
   }
 }
 
-
-// ---------------------------------------------------------------------------
-// MFMA decode attention: same contract as attn_decode_kernel, compute
-// reshaped for the matrix cores. The G (<=16) query heads of a
-// (batch, kv-head) group form the 16-row A operand; each of the 4 waves
-// owns a 16-position subtile of every 64-position chunk and keeps an
-// INDEPENDENT online-softmax state (m, l, acc) — position space is
-// fully partitioned across waves, so there is no per-chunk cross-wave
-// synchronization at all, just one merge at the end (intra-block
-// flash-decode split). Scores = Q[16,D] x K^T via v_mfma_f32_16x16x32,
-// P@V via the same MFMA with the per-wave P slab zero-padded to k=32.
-// Replaces a serial 64-iteration __shfl broadcast loop per (head,
-// chunk) in the scalar kernel (~26us -> ~14us per layer at batch 64,
-// and the win grows with context).
 template <int D, int DV, bool Q8>
-__global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
+__global__ __launch_bounds__(256, D == 192 ? 2 : 3) void attn_decode_kernel(
     const short* __restrict__ q, const void* __restrict__ kc,
     const void* __restrict__ vc, const short* __restrict__ kscale,
     const short* __restrict__ vscale, const int* __restrict__ pos,
     short* __restrict__ out, const int Hq, const int Hkv, const int Smax,
     const float scale, const int ldq, const int window,
     const short* __restrict__ sinks, float* __restrict__ partials,
-    const int splits) {
-  constexpr int DC = D / 32;   // QK k-chunks
-  constexpr int NV = DV / 16;  // PV n-tiles
-  constexpr int KP = D + 8;    // k_lds row pitch (16-lane frags bank-clean)
-  constexpr int VP = 88;       // vt_lds pitch: covers the k<=79 overread of
-                               // wave 3 (zero-P columns) and 44-dword row
-                               // stride hits all banks across 16 rows
-  constexpr int SP = 40;       // per-wave P slab pitch
-  constexpr int STAGE = 64 * KP * 2 + DV * VP * 2;
-  static_assert(STAGE >= 4 * 16 * DV * 4 + 4 * 16 * 2 * 4,
-                "merge area must fit in the staging LDS");
-  __shared__ __attribute__((aligned(16))) char smem[STAGE];
-  __shared__ short p_lds[4][16 * SP];
-  short* k_lds = reinterpret_cast<short*>(smem);
-  short* vt_lds = reinterpret_cast<short*>(smem + 64 * KP * 2);
+    const int splits, const int min_span, const bool combine) {
+  constexpr int DC = D / 32;         // contraction chunks of the scores
+  constexpr int NV = DV / 16;        // 16-dim blocks of the values
+  constexpr int VP = DV + 16;        // LDS pitch of a V row
+  constexpr int KL = Q8 ? D / 64 : D / 32;     // 16 B loads per K row and lane
+  constexpr int VL = Q8 ? DV / 32 : DV / 16;   // 16 B loads per V tile and lane
+  constexpr int NG = D / 64, NGV = DV / 64;    // scale groups of a row
+  constexpr int VE = Q8 ? 16 : 8;              // elements of a 16 B load
+  __shared__ __attribute__((aligned(16))) short smem[4 * kTile * VP];
+  static_assert(sizeof(smem) >= 4 * 16 * (DV + 2) * 4, "merge area");
 
   const int b = blockIdx.x / Hkv;
   const int hkv = blockIdx.x % Hkv;
   const int G = Hq / Hkv;
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  const int row = lane & 15;
+  const int c16 = lane & 15;
   const int hi = lane >> 4;
-  const int len = pos[b];
+  const int len = min(pos[b], Smax);
   const int start = (window > 0) ? max(0, len - window) : 0;
-  const int64_t kvbase = ((int64_t)b * Hkv + hkv) * Smax * D;
-  const int64_t vbase = ((int64_t)b * Hkv + hkv) * (int64_t)Smax * DV;
+  const int split = blockIdx.y;
+  const int nact = active_splits(len - start, splits, min_span);
+  if (split >= nact) return;
 
-  // Q fragments (A layout: lane holds Q[head=row][c*32 + hi*8 .. +8]);
-  // rows >= G duplicate head G-1 — their outputs are never stored and
-  // softmax is per-row, so they cannot contaminate real heads
-  const short* qp = q + (int64_t)b * ldq + (int64_t)(hkv * G + min(row, G - 1)) * D;
+  const int64_t row0 = ((int64_t)b * Hkv + hkv) * Smax;
+  const char* kbase = (const char*)kc + row0 * D * (Q8 ? 1 : 2);
+  const char* vbase = (const char*)vc + row0 * DV * (Q8 ? 1 : 2);
+  short* vt = smem + wave * kTile * VP;
+
+  // q in B layout: lane holds head c16 (rows past the group repeat its last
+  // head; what they give is never stored). int8: a 16 B load of codes covers
+  // 16 dims of a 64-dim group, so the contraction runs in that order
+  const short* qp =
+      q + (int64_t)b * ldq + (int64_t)(hkv * G + min(c16, G - 1)) * D;
   bf16x8 qf[DC];
 #pragma unroll
   for (int c = 0; c < DC; ++c)
-    qf[c] = *reinterpret_cast<const bf16x8*>(&qp[c * 32 + hi * 8]);
+    qf[c] = *reinterpret_cast<const bf16x8*>(
+        Q8 ? &qp[(c >> 1) * 64 + hi * 16 + (c & 1) * 8] : &qp[c * 32 + hi * 8]);
 
   f32x4 acc[NV];
 #pragma unroll
   for (int n = 0; n < NV; ++n) acc[n] = {0.f, 0.f, 0.f, 0.f};
-  float m_run[4], l_run[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    m_run[r] = -1e30f;
-    l_run[r] = 0.f;
-  }
+  float m = -1e30f, l = 0.f;   // l: this lane's positions only
 
-  // zero this wave's dead P columns (k = 16..31) once: the PV MFMA runs
-  // k=32 and the upper half multiplies whatever V rows it overreads
-  for (int i = lane; i < 16 * 16; i += 64)
-    p_lds[wave][(i >> 4) * SP + 16 + (i & 15)] = 0;
-  // zero vt's never-staged tail columns (s = 64..VP-1) once: wave 3's
-  // k>=16 B-fragment overreads them, and uninitialized LDS bits can be
-  // NaN — NaN * 0 is NaN, which would poison the accumulators
-  for (int i = threadIdx.x; i < DV * (VP - 64); i += 256)
-    vt_lds[(i / (VP - 64)) * VP + 64 + i % (VP - 64)] = 0;
-
-  const int nchunks = (len + kChunk - 1) / kChunk;
-  const int split = blockIdx.y;
-  for (int c = start / kChunk + split; c < nchunks; c += splits) {
-    const int s0 = c * kChunk;
-    const int valid = min(kChunk, len - s0);
-    __syncthreads();   // previous tile's consumers done
-    for (int i = threadIdx.x; i < kChunk * (D / 8); i += blockDim.x) {
-      const int sr = i / (D / 8);
-      const int col = (i % (D / 8)) * 8;
-      short8 kv8;
-      if (sr < valid) {
-        if (Q8) {
-          constexpr int NG = D / 64;
-          const int64_t rb = kvbase / D * (int64_t)NG
-                             + (int64_t)(s0 + sr) * NG + col / 64;
-          const float ks = bits2f(kscale[rb]);
-          const int2 kq = *reinterpret_cast<const int2*>(
-              (const int8_t*)kc + kvbase + (int64_t)(s0 + sr) * D + col);
-          const int8_t* kb = reinterpret_cast<const int8_t*>(&kq);
+  u32x4 kr[2][KL], vr[VL];
+  // rows past the end repeat the last one: in range, finite, masked below
+  auto load = [&](const int t) {
+    const int s0 = t * kTile;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) kv8.x[j] = f2bits((float)kb[j] * ks);
-        } else {
-          kv8 = *reinterpret_cast<const short8*>(
-              (const short*)kc + kvbase + (int64_t)(s0 + sr) * D + col);
+    for (int h = 0; h < 2; ++h) {
+      const int row = min(s0 + h * 16 + c16, len - 1);
+#pragma unroll
+      for (int c = 0; c < KL; ++c)
+        kr[h][c] = *reinterpret_cast<const u32x4*>(
+            kbase + (int64_t)row * (D * (Q8 ? 1 : 2)) + c * 64 + hi * 16);
+    }
+#pragma unroll
+    for (int i = 0; i < VL; ++i) {
+      const int e = i * 64 + lane;
+      const int row = min(s0 + e / (DV / VE), len - 1);
+      vr[i] = *reinterpret_cast<const u32x4*>(
+          vbase + (int64_t)row * (DV * (Q8 ? 1 : 2)) + (e % (DV / VE)) * 16);
+    }
+  };
+
+  const int tend = (len + kTile - 1) / kTile;
+  int t = start / kTile + split * 4 + wave;
+  if (t < tend) load(t);
+  for (; t < tend; t += nact * 4) {
+    const int s0 = t * kTile;
+    // V tile into LDS (row-major, wave-private: LDS keeps a wave's order)
+#pragma unroll
+    for (int i = 0; i < VL; ++i) {
+      const int e = i * 64 + lane;
+      short* dst = &vt[(e / (DV / VE)) * VP + (e % (DV / VE)) * VE];
+      if (Q8) {
+        *reinterpret_cast<bf16x8*>(dst) = codes8(vr[i].x, vr[i].y);
+        *reinterpret_cast<bf16x8*>(dst + 8) = codes8(vr[i].z, vr[i].w);
+      } else {
+        *reinterpret_cast<u32x4*>(dst) = vr[i];
+      }
+    }
+    f32x4 sc[2];
+    float ks[2][4][NG], vs[2][4][NGV];
+    if (Q8) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int64_t row =
+              row0 + min(s0 + h * 16 + hi * 4 + r, len - 1);
+#pragma unroll
+          for (int g = 0; g < NG; ++g) ks[h][r][g] = bits2f(kscale[row * NG + g]);
+#pragma unroll
+          for (int g = 0; g < NGV; ++g)
+            vs[h][r][g] = bits2f(vscale[row * NGV + g]);
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      sc[h] = {0.f, 0.f, 0.f, 0.f};
+      if (Q8) {
+#pragma unroll
+        for (int c = 0; c < KL; ++c) {
+          f32x4 part = {0.f, 0.f, 0.f, 0.f};
+          part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              codes8(kr[h][c].x, kr[h][c].y), qf[2 * c], part, 0, 0, 0);
+          part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              codes8(kr[h][c].z, kr[h][c].w), qf[2 * c + 1], part, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            sc[h][r] = fmaf(ks[h][r][c], part[r], sc[h][r]);
         }
       } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) kv8.x[j] = 0;
+        for (int c = 0; c < DC; ++c)
+          sc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, kr[h][c]), qf[c], sc[h], 0, 0, 0);
       }
-      *reinterpret_cast<short8*>(&k_lds[sr * KP + col]) = kv8;
     }
-    // V transposed [dv][s] so the PV B-fragment reads are contiguous;
-    // global side reads full short8 rows (the 8 scattered 2 B LDS
-    // stores are cheap, 4 B global loads were not)
-    for (int i = threadIdx.x; i < kChunk * (DV / 8); i += blockDim.x) {
-      const int sr = i / (DV / 8);
-      const int dc = (i % (DV / 8)) * 8;
-      short8 vv8;
-      if (sr < valid) {
-        if (Q8) {
-          constexpr int NGV = DV / 64;
-          const int64_t rb = vbase / DV * (int64_t)NGV
-                             + (int64_t)(s0 + sr) * NGV + dc / 64;
-          const float vs = bits2f(vscale[rb]);
-          const int2 vq = *reinterpret_cast<const int2*>(
-              (const int8_t*)vc + vbase + (int64_t)(s0 + sr) * DV + dc);
-          const int8_t* vb = reinterpret_cast<const int8_t*>(&vq);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) vv8.x[j] = f2bits((float)vb[j] * vs);
-        } else {
-          vv8 = *reinterpret_cast<const short8*>(
-              (const short*)vc + vbase + (int64_t)(s0 + sr) * DV + dc);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) vv8.x[j] = 0;
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) vt_lds[(dc + j) * VP + sr] = vv8.x[j];
-    }
-    __syncthreads();
+    const int tn = t + nact * 4;
+    if (tn < tend) load(tn);
 
-    // scores for this wave's 16 positions: C[head=hi*4+r][pos col=row]
-    f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+    // online softmax of head c16 over this lane's 8 positions and the three
+    // other lanes of the head
+    float p[8];
+    bool ok[8];
+    float mx = -1e30f;
 #pragma unroll
-    for (int cc = 0; cc < DC; ++cc) {
-      const bf16x8 kf = *reinterpret_cast<const bf16x8*>(
-          &k_lds[(wave * 16 + row) * KP + cc * 32 + hi * 8]);
-      sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[cc], kf, sc, 0, 0, 0);
+    for (int j = 0; j < 8; ++j) {
+      const int sp = s0 + (j >> 2) * 16 + hi * 4 + (j & 3);
+      ok[j] = sp < len && sp >= start;
+      p[j] = ok[j] ? sc[j >> 2][j & 3] * scale : -1e30f;
+      mx = fmaxf(mx, p[j]);
     }
-    const int spos = s0 + wave * 16 + row;
-    const bool dead = (spos >= len) || (spos < start);
-    float pv[4];
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mn = fmaxf(m, mx);
+    if (__any(mn > m)) {
+      const float alpha = __expf(m - mn);
+      l *= alpha;
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      pv[r] = dead ? -INFINITY : sc[r] * scale;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float mx = pv[r];
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1)
-        mx = fmaxf(mx, __shfl_xor(mx, off, 16));
-      const float mn = fmaxf(m_run[r], mx);
-      const float corr = __expf(m_run[r] - mn);
-      pv[r] = __expf(pv[r] - mn);   // -inf underflows to exactly 0
-      float ls = pv[r];
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1)
-        ls += __shfl_xor(ls, off, 16);
-      l_run[r] = l_run[r] * corr + ls;
-      m_run[r] = mn;
-#pragma unroll
-      for (int n = 0; n < NV; ++n) acc[n][r] *= corr;
+      for (int n = 0; n < NV; ++n) acc[n] *= alpha;
     }
-    // P slab (cols 0..15 = this wave's positions), then PV
+    m = mn;
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      p_lds[wave][(hi * 4 + r) * SP + row] = f2bits(pv[r]);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // wave-local slab
+    for (int j = 0; j < 8; ++j) {
+      p[j] = ok[j] ? __expf(p[j] - mn) : 0.f;
+      l += p[j];
+    }
+    bf16x8 phi[Q8 ? NGV : 1], plo[Q8 ? NGV : 1];
+    if (Q8) {
+#pragma unroll
+      for (int g = 0; g < NGV; ++g) {
+        float ps[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ps[j] = p[j] * vs[j >> 2][j & 3][g];
+        split8(ps, phi[g], plo[g]);
+      }
+    } else {
+      split8(p, phi[0], plo[0]);
+    }
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
-      const bf16x8 pf =
-          *reinterpret_cast<const bf16x8*>(&p_lds[wave][row * SP + hi * 8]);
-      const bf16x8 vf = *reinterpret_cast<const bf16x8*>(
-          &vt_lds[(n * 16 + row) * VP + wave * 16 + hi * 8]);
-      acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, vf, acc[n], 0, 0,
+      // positions h*16 + hi*4 + 0..3 of dim n*16 + c16, h = 0, 1
+      s16x8 vf;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const s16x4 part = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)&vt
+                [(h * 16 + hi * 4 + (c16 >> 2)) * VP + n * 16 + (c16 & 3) * 4]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vf[h * 4 + r] = part[r];
+      }
+      const bf16x8 v8 = __builtin_bit_cast(bf16x8, vf);
+      const int g = Q8 ? n / 4 : 0;
+      acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, phi[g], acc[n], 0, 0,
+                                                       0);
+      acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, plo[g], acc[n], 0, 0,
                                                        0);
     }
   }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
 
-  // ---- cross-wave merge (position space was partitioned; combine the
-  // four partial states like a split-S merge, in the freed staging LDS)
+  // merge the four waves' states (their positions are disjoint)
   __syncthreads();
-  float* mrg = reinterpret_cast<float*>(smem);            // [4][16][DV]
-  float* mml = mrg + 4 * 16 * DV;                         // [4][16][2]
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int head = hi * 4 + r;
+  float* mrg = reinterpret_cast<float*>(smem);   // [4][16][DV]
+  float* mml = mrg + 4 * 16 * DV;                // [4][16][2]
+  if (c16 < G) {
 #pragma unroll
     for (int n = 0; n < NV; ++n)
-      mrg[(wave * 16 + head) * DV + n * 16 + row] = acc[n][r];
-    if (row == 0) {
-      mml[(wave * 16 + head) * 2] = m_run[r];
-      mml[(wave * 16 + head) * 2 + 1] = l_run[r];
+      *reinterpret_cast<f32x4*>(
+          &mrg[(wave * 16 + c16) * DV + n * 16 + hi * 4]) = acc[n];
+    if (hi == 0) {
+      mml[(wave * 16 + c16) * 2] = m;
+      mml[(wave * 16 + c16) * 2 + 1] = l;
     }
   }
   __syncthreads();
-  if (wave != 0) return;
+  for (int i = threadIdx.x; i < G * (DV / 4); i += 256) {
+    const int head = i / (DV / 4);
+    const int d = (i % (DV / 4)) * 4;
+    float M = -1e30f, L = 0.f;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int head = hi * 4 + r;
-    float M = -1e30f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w)
-      M = fmaxf(M, mml[(w * 16 + head) * 2]);
-    float L = 0.f;
-#pragma unroll
-    for (int n = 0; n < NV; ++n) acc[n][r] = 0.f;
+    for (int w = 0; w < 4; ++w) M = fmaxf(M, mml[(w * 16 + head) * 2]);
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float wgt = __expf(mml[(w * 16 + head) * 2] - M);
       L += mml[(w * 16 + head) * 2 + 1] * wgt;
-#pragma unroll
-      for (int n = 0; n < NV; ++n)
-        acc[n][r] += mrg[(w * 16 + head) * DV + n * 16 + row] * wgt;
+      o += *reinterpret_cast<const f32x4*>(&mrg[(w * 16 + head) * DV + d]) * wgt;
     }
-    m_run[r] = M;
-    l_run[r] = L;
-  }
-
-  if (partials != nullptr) {
+    const int64_t bh = (int64_t)b * Hq + hkv * G + head;
+    if (nact > 1 || !combine) {
+      float* prow = partials + (bh * splits + split) * (DV + 2);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int head = hi * 4 + r;
-      if (head >= G) continue;
-      float* prow = partials
-          + (((int64_t)b * Hq + hkv * G + head) * splits + split) * (DV + 2);
-#pragma unroll
-      for (int n = 0; n < NV; ++n) prow[n * 16 + row] = acc[n][r];
-      if (row == 0) {
-        prow[DV] = m_run[r];
-        prow[DV + 1] = l_run[r];
+      for (int r = 0; r < 4; ++r) prow[d + r] = o[r];
+      if (d == 0) {
+        prow[DV] = M;
+        prow[DV + 1] = L;
       }
+      continue;
     }
-    return;
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int head = hi * 4 + r;
-    if (head >= G) continue;
     float inv;
     if (sinks != nullptr) {
+      // one extra learned softmax logit per q head whose probability mass is
+      // dropped from the output
       const float sk = bits2f(sinks[hkv * G + head]);
-      const float mx = fmaxf(m_run[r], sk);
-      const float num = __expf(m_run[r] - mx);
-      const float denom = l_run[r] * num + __expf(sk - mx);
+      const float mx = fmaxf(M, sk);
+      const float num = __expf(M - mx);
+      const float denom = L * num + __expf(sk - mx);
       inv = (denom > 0.f) ? num / denom : 0.f;
     } else {
-      inv = (l_run[r] > 0.f) ? 1.f / l_run[r] : 0.f;
+      inv = (L > 0.f) ? 1.f / L : 0.f;
     }
-    short* orow = out + ((int64_t)b * Hq + hkv * G + head) * DV;
+    short4v o4;
 #pragma unroll
-    for (int n = 0; n < NV; ++n)
-      orow[n * 16 + row] = f2bits(acc[n][r] * inv);
+    for (int r = 0; r < 4; ++r) o4.x[r] = f2bits(o[r] * inv);
+    *reinterpret_cast<short4v*>(&out[bh * DV + d]) = o4;
   }
 }
 
-// merge the per-split unnormalized partials: one 64-lane block per (b, h).
+// Merge the per-split unnormalized partials: one wave per (b, h). `pos` (with
+// window, min_span): only the splits that worked on the row are read, and a
+// row that one split finished is left alone; null: all of them are.
 template <int D>
 __global__ void attn_combine_kernel(const float* __restrict__ partials,
                                     const short* __restrict__ sinks,
                                     short* __restrict__ out, const int Hq,
-                                    const int splits) {
+                                    const int splits,
+                                    const int* __restrict__ pos,
+                                    const int Smax, const int window,
+                                    const int min_span) {
   constexpr int DPL = D / kWave;
   const int bh = blockIdx.x;          // b * Hq + h
   const int h = bh % Hq;
   const int lane = threadIdx.x;
+  int n = splits;
+  if (pos != nullptr) {
+    const int len = min(pos[bh / Hq], Smax);
+    n = active_splits(window > 0 ? min(len, window) : len, splits, min_span);
+    if (n == 1) return;
+  }
   const float* base = partials + (int64_t)bh * splits * (D + 2);
   float M = -1e30f;
-  for (int s = 0; s < splits; ++s) M = fmaxf(M, base[s * (D + 2) + D]);
+  for (int s = lane; s < n; s += kWave) M = fmaxf(M, base[s * (D + 2) + D]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
   if (sinks != nullptr) M = fmaxf(M, bits2f(sinks[h]));
   float denom = (sinks != nullptr) ? __expf(bits2f(sinks[h]) - M) : 0.f;
   float acc[DPL];
 #pragma unroll
   for (int j = 0; j < DPL; ++j) acc[j] = 0.f;
-  for (int s = 0; s < splits; ++s) {
+#pragma unroll 4
+  for (int s = 0; s < n; ++s) {
     const float* prow = base + s * (D + 2);
     const float w = __expf(prow[D] - M);
     denom += prow[D + 1] * w;
@@ -555,12 +394,14 @@ void attn_combine(torch::Tensor partials, c10::optional<torch::Tensor> sinks,
     hipLaunchKernelGGL((attn_combine_kernel<128>), dim3((unsigned)(B * Hq)),
                        dim3(kWave), 0, stream,
                        (const float*)partials.data_ptr(), skp,
-                       (short*)out.data_ptr(), (int)Hq, (int)splits);
+                       (short*)out.data_ptr(), (int)Hq, (int)splits,
+                       (const int*)nullptr, 0, 0, 0);
   else
     hipLaunchKernelGGL((attn_combine_kernel<64>), dim3((unsigned)(B * Hq)),
                        dim3(kWave), 0, stream,
                        (const float*)partials.data_ptr(), skp,
-                       (short*)out.data_ptr(), (int)Hq, (int)splits);
+                       (short*)out.data_ptr(), (int)Hq, (int)splits,
+                       (const int*)nullptr, 0, 0, 0);
 }
 
 // q may be a column slice of a fused-QKV buffer: strides (ldq, D, 1).
@@ -585,10 +426,6 @@ void attn_decode(torch::Tensor q, torch::Tensor kcache, torch::Tensor vcache,
   DNET_CHECK(kcache.is_contiguous() && vcache.is_contiguous() &&
                  out.is_contiguous(), "contig");
   auto stream = current_stream();
-  const int G = (int)(Hq / Hkv);
-  const size_t lds = (kChunk * ((int)D + 4) + kChunk * ((int)DV + 4)
-                      + (((int64_t)G * D + 7) & ~7)) * sizeof(short)
-                     + 4 * kChunk * sizeof(float);
   if (splits > 1 || !combine) {
     DNET_CHECK(partials.has_value()
                    && partials->numel() >= B * Hq * splits * (DV + 2),
@@ -603,35 +440,17 @@ void attn_decode(torch::Tensor q, torch::Tensor kcache, torch::Tensor vcache,
   const short* vsp = q8 ? (const short*)vscale->data_ptr() : nullptr;
   float* pp = (splits > 1 || !combine) ? (float*)partials->data_ptr()
                                        : nullptr;
-  // Scalar flash-decode is the default: the MFMA variant measured
-  // SLOWER end to end (3635 vs 3683 tok/s short-ctx, 1433 vs 1491 at
-  // 2k ctx) — decode attention has so little arithmetic per KV byte
-  // that the V-transpose staging the PV MFMA needs (8 scattered 2 B
-  // LDS stores per element vs one short8 row store) costs more than
-  // the matrix cores save. Kept for A/B via DNET_ATTN_MFMA=1.
-  static const bool mfma_on = []() {
-    const char* e = getenv("DNET_ATTN_MFMA");
-    return e != nullptr && e[0] == '1';
-  }();
+  // positions below which a split is not worth its launch and its partials:
+  // one tile per wave while the rows alone leave most CUs idle, two otherwise
+  // (64 rows x 8 kv heads at 160 positions: one split and no partials)
+  const int min_span = B * Hkv < 256 ? 4 * kTile : 8 * kTile;
 #define LAUNCH_ATTN(DD, DDV, QQ)                                              \
-  do {                                                                        \
-    if (mfma_on)                                                              \
-      hipLaunchKernelGGL((attn_decode_mfma_kernel<DD, DDV, QQ>), grid,        \
-                         dim3(256), 0, stream, (const short*)q.data_ptr(),    \
-                         kcache.data_ptr(), vcache.data_ptr(), ksp, vsp,      \
-                         (const int*)pos.data_ptr(), (short*)out.data_ptr(),  \
-                         (int)Hq, (int)Hkv, (int)Smax, (float)scale, ldq,     \
-                         (int)window, (splits > 1 ? nullptr : skp), pp,       \
-                         (int)splits);                                        \
-    else                                                                      \
-      hipLaunchKernelGGL((attn_decode_kernel<DD, DDV, QQ>), grid, dim3(256),  \
-                         lds, stream, (const short*)q.data_ptr(),             \
-                         kcache.data_ptr(), vcache.data_ptr(), ksp, vsp,      \
-                         (const int*)pos.data_ptr(), (short*)out.data_ptr(),  \
-                         (int)Hq, (int)Hkv, (int)Smax, (float)scale, ldq,     \
-                         (int)window, (splits > 1 ? nullptr : skp), pp,       \
-                         (int)splits);                                        \
-  } while (0)
+  hipLaunchKernelGGL((attn_decode_kernel<DD, DDV, QQ>), grid, dim3(256), 0,   \
+                     stream, (const short*)q.data_ptr(), kcache.data_ptr(),   \
+                     vcache.data_ptr(), ksp, vsp,                             \
+                     (const int*)pos.data_ptr(), (short*)out.data_ptr(),      \
+                     (int)Hq, (int)Hkv, (int)Smax, (float)scale, ldq,         \
+                     (int)window, skp, pp, (int)splits, min_span, combine)
   if (D == 192 && q8) LAUNCH_ATTN(192, 128, true);
   else if (D == 192) LAUNCH_ATTN(192, 128, false);
   else if (D == 128 && q8) LAUNCH_ATTN(128, 128, true);
@@ -643,11 +462,15 @@ void attn_decode(torch::Tensor q, torch::Tensor kcache, torch::Tensor vcache,
     if (DV == 128)
       hipLaunchKernelGGL((attn_combine_kernel<128>), dim3((unsigned)(B * Hq)),
                          dim3(kWave), 0, stream, pp, skp,
-                         (short*)out.data_ptr(), (int)Hq, (int)splits);
+                         (short*)out.data_ptr(), (int)Hq, (int)splits,
+                         (const int*)pos.data_ptr(), (int)Smax, (int)window,
+                         min_span);
     else
       hipLaunchKernelGGL((attn_combine_kernel<64>), dim3((unsigned)(B * Hq)),
                          dim3(kWave), 0, stream, pp, skp,
-                         (short*)out.data_ptr(), (int)Hq, (int)splits);
+                         (short*)out.data_ptr(), (int)Hq, (int)splits,
+                         (const int*)pos.data_ptr(), (int)Smax, (int)window,
+                         min_span);
   }
 }
 

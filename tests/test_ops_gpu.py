@@ -813,3 +813,76 @@ def test_deferred_combine_consumers_match_plain():
     # all consumers must have re-zeroed what they read
     scr = _get_scratch(dev)
     assert int((scr != 0).sum()) == 0, "scratch not re-zeroed by consumers"
+
+
+def _attend64(q, k, v, lens, scale, window, sinks):
+    """Decode attention in 64 bits; rows without positions give zeros."""
+    B, Hq, D = q.shape
+    G = k.shape[1]
+    out = torch.zeros(B, Hq, v.shape[-1], dtype=torch.float64)
+    for b in range(B):
+        n = int(lens[b])
+        s0 = max(0, n - window) if window else 0
+        for h in range(Hq if n else 0):
+            g = h // (Hq // G)
+            s = (k[b, g, s0:n] @ q[b, h]) * scale
+            if sinks is not None:
+                p = torch.softmax(torch.cat([s, sinks[h:h + 1]]), 0)[:-1]
+            else:
+                p = torch.softmax(s, 0)
+            out[b, h] = p @ v[b, g, s0:n]
+    return out
+
+
+@pytest.mark.parametrize("splits", [1, 4, 32])
+@pytest.mark.parametrize("d,dv,hq,hkv,cap,window,use_sinks,q8", [
+    (128, 128, 5, 1, 333, 0, False, False),     # odd capacity and group
+    (128, 128, 5, 1, 333, 0, False, True),
+    (64, 64, 16, 1, 257, 0, True, False),       # the widest group
+    (64, 64, 8, 2, 257, 31, True, True),        # window inside one tile
+    (64, 64, 8, 2, 640, 97, True, False),       # window over tile borders
+    (192, 128, 3, 3, 290, 0, False, True),
+])
+def test_attn_decode_tile_edges(d, dv, hq, hkv, cap, window, use_sinks, q8,
+                                splits, monkeypatch):
+    """Lengths around the 32-position tiles, the 128-position steps of a
+    workgroup and the capacity, also none at all; what lies past a row's end
+    is not finite. Bound per value: bf16 output (half a unit of 8 bits: up to
+    2^-8 of it) plus the weights'
+    16 bits and fp32 sums (2^-15 of sum p|v| <= max |v|)."""
+    monkeypatch.setenv("DNET_ATTN_SPLITS", str(splits))
+    torch.manual_seed(21)
+    dev = _dev()
+    lens = [0, 1, 31, 32, 33, 127, 128, 129, 256, cap - 1, cap]
+    B = len(lens)
+    q = torch.randn(B, hq, d, dtype=torch.bfloat16) * 1.5
+    k = torch.randn(B, hkv, cap, d, dtype=torch.bfloat16)
+    v = torch.randn(B, hkv, cap, dv, dtype=torch.bfloat16)
+    ks = vs = None
+    if q8:
+        k, ks = ref.quantize_kv_rows(k)
+        v, vs = ref.quantize_kv_rows(v)
+        k64 = (k.double().unflatten(-1, (-1, 64))
+               * ks.double().unsqueeze(-1)).flatten(-2)
+        v64 = (v.double().unflatten(-1, (-1, 64))
+               * vs.double().unsqueeze(-1)).flatten(-2)
+        for t in (ks, vs):
+            for b, n in enumerate(lens):
+                t[b, :, n:] = float("nan")
+    else:
+        k64, v64 = k.double(), v.double()
+        for t in (k, v):
+            for b, n in enumerate(lens):
+                t[b, :, n:] = float("nan")
+    sinks = torch.randn(hq, dtype=torch.bfloat16) if use_sinks else None
+    pos = torch.tensor(lens, dtype=torch.int32)
+    want = _attend64(q.double(), k64, v64, lens, d ** -0.5, window,
+                     sinks.double() if use_sinks else None)
+
+    def gpu(t):
+        return None if t is None else t.to(dev)
+    got = ops.attn_decode(gpu(q), gpu(k), gpu(v), gpu(pos), d ** -0.5, window,
+                          gpu(sinks), gpu(ks), gpu(vs)).double().cpu()
+    bound = want.abs() * 2 ** -8 + float(v64.abs().max()) * 2 ** -15
+    assert torch.isfinite(got).all()
+    assert ((got - want).abs() <= bound).all()
