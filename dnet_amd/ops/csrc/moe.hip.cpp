@@ -27,6 +27,8 @@ namespace dnet {
 constexpr int kMoeWaves = 4;
 
 using i32x4 = __attribute__((ext_vector_type(4))) int;
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
 
 template <int M>
 __device__ __forceinline__ bool expert_routed(const float* __restrict__ we,
@@ -64,11 +66,10 @@ __device__ __forceinline__ float apply_glu(float g, float u, const float alpha,
 }
 
 // QMODE: 0 = bf16, 1 = grouped int8, 2 = mxfp4 (nibble rows + e8m0)
-// launch bounds: M<=8 keeps the tight 128-VGPR budget (measured faster
-// at high occupancy); the wide tiles trade occupancy for bank-read
-// amortization and need the bigger register file.
+// Few rows, mxfp4 and odd scale groups (moe_on_cores); M <= 8 per pass at a
+// 128-register budget.
 template <int M, int QMODE, bool PACKED, int GLU>
-__global__ __launch_bounds__(256, M <= 8 ? 4 : 2) void moe_gateup_kernel(
+__global__ __launch_bounds__(256, 4) void moe_gateup_kernel(
     const short* __restrict__ x, const void* __restrict__ w,
     const short* __restrict__ scales, const short* __restrict__ bias,
     const float* __restrict__ we, short* __restrict__ act, const int K,
@@ -209,7 +210,7 @@ __global__ __launch_bounds__(256, M <= 8 ? 4 : 2) void moe_gateup_kernel(
 // Same layout as moe_gateup_kernel's bf16 branch with one weight row per
 // wave; experts nobody in the tile chose are skipped.
 template <int M>
-__global__ __launch_bounds__(256, M <= 8 ? 4 : 2) void moe_up_act_kernel(
+__global__ __launch_bounds__(256, 4) void moe_up_act_kernel(
     const short* __restrict__ x, const short* __restrict__ w,
     const float* __restrict__ we, short* __restrict__ act, const int K,
     const int I, const int E, const int Mtot, const int m0) {
@@ -350,6 +351,325 @@ __global__ __launch_bounds__(256, 4) void moe_down_kernel(
   }
 }
 
+// ---- routed rows on matrix cores ------------------------------------------------
+// What both kernels above compute, for a batch: the weights of an expert that
+// any of up to 64 rows chose are read once (the scalar kernels read them once
+// per 8 rows and hold 2 M accumulators per lane). Only the rows that chose the
+// expert are multiplied: their numbers are compacted (a ballot, one list in
+// LDS), so 20 rows with 4 of 32 experts cost one 16-row tile per expert.
+//
+// grid (column tiles, K splits, E), 4 waves. Weights are the B operand of
+// v_mfma_f32_16x16x32_bf16 and go from memory straight to registers, 64 B of
+// every one of 16 NF rows per wave and step; the waves take neighbouring steps
+// and fold their sums through LDS. Rows of x come from L2 in the A layout. The
+// next group of steps is in flight while one is multiplied. int8 weights are
+// multiplied as whole numbers (exact in bf16), their scale applies to the fp32
+// sums of a 64-wide step.
+// Measured, MI355X: 20 rows, 32 bf16 experts of 2880 x 2880 (4 chosen): gate
+// and up 651 -> 180 us (5.5 TB/s), down 484 -> 106 us (4.7); 20 rows, 8 int8
+// experts of 4096 x 14336 (2 chosen): 1034 -> 248 us (3.8 TB/s, bound by the
+// conversions at 2 waves per SIMD), 761 -> 145 us. Error of the fp32 result
+// against 64 bits 1.0e-7 (bf16, as before), 1.2e-7 (int8; 2.5e-7).
+// KIND: 0 / 1 = gated (GLU 0 / 1; the first half of the NF fragments are gate
+// columns, the second the up columns beside them), 2 = weighted sum of the
+// experts' results by fp32 atomics.
+template <int MT, int NF, bool Q8, bool PACKED, int KIND>
+__device__ __forceinline__ void moe_experts_body(
+    const int* list, const int rows, f32x4 (*part)[MT * NF][64],
+    const short* __restrict__ x, const void* __restrict__ w,
+    const short* __restrict__ scales, const short* __restrict__ bias,
+    const float* __restrict__ we, void* __restrict__ out, const int K,
+    const int N, const int E, const int Mtot, const int m0,
+    const int64_t x_expert, const int G, const float alpha,
+    const float limit) {
+  constexpr bool GLU = KIND != 2;
+  constexpr int NC = GLU ? NF / 2 : NF;      // column fragments of the result
+  constexpr int NJ = Q8 ? 2 : 1;             // products per step
+  constexpr int U = Q8 && MT > 1 ? 1 : 2;    // neighbouring steps of a wave
+  constexpr int KS = Q8 ? 64 : 32;           // inner width of a step (64 B)
+  const int e = blockIdx.z;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int c = lane & 15, hi = lane >> 4;
+  const int n0 = blockIdx.x * (16 * NC);
+
+  const int rb = Q8 ? K : 2 * K;             // bytes of a weight row
+  // step / (steps per scale group): exact for fewer than 2^16 steps
+  const uint64_t ginv = Q8 ? ((1ull << 32) + G / 64 - 1) / (G / 64) : 0;
+  const char* wp[NF];
+  const short* sp[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    const int col = min(n0 + (f % NC) * 16 + c, N - 1);
+    const int64_t row = GLU ? ((int64_t)e * 2 + f / NC) * N + col
+                            : (int64_t)e * N + col;
+    wp[f] = (const char*)w + row * rb + hi * 16;
+    sp[f] = Q8 ? scales + row * (K / G) : nullptr;
+  }
+  const short* xp[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+    xp[m] = x + e * x_expert +
+            (int64_t)(m0 + list[min(m * 16 + c, rows - 1)]) * K +
+            (Q8 && !PACKED ? hi * 16 : hi * 8);
+  f32x4 acc[MT][NF];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int f = 0; f < NF; ++f) acc[m][f] = {0.f, 0.f, 0.f, 0.f};
+
+  struct Batch {
+    i32x4 wf[U][NF];
+    bf16x8 xf[U][NJ][MT];
+    float sc[U][NF];
+  };
+  // a step past the row's end, or the part of the last one that is, is zero
+  // (K is a multiple of what one lane loads)
+  auto load = [&](Batch& q, const int s, const bool whole) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int at = (s + u) * 64;
+        const bool in = whole || at + hi * 16 < rb;
+        q.wf[u][f] = in ? *reinterpret_cast<const i32x4*>(wp[f] + at)
+                        : i32x4{0, 0, 0, 0};
+        if (Q8) q.sc[u][f] = in ? bits2f(sp[f][((uint64_t)(s + u) * ginv) >> 32]) : 0.f;
+      }
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool in = whole || (s + u) * 64 + hi * 16 < rb;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const i32x4 v =
+              in ? *reinterpret_cast<const i32x4*>(
+                       xp[m] + (s + u) * KS + j * (PACKED ? 32 : 8))
+                 : i32x4{0, 0, 0, 0};
+          q.xf[u][j][m] = __builtin_bit_cast(bf16x8, v);
+        }
+      }
+    }
+  };
+  // products of a step (bf16: of the U steps) from zero, added to the sums by
+  // the vector unit: the matrix core's own sums round less exactly
+  auto mul = [&](const Batch& q) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      if (Q8) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          bf16x8 wf[NJ];
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+              wf[j][k] = (__bf16)(float)(signed char)(
+                  q.wf[u][f][2 * j + k / 4] >> (8 * (k & 3)));
+#pragma unroll
+          for (int m = 0; m < MT; ++m) {
+            f32x4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+              p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.xf[u][j][m], wf[j],
+                                                          p, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              acc[m][f][r] = fmaf(q.sc[u][f], p[r], acc[m][f][r]);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          f32x4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                q.xf[u][0][m], __builtin_bit_cast(bf16x8, q.wf[u][f]), p, 0, 0,
+                0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[m][f][r] += p[r];
+        }
+      }
+    }
+  };
+  // this split's steps; whole groups of 4 x U steps, then the rest one by one.
+  // Workgroups start at different places: weight rows are often a power of two
+  // apart, in step they would all read from the same few memory channels
+  const int total = (rb + 63) / 64;
+  const int per = (total + gridDim.y - 1) / gridDim.y;
+  const int s0 = blockIdx.y * per, s1 = min(total, s0 + per);
+  const int full = max(s0, min(s1, rb / 64));     // whole steps end here
+  const int groups = (full - s0) / (4 * U);
+  const int turn =
+      groups > 1 ? (int)((blockIdx.x * 5 + blockIdx.z * 3) % groups) : 0;
+  auto place = [&](int g) {
+    g += turn;
+    if (g >= groups) g -= groups;
+    return s0 + (g * 4 + wave) * U;
+  };
+  Batch q0, q1;
+  if (groups > 0) {
+    load(q0, place(0), true);
+    int g = 0;
+    for (; g + 2 <= groups; g += 2) {
+      load(q1, place(g + 1), true);
+      __builtin_amdgcn_sched_barrier(0);
+      mul(q0);
+      if (g + 2 < groups) load(q0, place(g + 2), true);
+      __builtin_amdgcn_sched_barrier(0);
+      mul(q1);
+    }
+    if (g < groups) mul(q0);
+  }
+  for (int s = s0 + groups * 4 * U + wave * U; s < s1; s += 4 * U) {
+    load(q0, s, false);
+    // a step of the next split, or past the end, counts nothing
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s + u >= s1)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) q0.wf[u][f] = i32x4{0, 0, 0, 0};
+    mul(q0);
+  }
+
+  // the last products' results are read below, behind a branch: past their
+  // latency in any case
+  asm volatile("s_nop 15" ::: "memory");
+  // fold the four waves' sums
+#pragma unroll
+  for (int half = 2; half > 0; half >>= 1) {
+    if (wave >= half && wave < 2 * half)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) part[wave - half][m * NF + f][lane] = acc[m][f];
+    __syncthreads();
+    if (wave < half)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          const f32x4 p = part[wave][m * NF + f][lane];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[m][f][r] += p[r];
+        }
+    __syncthreads();
+  }
+  if (wave != 0) return;
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int f = 0; f < NC; ++f) {
+      const int i = n0 + f * 16 + c;
+      if (i >= N) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int p = m * 16 + hi * 4 + r;
+        if (p >= rows) continue;
+        const int t = m0 + list[p];
+        float v = acc[m][f][r];
+        if constexpr (GLU) {
+          float u = acc[m][NC + f][r];
+          if (bias != nullptr) {
+            v += bits2f(bias[(int64_t)e * 2 * N + i]);
+            u += bits2f(bias[((int64_t)e * 2 + 1) * N + i]);
+          }
+          ((short*)out)[((int64_t)e * Mtot + t) * N + i] =
+              f2bits(apply_glu<KIND>(v, u, alpha, limit));
+        } else {
+          if (bias != nullptr && blockIdx.y == 0)
+            v += bits2f(bias[(int64_t)e * N + i]);
+          atomicAdd(&((float*)out)[(int64_t)t * N + i],
+                    v * we[(int64_t)t * E + e]);
+        }
+      }
+    }
+}
+
+template <int MT, int NF, bool Q8, bool PACKED, int KIND>
+__global__ __launch_bounds__(256, 2) void moe_experts_kernel(
+    const short* __restrict__ x, const void* __restrict__ w,
+    const short* __restrict__ scales, const short* __restrict__ bias,
+    const float* __restrict__ we, void* __restrict__ out, const int K,
+    const int N, const int E, const int Mtot, const int m0,
+    const int64_t x_expert, const int G, const float alpha,
+    const float limit) {
+  __shared__ __attribute__((aligned(16))) char part[2 * MT * NF * 64 * 16];
+  __shared__ int list[64];
+  const int e = blockIdx.z;
+  const int lane = threadIdx.x & 63;
+  const bool hit = lane < 16 * MT && m0 + lane < Mtot &&
+                   we[(int64_t)(m0 + lane) * E + e] != 0.f;
+  const unsigned long long mask = __ballot(hit);
+  const int rows = __popcll(mask);
+  if (rows == 0) return;                     // the same in all waves
+  if (threadIdx.x < 64 && hit)
+    list[__popcll(mask & ((1ull << lane) - 1ull))] = lane;
+  __syncthreads();
+  // as many row tiles as hold anything, each number its own code: a branch
+  // around a tile's products inside the loop would stand between them and the
+  // reads of their results
+#define ME_BODY(TT)                                                           \
+  moe_experts_body<TT, NF, Q8, PACKED, KIND>(                                 \
+      list, rows, reinterpret_cast<f32x4(*)[(TT) * NF][64]>(part), x, w,      \
+      scales, bias, we, out, K, N, E, Mtot, m0, x_expert, G, alpha, limit)
+  if (MT == 1 || rows <= 16) ME_BODY(1);
+  else if (MT == 2 || rows <= 32) ME_BODY(MT == 1 ? 1 : 2);
+  else ME_BODY(MT);
+#undef ME_BODY
+}
+
+// x [M, K] or [E, M, K] through the experts w [E, N (gated: 2 N), K]
+static void moe_experts(int kind, const torch::Tensor& x,
+                        const torch::Tensor& w, const short* scales,
+                        const short* bias, const torch::Tensor& we,
+                        torch::Tensor& out, int64_t K, int64_t N, int64_t M,
+                        int64_t x_expert, int64_t group, bool q8, bool packed,
+                        float alpha, float limit) {
+  const int64_t E = we.size(1);
+  auto stream = current_stream();
+  const int nf = M <= 4 ? 2 : 4;
+  const unsigned tiles = (unsigned)cdiv(N, 16 * (kind == 2 ? nf : nf / 2));
+  // the weighted sum is by atomics anyway: the inner dimension is split where
+  // the chosen experts' column tiles may leave CUs idle
+  unsigned ks = 1;
+  while (kind == 2 && ks < 4 && tiles * ks * std::min<int64_t>(E, 2 * M) < 768 &&
+         K / (ks * 2) >= 1024)
+    ks *= 2;
+  const dim3 grid(tiles, ks, (unsigned)E);
+  for (int64_t m0 = 0; m0 < M; m0 += 64) {
+    const int64_t left = M - m0;
+#define ME(MM, NN, QQ, PP, KK)                                                \
+  hipLaunchKernelGGL((moe_experts_kernel<MM, NN, QQ, PP, KK>), grid,          \
+                     dim3(256), 0, stream, (const short*)x.data_ptr(),        \
+                     w.data_ptr(), scales, bias,                              \
+                     (const float*)we.data_ptr(), out.data_ptr(), (int)K,     \
+                     (int)N, (int)E, (int)M, (int)m0, x_expert, (int)group,   \
+                     alpha, limit)
+#define ME_K(MM, NN, QQ, PP)                 \
+  do {                                       \
+    if (kind == 0) ME(MM, NN, QQ, PP, 0);    \
+    else if (kind == 1) ME(MM, NN, QQ, PP, 1); \
+    else ME(MM, NN, QQ, PP, 2);              \
+  } while (0)
+#define ME_Q(MM, NN)                              \
+  do {                                            \
+    if (q8 && packed) ME_K(MM, NN, true, true);   \
+    else if (q8) ME_K(MM, NN, true, false);       \
+    else ME_K(MM, NN, false, false);              \
+  } while (0)
+    if (nf == 2) ME_Q(1, 2);
+    else if (left <= 16) ME_Q(1, 4);
+    else if (left <= 32) ME_Q(2, 4);
+    else ME_Q(4, 4);
+#undef ME_Q
+#undef ME_K
+#undef ME
+  }
+}
+
 // ---- routing and merging for batched expert products -----------------------
 // moe_route: we[t, e] = softmax(logits[t, :])[e] * scale for the `top`
 // largest probabilities of row t, 0 elsewhere (the weights are not
@@ -429,31 +749,26 @@ static void moe_dispatch_m(int M, LaunchFn&& fn) {
     case 4: fn(std::integral_constant<int, 4>{}); break;
     case 6: fn(std::integral_constant<int, 6>{}); break;
     case 8: fn(std::integral_constant<int, 8>{}); break;
-    case 16: fn(std::integral_constant<int, 16>{}); break;
-    case 32: fn(std::integral_constant<int, 32>{}); break;
     default: TORCH_CHECK(false, "moe: unsupported M tile ", M);
   }
 }
 
-static int moe_mtile(int64_t rem, bool mx4, int cap) {
-  // Wider M tiles amortize the expert-bank read (at batch 32, M=8
-  // re-reads every routed bank 4x per layer) but MEASURED SLOWER:
-  // gpt-oss b32 gu8/dn8 2434 tok/s vs dn32 2386 / gu16 2141 — the
-  // occupancy cost (VGPR 2M accumulators) outweighs the traffic cut;
-  // these kernels are latency-bound. M=16/32 tiers kept behind
-  // DNET_MOE_MT_GU / DNET_MOE_MT_DN; the structural fix is an
-  // LDS-staged-x MFMA expert GEMM (round-3 lever).
+static int moe_mtile(int64_t rem, bool mx4) {
   if (mx4 && rem >= 6) return 6;   // M=8 mxfp4 spills ~30 regs
-  if (cap >= 32 && rem >= 32) return 32;
-  if (cap >= 16 && rem >= 16) return 16;
   if (rem >= 8) return 8;
   if (rem == 7 || rem == 5) return 4;
   return (int)rem;
 }
 
-static int moe_cap(const char* env, int dflt) {
-  const char* e = getenv(env);
-  return e ? atoi(e) : dflt;
+// Rows from which the matrix-core kernel is the faster one (us, gateup + down,
+// scalar / matrix cores). bf16, 32 experts of 2880 x 2880, 4 chosen: 2 rows
+// 66 / 80, 3 rows 121 / 126, 4 rows 160 / 132, 20 rows 1135 / 287, 64 rows
+// 3376 / 315; int8, 8 experts of 4096 x 14336, 2 chosen: 2 rows 192 / 200,
+// 3 rows 291 / 258, 20 rows 1795 / 393, 64 rows 5617 / 467. mxfp4, and scale
+// groups that a 64-wide step does not divide into, stay with the scalar one.
+static bool moe_on_cores(int64_t M, bool mx4, bool q8, int64_t group) {
+  if (mx4) return false;
+  return q8 ? M >= 3 && group % 64 == 0 : M >= 4;
 }
 
 void moe_gateup(torch::Tensor x, torch::Tensor w,
@@ -490,11 +805,15 @@ void moe_gateup(torch::Tensor x, torch::Tensor w,
   }
   const short* bptr = bias.has_value() ? (const short*)bias->data_ptr() : nullptr;
   auto stream = current_stream();
+  if (moe_on_cores(M, mx4, q8, group)) {
+    moe_experts(glu == 1 ? 1 : 0, x, w, sptr, bptr, we, act, K, I, M, 0, group,
+                q8, packed, (float)alpha, (float)limit);
+    return;
+  }
   const dim3 grid(cdiv((int)I, kMoeWaves), 1, (unsigned)E);
-  static const int gu_cap = moe_cap("DNET_MOE_MT_GU", 8);
   int64_t m0 = 0;
   while (m0 < M) {
-    const int mt = moe_mtile(M - m0, mx4, gu_cap);
+    const int mt = moe_mtile(M - m0, mx4);
     moe_dispatch_m(mt, [&](auto mc) {
       constexpr int MV = decltype(mc)::value;
       auto launch = [&](auto qmc, auto pkc, auto gluc) {
@@ -520,7 +839,7 @@ void moe_gateup(torch::Tensor x, torch::Tensor w,
           with_glu(std::integral_constant<int, 1>{}, std::false_type{});
       } else if (mx4) {
         with_glu(std::integral_constant<int, 2>{}, std::false_type{});
-      } else {
+      } else if constexpr (MV < 4) {
         with_glu(std::integral_constant<int, 0>{}, std::false_type{});
       }
     });
@@ -546,7 +865,7 @@ void moe_up_act(torch::Tensor x, torch::Tensor w, torch::Tensor we,
   const dim3 grid(cdiv((int)I, kMoeWaves), 1, (unsigned)E);
   int64_t m0 = 0;
   while (m0 < M) {
-    const int mt = moe_mtile(M - m0, false, 8);
+    const int mt = moe_mtile(M - m0, false);
     moe_dispatch_m(mt, [&](auto mc) {
       constexpr int MV = decltype(mc)::value;
       hipLaunchKernelGGL((moe_up_act_kernel<MV>), grid,
@@ -630,11 +949,15 @@ void moe_down(torch::Tensor act, torch::Tensor w,
   }
   const short* bptr = bias.has_value() ? (const short*)bias->data_ptr() : nullptr;
   auto stream = current_stream();
+  if (moe_on_cores(M, mx4, q8, group)) {
+    moe_experts(2, act, w, sptr, bptr, we, out, I, H, M, M * I, group, q8,
+                packed, 0.f, 0.f);
+    return;
+  }
   const dim3 grid(cdiv((int)H, kMoeWaves), 1, (unsigned)E);
-  static const int dn_cap = moe_cap("DNET_MOE_MT_DN", 8);
   int64_t m0 = 0;
   while (m0 < M) {
-    const int mt = moe_mtile(M - m0, mx4, dn_cap);
+    const int mt = moe_mtile(M - m0, mx4);
     moe_dispatch_m(mt, [&](auto mc) {
       constexpr int MV = decltype(mc)::value;
       auto launch = [&](auto qmc, auto pkc) {
@@ -653,7 +976,7 @@ void moe_down(torch::Tensor act, torch::Tensor w,
           launch(std::integral_constant<int, 1>{}, std::false_type{});
       } else if (mx4) {
         launch(std::integral_constant<int, 2>{}, std::false_type{});
-      } else {
+      } else if constexpr (MV < 4) {
         launch(std::integral_constant<int, 0>{}, std::false_type{});
       }
     });

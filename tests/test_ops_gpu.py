@@ -886,3 +886,77 @@ def test_attn_decode_tile_edges(d, dv, hq, hkv, cap, window, use_sinks, q8,
     bound = want.abs() * 2 ** -8 + float(v64.abs().max()) * 2 ** -15
     assert torch.isfinite(got).all()
     assert ((got - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M", [4, 16, 17, 33, 48, 64, 67])
+@pytest.mark.parametrize("mode,K,I,glu", [
+    ("bf16", 104, 72, 1),       # inner sizes that end inside a step
+    ("bf16", 520, 2056, 0),     # the second product is split
+    ("packed", 512, 320, 0),
+    ("plain", 192, 64, 1),      # int8 in row order, 3 scale groups
+    ("packed", 128, 2112, 1),   # 33 steps: a split ends between two
+])
+def test_moe_experts_row_tiles(mode, K, I, glu, M):
+    """Experts that all rows, some, one and none chose: 0 to 4 tiles of 16 rows
+    in one launch, and a second pass past 64 rows. The sums are fp32: each
+    value within (K + 8) 2^-24 of sum |x w| (the order is free), the gated
+    result through its derivative (at most 1.1 |u| + 1.1 |g|) plus bf16."""
+    torch.manual_seed(M)
+    E, G, dev = 6, 64, _dev()
+    x = torch.randn(M, K, dtype=torch.bfloat16)
+    gw = (torch.randn(E, 2 * I, K) / K ** 0.5).to(torch.bfloat16)
+    dw = (torch.randn(E, K, I) / I ** 0.5).to(torch.bfloat16)
+    gb = torch.randn(E, 2 * I, dtype=torch.bfloat16) / 4
+    db = torch.randn(E, K, dtype=torch.bfloat16) / 4
+    we = torch.zeros(M, E)
+    we[:, 0] = torch.rand(M) + 0.1                # everyone
+    we[::2, 1] = torch.rand((M + 1) // 2) + 0.1   # every second
+    we[M - 1, 2] = 0.5                            # one, the last
+    we[: min(M, 18), 4] = 0.25                    # 3 and 5: nobody
+    gs = ds = None
+    w64, d64 = gw.double(), dw.double()
+    if mode != "bf16":
+        gq, gs = ops.quantize_int8(gw.view(-1, K), G)
+        dq, ds = ops.quantize_int8(dw.view(-1, I), G)
+        w64 = (gq.double().view(-1, K // G, G)
+               * gs.double().unsqueeze(-1)).view(E, 2 * I, K)
+        d64 = (dq.double().view(-1, I // G, G)
+               * ds.double().unsqueeze(-1)).view(E, K, I)
+        if mode == "packed":
+            gq, dq = ops.pack_int8_mfma(gq), ops.pack_int8_mfma(dq)
+        gw, dw = gq.view(E, 2 * I, K), dq.view(E, K, I)
+        gs, ds = gs.view(E, 2 * I, -1), ds.view(E, K, -1)
+
+    def gpu(t):
+        return None if t is None else t.contiguous().to(dev)
+    g = 0 if mode == "bf16" else G
+    act = ops.moe_gateup(gpu(x), gpu(gw), gpu(gs), gpu(gb), gpu(we), g,
+                         mode == "packed", glu).cpu()
+    h = torch.einsum("mk,enk->emn", x.double(), w64) + gb.double().unsqueeze(1)
+    mass = torch.einsum("mk,enk->emn", x.double().abs(), w64.abs()) + 1
+    a, u = h[..., :I], h[..., I:]
+    lim = mass[..., :I] + mass[..., I:]
+    if glu:
+        a, u = a.clamp(max=7.0), u.clamp(-7.0, 7.0)
+        want = (u + 1) * a * torch.sigmoid(1.702 * a)
+        slope = 1.1 * (u + 1).abs() + a.abs()
+    else:
+        want = torch.nn.functional.silu(a) * u
+        slope = 1.1 * u.abs() + 1.1 * a.abs()
+    chosen = (we != 0).t()
+    bound = (slope * lim * (K + 8) * 2 ** -24 + want.abs() * 2 ** -8
+             + want.abs() * 2 ** -18 + 1e-6)
+    assert ((act.double() - want).abs() <= bound)[chosen].all()
+
+    act_in = want.to(torch.bfloat16)
+    out = ops.moe_down(gpu(act_in), gpu(dw), gpu(ds), gpu(db), gpu(we), g,
+                       mode == "packed").cpu()
+    a64 = act_in.double() * chosen.unsqueeze(-1)
+    want = torch.einsum("me,emk->mk", we.double(),
+                        torch.einsum("emi,eki->emk", a64, d64)
+                        + db.double().unsqueeze(1))
+    mass = torch.einsum("me,emk->mk", we.double(),
+                        torch.einsum("emi,eki->emk", a64.abs(), d64.abs())
+                        + db.double().abs().unsqueeze(1))
+    assert ((out.double() - want).abs()
+            <= mass * (I + 8 + E) * 2 ** -24).all()
