@@ -450,7 +450,7 @@ def _chunked_causal_attention(q, k, v, scale, q_offsets, window=0,
     qc = 512
     kk = k.unsqueeze(2)  # [B, Hkv, 1, S, D]
     vv = v.unsqueeze(2)
-    qg = q.view(B, Hkv, G, T, D)
+    qg = q.reshape(B, Hkv, G, T, D)
     og = out.view(B, Hkv, G, T, Dv)
     pos_k = torch.arange(S, device=q.device)
     compute_dtype = q.dtype  # bf16 GEMMs (hipBLASLt MFMA); fp32 softmax

@@ -204,15 +204,26 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                  sinks: torch.Tensor | None = None) -> torch.Tensor:
     """Fused MFMA flash prefill attention (causal + window + sinks).
 
-    q [B,Hq,T,D], k/v [B,Hkv,S,D(v)] -> [B,Hq,T,Dv]. GPU-only; callers
-    gate on attn_prefill_supported and fall back to the chunked-einsum
-    path otherwise (models/base.py)."""
+    q [B,Hq,T,D], k/v [B,Hkv,S,D(v)] -> [B,Hq,T,Dv]. Token-major tensors
+    and cache slices come as transposed views: any strides with contiguous
+    rows on 16 B boundaries are read in place. The result is such a view too,
+    token-major in memory (what the output projection reads). GPU-only;
+    callers gate on attn_prefill_supported and fall back to the
+    chunked-einsum path otherwise (models/base.py)."""
     B, Hq, T, D = q.shape
     Dv = v.shape[-1]
-    out = torch.empty(B, Hq, T, Dv, dtype=q.dtype, device=q.device)
-    _native().attn_prefill(q.contiguous(), k.contiguous(), v.contiguous(),
-                           sinks, out, q_off, window, scale)
+    out = torch.empty(B, T, Hq, Dv, dtype=q.dtype,
+                      device=q.device).transpose(1, 2)
+    _native().attn_prefill(_rows16(q), _rows16(k), _rows16(v), sinks, out,
+                           q_off, window, scale)
     return out
+
+
+def _rows16(t: torch.Tensor) -> torch.Tensor:
+    """t itself where its rows can be read 16 B at a time, else a copy."""
+    ok = (t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(
+        n == 1 or st % 8 == 0 for n, st in zip(t.shape[:-1], t.stride())))
+    return t if ok else t.contiguous()
 
 
 def rope_append(q, k, v, kcache, vcache, pos, cos, sin,

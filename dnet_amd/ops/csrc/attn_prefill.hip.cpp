@@ -1,258 +1,301 @@
-// MFMA flash prefill attention (gfx950), causal + sliding window + sinks.
+// Flash attention of a prompt (gfx950): causal, sliding window, sinks.
 //
-// Replaces the chunked-einsum prefill path (models/base.py
-// _chunked_causal_attention: hipBLASLt GEMMs + materialized fp32 score
-// tensors + masked_fill + softmax — ~160 ms of the round-1 TTFT). One
-// fused kernel: QK^T and PV on v_mfma_f32_16x16x32_bf16, fp32 online
-// softmax in the C fragments, score tiles never touch HBM.
 // Reference counterpart: src/dnet/core/models/llama.py:76-102 (MLX SDPA).
 //
-// Geometry: block = 4 waves; each wave owns 16 q rows of a 64-row q tile
-// (grid.x = ceil(T/64), grid.y = Hq, grid.z = B). Per 32-position s tile:
-//   - the 4 waves cooperatively stage K [32][D] and V-transposed [Dv][32]
-//     into LDS (coalesced 16B lines; Vt transposed on the write side),
-//   - QK^T: 2 x (D/32) MFMAs -> scores [16q x 16s] fp32 in C layout
-//     (lane l holds col=l&15, rows (l>>4)*4+0..3),
-//   - causal/window masking in registers; online softmax: row max/sum via
-//     16-lane shfl_xor reductions along the col axis,
-//   - P (bf16) relayed to a per-wave LDS slab -> read back as A
-//     fragments; PV: (Dv/16) MFMAs per s tile accumulate O.
-// Epilogue folds the gpt-oss sink logit into the denominator and writes
-// O / rowsum.
+// The matrix cores bound it, and what feeds them: LDS reads of the key and
+// value tile and, beside them, one exponential and a handful of vector
+// operations per score.
+//   * A workgroup of 4 waves takes 128 rows of one kv head: a row is a (token,
+//     query head of the group) pair, so one tile in LDS serves every head of
+//     the group and few rows are wasted at the diagonal. Each wave owns 32 rows
+//     and holds their q in registers.
+//   * scores^T = K q^T on v_mfma_f32_32x32x16_bf16: a lane's 16 results belong
+//     to one row (its column), and are the positions that the B operand of the
+//     value product wants from this lane: the weights stay in their lane (the
+//     order of the contraction index is free as long as V follows it), the
+//     row's maximum takes one exchange between two lanes, its sum one at the
+//     end.
+//   * V is kept row-major in LDS and read transposed by ds_read_b64_tr_b16.
+//   * 64 positions per tile, two tiles in LDS: the next one is loaded into
+//     registers before the products of this one and written after them, one
+//     barrier per tile. Pitches: K D + 8 (16 rows of a 16 B column fall into
+//     all banks), V a row step of 16 or 48 banks (4 rows x 64 B of half a wave).
+// Tiles from the largest row on (the longest first); kv heads vary fastest, so
+// that with 8 of them each XCD's L2 holds one head's keys and values.
+//
+// Measured, MI355X, 2048 tokens x 32 heads (8 kv heads), D 128: first chunk
+// 355 -> 76 us (454 TFLOP/s on the causal half), behind 5000 positions
+// 1191 -> 264 us (765 TFLOP/s); 64 prompts of 128 tokens x 40 heads 139 -> 59
+// us; 1500 tokens x 64 heads of 64 201 -> 47 us. Before: 16x16 tiles, weights
+// and transposed V through LDS, one query head per workgroup, loads not
+// overlapped. Error against 64 bits unchanged (weights are bf16 in both).
 #include "common.h"
 
 namespace dnet {
 
 using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
-using f32x4 = __attribute__((ext_vector_type(4))) float;
+using s16x4 = __attribute__((ext_vector_type(4))) short;
+using s16x8 = __attribute__((ext_vector_type(8))) short;
+using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
+using f32x16 = __attribute__((ext_vector_type(16))) float;
 
-// D: qk head dim (64/128/192); DV: v head dim (64/128).
-template <int D, int DV, bool WINDOW, bool SINKS>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(
-    const short* __restrict__ q,    // [B, Hq, T, D]
-    const short* __restrict__ k,    // [B, Hkv, S, D]
-    const short* __restrict__ v,    // [B, Hkv, S, DV]
-    const short* __restrict__ sinks,  // [Hq] or null
-    short* __restrict__ out,        // [B, Hq, T, DV]
-    const int B, const int Hq, const int Hkv, const int T, const int S,
-    const int q_off, const int window, const float scale) {
-  constexpr int ST = 32;            // s positions per tile
-  constexpr int DC = D / 32;        // QK k-chunks
-  constexpr int NV = DV / 16;       // PV n-tiles
-  constexpr int KP = D + 8;         // k_lds row stride (pad: 16-lane
-  constexpr int SP = ST + 8;        //   fragment reads hit all banks)
-  __shared__ short k_lds[ST * KP];      // [32][D+8]
-  __shared__ short vt_lds[DV * SP];     // [DV][32+8] (transposed)
-  __shared__ short p_lds[4][16 * SP];   // per-wave P slab [16q][32+8 s]
+constexpr int kKeys = 64;    // positions of a tile
+constexpr int kRows = 128;   // rows of a workgroup
 
+struct Strides {             // elements; the last axis is contiguous
+  int64_t b, h, t;
+};
+
+template <int D, int DV, bool WINDOW>
+__global__ __launch_bounds__(256, D == 192 ? 1 : 2) void attn_prefill_kernel(
+    const short* __restrict__ q, const short* __restrict__ k,
+    const short* __restrict__ v, const short* __restrict__ sinks,
+    short* __restrict__ out, const Strides qs, const Strides ks,
+    const Strides vs, const Strides os, const int G, const int Hkv,
+    const int T, const int S, const int tiles, const int q_off,
+    const int window, const float scale2, const bool flip) {
+  constexpr int NC = D / 16;                 // contraction steps of the scores
+  constexpr int NV = DV / 32;                // 32-dim blocks of the values
+  constexpr int KP = D + 8;
+  constexpr int VP = DV == 96 ? 96 : DV + 32;
+  constexpr int KL = kKeys * D / 8 / 256, VL = kKeys * DV / 8 / 256;
+  static_assert(kKeys * D / 8 % 256 == 0 && kKeys * DV / 8 % 256 == 0, "tile");
+  __shared__ __attribute__((aligned(16))) short k_lds[2][kKeys * KP];
+  __shared__ __attribute__((aligned(16))) short v_lds[2][kKeys * VP];
+
+  const int hkv = blockIdx.x % Hkv;
+  const int tile = tiles - 1 - (blockIdx.x / Hkv) % tiles;
+  const int b = blockIdx.x / (Hkv * tiles);
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  const int h = blockIdx.y;
-  const int b = blockIdx.z;
-  const int hk = h / (Hq / Hkv);
-  const int qt = blockIdx.x * 64 + wave * 16;   // this wave's first q row
-  const int row = lane & 15;
-  const int hi = lane >> 4;                      // 0..3
-  const int qrow = min(qt + row, T - 1);
+  const int c = lane & 31;
+  const int hi = lane >> 5;
+  const int rows = T * G;
+  const int r0 = tile * kRows;
+  const int row = min(r0 + wave * 32 + c, rows - 1);
+  const int t = row / G, g = row % G;
+  const int qpos = q_off + t;
 
-  const short* qp = q + (((int64_t)b * Hq + h) * T + qrow) * D;
-  const short* kp = k + ((int64_t)b * Hkv + hk) * S * D;
-  const short* vp = v + ((int64_t)b * Hkv + hk) * S * DV;
+  // positions that any row of the workgroup sees
+  const int last = q_off + min(r0 + kRows - 1, rows - 1) / G;
+  const int first = WINDOW ? max(0, q_off + r0 / G - window + 1) : 0;
+  const int k_end = min(S, last + 1);
+  const int tile0 = first / kKeys, tile1 = (k_end + kKeys - 1) / kKeys;
+  // tiles up to here are seen whole by every row of this wave (the rows of a
+  // wave ascend; wave-uniform)
+  const int wrow0 = min(r0 + wave * 32, rows - 1);
+  const int whole_end = q_off + wrow0 / G;
 
-  // Q fragments once (A layout: lane holds Q[row][c*32 + hi*8 .. +8])
-  bf16x8 qf[DC];
+  const short* qp = q + b * qs.b + (int64_t)(hkv * G + g) * qs.h + t * qs.t;
+  bf16x8 qf[NC];
 #pragma unroll
-  for (int c = 0; c < DC; ++c)
-    qf[c] = *reinterpret_cast<const bf16x8*>(&qp[c * 32 + hi * 8]);
+  for (int i = 0; i < NC; ++i)
+    qf[i] = *reinterpret_cast<const bf16x8*>(&qp[i * 16 + hi * 8]);
 
-  f32x4 acc[NV];
+  const short* kb = k + b * ks.b + hkv * ks.h;
+  const short* vb = v + b * vs.b + hkv * vs.h;
+  u32x4 kr[KL], vr[VL];
+  // positions past the end repeat the last one: in range and finite, masked
+  auto load = [&](const int kt) {
 #pragma unroll
-  for (int n = 0; n < NV; ++n) acc[n] = {0.f, 0.f, 0.f, 0.f};
-  float m_run[4], l_run[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    m_run[r] = -1e30f;
-    l_run[r] = 0.f;
-  }
-
-  // causal bound for the whole 64-row block (uniform): last s needed
-  const int q_hi = min((int)blockIdx.x * 64 + 63, T - 1);
-  const int s_end = min(S, q_off + q_hi + 1);
-  // window lower bound for the block (uniform, conservative)
-  int s_begin = 0;
-  if (WINDOW) {
-    const int q_lo = (int)blockIdx.x * 64;
-    s_begin = max(0, (q_off + q_lo) - window + 1);
-    s_begin &= ~(ST - 1);  // tile-aligned; in-tile mask handles the rest
-  }
-
-  for (int s0 = s_begin; s0 < s_end; s0 += ST) {
-    // ---- stage K[32][D] + Vt[DV][32] (all 4 waves cooperate) ----
-    __syncthreads();   // previous tile's consumers done
-    for (int idx = threadIdx.x; idx < ST * (D / 8); idx += 256) {
-      const int sr = idx / (D / 8);
-      const int dc = idx % (D / 8);
-      const int sg = min(s0 + sr, S - 1);
-      *reinterpret_cast<short8*>(&k_lds[sr * KP + dc * 8]) =
-          *reinterpret_cast<const short8*>(&kp[(int64_t)sg * D + dc * 8]);
+    for (int i = 0; i < KL; ++i) {
+      const int e = i * 256 + threadIdx.x;
+      const int p = min(kt * kKeys + e / (D / 8), S - 1);
+      kr[i] = *reinterpret_cast<const u32x4*>(&kb[p * ks.t + e % (D / 8) * 8]);
     }
-    // V transposed: thread reads V[s][dv..dv+1] pairs; write [dv][s].
-    // 2 elems per thread-iter keeps the global reads 4B; fine once per
-    // tile (the PV reads hit LDS many times).
-    for (int idx = threadIdx.x; idx < ST * (DV / 2); idx += 256) {
-      const int sr = idx / (DV / 2);
-      const int dc = (idx % (DV / 2)) * 2;
-      const int sg = min(s0 + sr, S - 1);
-      const short v0 = vp[(int64_t)sg * DV + dc];
-      const short v1 = vp[(int64_t)sg * DV + dc + 1];
-      vt_lds[dc * SP + sr] = v0;
-      vt_lds[(dc + 1) * SP + sr] = v1;
+#pragma unroll
+    for (int i = 0; i < VL; ++i) {
+      const int e = i * 256 + threadIdx.x;
+      const int p = min(kt * kKeys + e / (DV / 8), S - 1);
+      vr[i] = *reinterpret_cast<const u32x4*>(&vb[p * vs.t + e % (DV / 8) * 8]);
     }
-    __syncthreads();
+  };
+  auto store = [&](const int buf) {
+#pragma unroll
+    for (int i = 0; i < KL; ++i) {
+      const int e = i * 256 + threadIdx.x;
+      *reinterpret_cast<u32x4*>(
+          &k_lds[buf][e / (D / 8) * KP + e % (D / 8) * 8]) = kr[i];
+    }
+#pragma unroll
+    for (int i = 0; i < VL; ++i) {
+      const int e = i * 256 + threadIdx.x;
+      *reinterpret_cast<u32x4*>(
+          &v_lds[buf][e / (DV / 8) * VP + e % (DV / 8) * 8]) = vr[i];
+    }
+  };
 
-    // ---- QK^T for two 16-s subtiles ----
-    float p_val[2][4];   // [subtile][r] masked+exp'd scores (this lane)
-    float m_new[4];
+  f32x16 acc[NV];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) m_new[r] = m_run[r];
+  for (int n = 0; n < NV; ++n) acc[n] = f32x16{};
+  float m = -1e30f, l = 0.f;      // of scores * scale * log2(e)
+
+  load(tile0);
+  store(tile0 & 1);
+  __syncthreads();
+  for (int kt = tile0; kt < tile1; ++kt) {
+    const int buf = kt & 1;
+    if (kt + 1 < tile1) load(kt + 1);
+    f32x16 s[2];
 #pragma unroll
-    for (int sub = 0; sub < 2; ++sub) {
-      f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < 2; ++h) {
+      s[h] = f32x16{};
+      const short* kl = &k_lds[buf][(h * 32 + c) * KP + hi * 8];
 #pragma unroll
-      for (int c = 0; c < DC; ++c) {
-        // B fragment: lane holds K[scol = lane&15][c*32 + hi*8 .. +8]
-        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(
-            &k_lds[(sub * 16 + row) * KP + c * 32 + hi * 8]);
-        sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[c], kf, sc, 0, 0, 0);
+      for (int i = 0; i < NC; ++i)
+        s[h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            *reinterpret_cast<const bf16x8*>(&kl[i * 16]), qf[i], s[h], 0, 0,
+            0);
+    }
+    // the branch below stands between the products and the first read of
+    // their results: past the products' latency in any case
+    asm volatile("s_nop 15\n\ts_nop 3" : "+v"(s[0]), "+v"(s[1]));
+    if (flip) {
+      s[0] = -s[0];
+      s[1] = -s[1];
+    }
+    // position of result r of half h: kt * 64 + h * 32 + r / 4 * 8 + hi * 4 +
+    // r % 4
+    const int k0 = kt * kKeys;
+    const bool whole = k0 + kKeys - 1 <= whole_end && k0 + kKeys <= S &&
+                       (!WINDOW || k0 > last - window);
+    if (!whole) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int p = k0 + h * 32 + r / 4 * 8 + hi * 4 + r % 4;
+          const bool dead = p > qpos || p >= S ||
+                            (WINDOW && p <= qpos - window);
+          if (dead) s[h][r] = -INFINITY;
+        }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[h][r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mn = fmaxf(m, mx * scale2);
+    if (__any(mn > m)) {
+      const float alpha = __builtin_amdgcn_exp2f(m - mn);
+      l *= alpha;
+#pragma unroll
+      for (int n = 0; n < NV; ++n) acc[n] *= alpha;
+      m = mn;
+    }
+    bf16x8 p[2][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float e =
+            __builtin_amdgcn_exp2f(fmaf(s[h][r], scale2, -m));
+        l += e;
+        p[h][r / 8][r % 8] = (__bf16)e;
       }
-      // C layout: this lane holds scores[q = hi*4 + r][s = row] (within
-      // the subtile); note role swap: A rows = q, B cols = s.
-      const int spos = s0 + sub * 16 + row;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int qq = qt + hi * 4 + r;          // global q row of sc[r]
-        const float val = sc[r] * scale;
-        const int qpos = q_off + qq;
-        bool dead = (spos > qpos) || (spos >= S) || (qq >= T);
-        if (WINDOW) dead |= (spos <= qpos - window);
-        // dead = -inf (not a finite floor): with m_run still at its
-        // finite init, exp(-inf - m) underflows to exactly 0, so fully
-        // masked tiles contribute nothing (a finite floor would give
-        // exp(0)=1 when a whole tile is dead)
-        p_val[sub][r] = dead ? -INFINITY : val;
-      }
-    }
-    // ---- online softmax (rows live across 16 lanes of each hi group,
-    // but C rows are hi*4+r — row r's 16 col values sit in lanes with
-    // the SAME hi, lane&15 = col). shfl_xor over the low 4 lane bits.
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float mx = fmaxf(p_val[0][r], p_val[1][r]);
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1)
-        mx = fmaxf(mx, __shfl_xor(mx, off, 16));
-      m_new[r] = fmaxf(m_run[r], mx);
-      const float corr = __expf(m_run[r] - m_new[r]);
-      float ls = 0.f;
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub) {
-        p_val[sub][r] = __expf(p_val[sub][r] - m_new[r]);
-        ls += p_val[sub][r];
-      }
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1)
-        ls += __shfl_xor(ls, off, 16);
-      l_run[r] = l_run[r] * corr + ls;
-      m_run[r] = m_new[r];
-      // rescale O accumulators for this row: row r of C fragments = acc
-      // element [r] of every n-tile
-#pragma unroll
-      for (int n = 0; n < NV; ++n) acc[n][r] *= corr;
-    }
-    // ---- P -> per-wave LDS slab (bf16), then PV ----
-    // this lane wrote scores for q rows hi*4+r at col `row` (per sub)
-#pragma unroll
-    for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        p_lds[wave][(hi * 4 + r) * SP + sub * 16 + row] =
-            f2bits(p_val[sub][r]);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // wave-local slab
-#pragma unroll
-    for (int n = 0; n < NV; ++n) {
-      // A fragment: P[q = lane&15][hi*8 + j], k-dim = 32 s positions
-      const bf16x8 pf =
-          *reinterpret_cast<const bf16x8*>(&p_lds[wave][row * SP + hi * 8]);
-      // B fragment: Vt[dv = n*16 + lane&15][hi*8 + j]
-      const bf16x8 vf = *reinterpret_cast<const bf16x8*>(
-          &vt_lds[(n * 16 + row) * SP + hi * 8]);
-      acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf, vf, acc[n], 0, 0,
-                                                       0);
-    }
-  }
-
-  // ---- epilogue: sinks + normalize + store ----
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    if (SINKS) {
-      const float sk = bits2f(sinks[h]);
-      const float m2 = fmaxf(m_run[r], sk);
-      l_run[r] = l_run[r] * __expf(m_run[r] - m2) + __expf(sk - m2);
-      const float corr = __expf(m_run[r] - m2);
-#pragma unroll
-      for (int n = 0; n < NV; ++n) acc[n][r] *= corr;
-      m_run[r] = m2;
-    }
-  }
-  // store: lane holds O[q = hi*4 + r][dv = n*16 + row]
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int qq = qt + hi * 4 + r;
-    if (qq >= T) continue;
-    const float inv = 1.0f / fmaxf(l_run[r], 1e-30f);
-    short* op = out + (((int64_t)b * Hq + h) * T + qq) * DV;
 #pragma unroll
     for (int n = 0; n < NV; ++n)
-      op[n * 16 + row] = f2bits(acc[n][r] * inv);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          s16x8 vf;
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const s16x4 part = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4*)&v_lds[buf]
+                    [(h * 32 + u * 16 + x * 8 + hi * 4 + ((lane & 15) >> 2)) *
+                         VP +
+                     n * 32 + (c >> 4) * 16 + (lane & 3) * 4]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) vf[x * 4 + j] = part[j];
+          }
+          acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              __builtin_bit_cast(bf16x8, vf), p[h][u], acc[n], 0, 0, 0);
+        }
+    if (kt + 1 < tile1) store(buf ^ 1);
+    __syncthreads();
   }
+  l += __shfl_xor(l, 32, 64);
+  if (r0 + wave * 32 + c >= rows) return;
+  float f = 1.f;
+  if (sinks != nullptr) {
+    // one extra logit per head whose mass has no value
+    const float sk = bits2f(sinks[hkv * G + g]) * 1.44269504f;
+    const float m2 = fmaxf(m, sk);
+    f = __builtin_amdgcn_exp2f(m - m2);
+    l = l * f + __builtin_amdgcn_exp2f(sk - m2);
+  }
+  const float inv = f / fmaxf(l, 1e-30f);
+  short* op = out + b * os.b + (int64_t)(hkv * G + g) * os.h + t * os.t;
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; r += 4) {
+      short4v o4;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o4.x[j] = f2bits(acc[n][r + j] * inv);
+      *reinterpret_cast<short4v*>(&op[n * 32 + r * 2 + hi * 4]) = o4;
+    }
 }
 
+static Strides strides_of(const torch::Tensor& t, const char* what) {
+  // 16 B accesses along the last axis (an axis of one entry may have any
+  // stride, it is never stepped over)
+  DNET_CHECK(t.stride(3) == 1 && (uintptr_t)t.data_ptr() % 16 == 0, what);
+  for (int i = 0; i < 3; ++i)
+    DNET_CHECK(t.size(i) == 1 || t.stride(i) % 8 == 0, what);
+  return {t.stride(0), t.stride(1), t.stride(2)};
+}
+
+// q [B,Hq,T,D], k [B,Hkv,S,D], v [B,Hkv,S,DV], out [B,Hq,T,DV]: any strides
+// with contiguous rows on 16 B boundaries
 void attn_prefill(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                   c10::optional<torch::Tensor> sinks, torch::Tensor out,
                   int64_t q_off, int64_t window, double scale) {
-  // q [B,Hq,T,D], k [B,Hkv,S,D], v [B,Hkv,S,DV], out [B,Hq,T,DV]
   const int B = q.size(0), Hq = q.size(1), T = q.size(2), D = q.size(3);
   const int Hkv = k.size(1), S = k.size(2), DV = v.size(3);
-  DNET_CHECK(q.is_contiguous() && k.is_contiguous() && v.is_contiguous() &&
-                 out.is_contiguous(),
-             "contig");
-  DNET_CHECK(Hq % Hkv == 0, "GQA heads");
-  DNET_CHECK(out.size(2) == T && out.size(3) == DV, "out shape");
+  DNET_CHECK(q.scalar_type() == torch::kBFloat16 &&
+                 k.scalar_type() == torch::kBFloat16 &&
+                 v.scalar_type() == torch::kBFloat16 &&
+                 out.scalar_type() == torch::kBFloat16, "bf16");
+  DNET_CHECK(Hkv > 0 && Hq % Hkv == 0, "GQA heads");
+  DNET_CHECK(k.size(0) == B && v.size(0) == B && v.size(1) == Hkv &&
+                 v.size(2) == S && k.size(3) == D, "k, v shape");
+  DNET_CHECK(out.size(0) == B && out.size(1) == Hq && out.size(2) == T &&
+                 out.size(3) == DV, "out shape");
+  if (B == 0 || T == 0) return;
+  DNET_CHECK(S > 0 && q_off >= 0 && (int64_t)T * (Hq / Hkv) < (1ll << 30),
+             "prompt size");
+  const Strides qs = strides_of(q, "q rows"), ks = strides_of(k, "k rows");
+  const Strides vs = strides_of(v, "v rows"), os = strides_of(out, "out rows");
   const short* sp =
       sinks.has_value() ? (const short*)sinks->data_ptr() : nullptr;
-  auto stream = current_stream();
-  const dim3 grid((T + 63) / 64, Hq, B);
-  const bool win = window > 0;
-#define LAUNCH_AP(DD, DDV, WW, SS)                                          \
-  hipLaunchKernelGGL((attn_prefill_kernel<DD, DDV, WW, SS>), grid,          \
-                     dim3(256), 0, stream, (const short*)q.data_ptr(),      \
-                     (const short*)k.data_ptr(), (const short*)v.data_ptr(),\
-                     sp, (short*)out.data_ptr(), B, Hq, Hkv, T, S,          \
-                     (int)q_off, (int)window, (float)scale)
-#define LAUNCH_AP_WS(DD, DDV)                                 \
-  do {                                                        \
-    if (win && sp) LAUNCH_AP(DD, DDV, true, true);            \
-    else if (win) LAUNCH_AP(DD, DDV, true, false);            \
-    else if (sp) LAUNCH_AP(DD, DDV, false, true);             \
-    else LAUNCH_AP(DD, DDV, false, false);                    \
+  const int G = Hq / Hkv;
+  const int tiles = cdiv((int64_t)T * G, kRows);
+  const dim3 grid((unsigned)(tiles * Hkv * B));
+  // the kernel's maximum is taken before the factor, which has to be positive
+  const float scale2 =
+      (float)(std::max(std::abs(scale), 1e-30) * 1.4426950408889634);
+#define LAUNCH_AP(DD, DDV, WW)                                               \
+  hipLaunchKernelGGL((attn_prefill_kernel<DD, DDV, WW>), grid, dim3(256), 0, \
+                     current_stream(), (const short*)q.data_ptr(),           \
+                     (const short*)k.data_ptr(), (const short*)v.data_ptr(), \
+                     sp, (short*)out.data_ptr(), qs, ks, vs, os, G, Hkv, T,  \
+                     S, tiles, (int)q_off, (int)window, scale2, scale < 0)
+#define LAUNCH_AP_W(DD, DDV)                \
+  do {                                      \
+    if (window > 0) LAUNCH_AP(DD, DDV, true); \
+    else LAUNCH_AP(DD, DDV, false);         \
   } while (0)
-  if (D == 128 && DV == 128) LAUNCH_AP_WS(128, 128);
-  else if (D == 64 && DV == 64) LAUNCH_AP_WS(64, 64);
-  else if (D == 192 && DV == 128) LAUNCH_AP_WS(192, 128);
-  else if (D == 96 && DV == 96) LAUNCH_AP_WS(96, 96);
+  if (D == 128 && DV == 128) LAUNCH_AP_W(128, 128);
+  else if (D == 64 && DV == 64) LAUNCH_AP_W(64, 64);
+  else if (D == 192 && DV == 128) LAUNCH_AP_W(192, 128);
+  else if (D == 96 && DV == 96) LAUNCH_AP_W(96, 96);
   else DNET_CHECK(false, "attn_prefill: unsupported head dims");
 #undef LAUNCH_AP
-#undef LAUNCH_AP_WS
+#undef LAUNCH_AP_W
 }
 
 }  // namespace dnet

@@ -960,3 +960,52 @@ def test_moe_experts_row_tiles(mode, K, I, glu, M):
                         + db.double().abs().unsqueeze(1))
     assert ((out.double() - want).abs()
             <= mass * (I + 8 + E) * 2 ** -24).all()
+
+
+@pytest.mark.parametrize("hq,hkv,d,dv,t,qoff,extra,window,use_sinks", [
+    (5, 1, 128, 128, 26, 0, 0, 0, False),      # 130 rows: one past a tile
+    (5, 1, 128, 128, 64, 64, 0, 0, False),     # positions end on a tile
+    (8, 2, 128, 128, 33, 95, 7, 0, True),      # keys past the last row
+    (8, 2, 64, 64, 200, 61, 0, 64, True),      # window as wide as a tile
+    (3, 3, 64, 64, 1, 0, 0, 0, False),         # one token
+    (3, 3, 64, 64, 300, 130, 0, 5, False),     # window inside a tile
+    (4, 4, 192, 128, 129, 3, 0, 0, False),
+    (6, 2, 96, 96, 65, 1, 0, 33, True),
+])
+def test_attn_prefill_tile_edges(hq, hkv, d, dv, t, qoff, extra, window,
+                                 use_sinks):
+    """Rows around the 128-row and 64-position tiles, token-major q and a slice
+    of a longer cache read in place; cache rows past the keys are not finite.
+    Bound per value: weights rounded to bf16 (2^-8 of sum p|v|), bf16 output
+    (2^-8 of it), fp32 sums."""
+    torch.manual_seed(t * 7 + hq)
+    B, s = 2, qoff + t + extra
+    dev = _dev()
+    q = torch.randn(B, t, hq, d, dtype=torch.bfloat16).mul_(1.5).transpose(1, 2)
+    k = torch.full((B, hkv, s + 9, d), float("nan"), dtype=torch.bfloat16)
+    v = torch.full((B, hkv, s + 9, dv), float("nan"), dtype=torch.bfloat16)
+    k[:, :, :s] = torch.randn(B, hkv, s, d)
+    v[:, :, :s] = torch.randn(B, hkv, s, dv)
+    sinks = torch.randn(hq, dtype=torch.bfloat16) if use_sinks else None
+    got = ops.attn_prefill(
+        q.to(dev), k.to(dev)[:, :, :s], v.to(dev)[:, :, :s], d ** -0.5, qoff,
+        window, sinks.to(dev) if use_sinks else None).double().cpu()
+    n = hq // hkv
+    k64 = k[:, :, :s].double().repeat_interleave(n, 1)
+    v64 = v[:, :, :s].double().repeat_interleave(n, 1)
+    sc = q.double() @ k64.transpose(-1, -2) * d ** -0.5
+    i = qoff + torch.arange(t).view(-1, 1)
+    j = torch.arange(s)
+    dead = j > i
+    if window:
+        dead = dead | (j <= i - window)
+    sc = sc.masked_fill(dead, float("-inf"))
+    if use_sinks:
+        z = sinks.double().view(1, hq, 1, 1).expand(B, hq, t, 1)
+        p = torch.softmax(torch.cat([sc, z], -1), -1)[..., :-1]
+    else:
+        p = torch.softmax(sc, -1)
+    want, mass = p @ v64, p @ v64.abs()
+    assert got.shape == want.shape
+    bound = (want.abs() + mass) * 2 ** -8 + mass * 2 ** -14
+    assert ((got - want).abs() <= bound).all()
