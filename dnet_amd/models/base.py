@@ -955,14 +955,33 @@ class RingModel:
         positions = torch.arange(p0, p0 + T, device=h.device)
         layer_ids = list(layer_ids)
         dq_ev = self._dequant_prefetch(layer_ids, -1)  # prefetch layer 0
+        delta = None     # the previous layer's output, not yet in the residual
         for i, lid in enumerate(layer_ids):
             lw = self._layer(lid)
             if dq_ev is not None:
                 torch.cuda.current_stream().wait_event(dq_ev)
             dq_ev = self._dequant_prefetch(layer_ids, i)
             flat = h.view(B * T, H)
-            y = ops.rmsnorm(flat, None, lw.attn_norm, c.rms_eps)
+            y = ops.rmsnorm(delta if delta is not None else flat,
+                            flat if delta is not None else None,
+                            lw.attn_norm, c.rms_eps)
             qkv = lw.qkv(y)
+            li = kv.local[lid]
+            if (self.cp_size == 1 and not kv.quantized
+                    and ops.rope_prefill_supported(d, kv.k[li])):
+                # norms, rotation and append in one pass; attention reads
+                # q and the cache in place
+                q = ops.rope_prefill(
+                    qkv, lw.q_norm if c.qk_norm else None,
+                    lw.k_norm if c.qk_norm else None, self.cos, self.sin,
+                    kv.k[li], kv.v[li], nq, T, p0, c.rms_eps)
+                window, sinks = self._attn_params(lid, lw)
+                attn = _chunked_causal_attention(
+                    q.view(B, T, nq, d).transpose(1, 2),
+                    kv.k[li][:, :, :p0 + T], kv.v[li][:, :, :p0 + T],
+                    d ** -0.5, p0, window, sinks)
+                delta = self._prefill_rest(attn, flat, lw)
+                continue
             q = qkv[:, :nq * d].view(B, T, nq, d)
             k = qkv[:, nq * d:(nq + nkv) * d].view(B, T, nkv, d)
             v = qkv[:, (nq + nkv) * d:].view(B, T, nkv, d)
@@ -973,7 +992,6 @@ class RingModel:
                                 c.rms_eps).view(B, T, nkv, d)
             q = ops.rope_apply(q, self.cos, self.sin, positions)
             k = ops.rope_apply(k, self.cos, self.sin, positions)
-            li = kv.local[lid]
             kt, vt = k.transpose(1, 2), v.transpose(1, 2)
             if self.cp_size > 1:
                 # write only this rank's sequence shard; attention gathers
@@ -1022,12 +1040,19 @@ class RingModel:
                 attn = _chunked_causal_attention(
                     q.transpose(1, 2), kv.k_deq(li)[:, :, :p0 + T],
                     kv.v_deq(li)[:, :, :p0 + T], d ** -0.5, p0, window, sinks)
-            o = self._tp_reduce(
-                lw.o(attn.transpose(1, 2).reshape(B * T, nq * d).contiguous()))
-            y2 = ops.rmsnorm(o, flat, lw.mlp_norm, c.rms_eps)
-            delta = self._tp_reduce(self._mlp(y2, lw))
-            flat.add_(delta)
+            delta = self._prefill_rest(attn, flat, lw)
+        flat.add_(delta)
         return h
+
+    def _prefill_rest(self, attn: torch.Tensor, flat: torch.Tensor,
+                      lw: LayerWeights) -> torch.Tensor:
+        """Output projection and feed-forward of a prompt: ``attn``
+        [B, heads, T, d], the residual rows ``flat`` get the attention's part.
+        Returns the feed-forward's, which the next norm adds."""
+        o = self._tp_reduce(
+            lw.o(attn.transpose(1, 2).reshape(flat.shape[0], -1).contiguous()))
+        y2 = ops.rmsnorm(o, flat, lw.mlp_norm, self.cfg.rms_eps)
+        return self._tp_reduce(self._mlp(y2, lw))
 
     def normalize_project(self, h: torch.Tensor) -> torch.Tensor:
         """Final RMSNorm + lm head -> logits [B, V] (last shard only)."""

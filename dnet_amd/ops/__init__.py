@@ -226,6 +226,25 @@ def _rows16(t: torch.Tensor) -> torch.Tensor:
     return t if ok else t.contiguous()
 
 
+def rope_prefill_supported(d: int, kcache: torch.Tensor) -> bool:
+    return (kcache.is_cuda and kcache.dtype == torch.bfloat16
+            and d % 16 == 0 and d <= 128 and kcache.stride(2) == d
+            and kcache.data_ptr() % 16 == 0)
+
+
+def rope_prefill(qkv: torch.Tensor, q_norm, k_norm, cos, sin, kcache, vcache,
+                 nq: int, T: int, p0: int, eps: float) -> torch.Tensor:
+    """The rows of a prompt's fused projection, [B*T, (nq + 2 nkv) d]: per-head
+    norms (optional), rotation at positions p0 + t, k and v written to the
+    cache rows of kcache / vcache [B, nkv, Smax, d]. Returns the rotated
+    q [B*T, nq, d]. GPU only, callers gate on rope_prefill_supported."""
+    q = torch.empty(qkv.shape[0], nq, kcache.shape[3], dtype=qkv.dtype,
+                    device=qkv.device)
+    _native().rope_prefill(qkv, q_norm, k_norm, cos, sin, q, kcache, vcache,
+                           T, p0, eps)
+    return q
+
+
 def rope_append(q, k, v, kcache, vcache, pos, cos, sin,
                 kscale=None, vscale=None, wpos=None) -> None:
     if q.is_cuda:

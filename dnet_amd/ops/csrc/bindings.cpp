@@ -32,6 +32,10 @@ void rope_append_f32(torch::Tensor src, c10::optional<torch::Tensor> bias,
                      c10::optional<torch::Tensor> kscale,
                      c10::optional<torch::Tensor> vscale,
                      c10::optional<torch::Tensor> wpos);
+void rope_prefill(torch::Tensor qkv, c10::optional<torch::Tensor> qw,
+                  c10::optional<torch::Tensor> kw, torch::Tensor cos,
+                  torch::Tensor sin, torch::Tensor qout, torch::Tensor kcache,
+                  torch::Tensor vcache, int64_t T, int64_t p0, double eps);
 void rope_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                  torch::Tensor kcache, torch::Tensor vcache, torch::Tensor pos,
                  torch::Tensor cos_table, torch::Tensor sin_table,
@@ -275,6 +279,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("scale"));
   m.def("attn_combine", &dnet::attn_combine,
         "merge split/rank flash-decode partials");
+  m.def("rope_prefill", &dnet::rope_prefill,
+        "per-head norm + RoPE + KV append of a prompt");
   m.def("rope_append", &dnet::rope_append, "fused RoPE + KV append (decode)",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("kcache"),
         py::arg("vcache"), py::arg("pos"), py::arg("cos_table"),

@@ -249,4 +249,136 @@ void rope_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   }
 }
 
+// A prompt's rotation and append: q and k of the fused projection's rows,
+// optionally RMS-normalized per head (rounded to bf16 as a norm of its own
+// would), rotated; q to a buffer, k and v to their cache rows. 8 lanes per
+// (token, head), each with 8 neighbouring dims of both halves: every access
+// 16 B, every value read and written once (before: gather, multiply, subtract,
+// concatenate, convert and copy as 16 passes of their own per layer).
+// Measured, MI355X: a 37-token prompt through 4 layers of 4096 wide, with the
+// residual sum inside the next norm, 1310 -> 948 us; 64 x 128 tokens through 2
+// layers of 5120 wide 16290 -> 14960 us.
+template <bool NORM>
+__global__ __launch_bounds__(256) void rope_prefill_kernel(
+    const short* __restrict__ qkv, const short* __restrict__ qw,
+    const short* __restrict__ kw, const float* __restrict__ cost,
+    const float* __restrict__ sint, short* __restrict__ qout,
+    short* __restrict__ kc, short* __restrict__ vc, const int64_t kb,
+    const int64_t kh, const int64_t vb, const int64_t vh, const int T,
+    const int nq, const int nkv, const int D, const int p0, const float eps,
+    const int64_t items) {
+  const int64_t item = (int64_t)blockIdx.x * 32 + threadIdx.x / 8;
+  if (item >= items) return;
+  const int heads = nq + 2 * nkv;
+  const int64_t row = item / heads;
+  const int h = (int)(item % heads);
+  const int half = D / 2;
+  const int d = (threadIdx.x & 7) * 8;
+  const bool act = d < half;      // lanes past the half only join the norm
+  const int64_t b = row / T;
+  const int p = p0 + (int)(row % T);
+  const short* src = qkv + (row * heads + h) * D + d;
+  short8 x1 = {}, x2 = {};
+  if (act) {
+    x1 = *reinterpret_cast<const short8*>(src);
+    x2 = *reinterpret_cast<const short8*>(src + half);
+  }
+  short* dst;
+  if (h < nq) dst = qout + (row * nq + h) * D;
+  else if (h < nq + nkv) dst = kc + b * kb + (h - nq) * kh + (int64_t)p * D;
+  else dst = vc + b * vb + (h - nq - nkv) * vh + (int64_t)p * D;
+  if (h < nq + nkv) {
+    if (NORM) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        ss += bits2f(x1.x[j]) * bits2f(x1.x[j]) +
+              bits2f(x2.x[j]) * bits2f(x2.x[j]);
+#pragma unroll
+      for (int off = 4; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 8);
+      const float sc = rsqrtf(ss / (float)D + eps);
+      if (act) {
+        const short* w = (h < nq ? qw : kw) + d;
+        const short8 w1 = *reinterpret_cast<const short8*>(w);
+        const short8 w2 = *reinterpret_cast<const short8*>(w + half);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          x1.x[j] = f2bits(bits2f(x1.x[j]) * sc * bits2f(w1.x[j]));
+          x2.x[j] = f2bits(bits2f(x2.x[j]) * sc * bits2f(w2.x[j]));
+        }
+      }
+    }
+    if (act) {
+      float cs[8], sn[8];
+      const float* cp = cost + (int64_t)p * half + d;
+      const float* sp = sint + (int64_t)p * half + d;
+#pragma unroll
+      for (int j = 0; j < 8; j += 4) {
+        *reinterpret_cast<float4*>(&cs[j]) =
+            *reinterpret_cast<const float4*>(cp + j);
+        *reinterpret_cast<float4*>(&sn[j]) =
+            *reinterpret_cast<const float4*>(sp + j);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float a = bits2f(x1.x[j]), c = bits2f(x2.x[j]);
+        x1.x[j] = f2bits(a * cs[j] - c * sn[j]);
+        x2.x[j] = f2bits(c * cs[j] + a * sn[j]);
+      }
+    }
+  }
+  if (act) {
+    *reinterpret_cast<short8*>(dst + d) = x1;
+    *reinterpret_cast<short8*>(dst + half + d) = x2;
+  }
+}
+
+void rope_prefill(torch::Tensor qkv, c10::optional<torch::Tensor> qw,
+                  c10::optional<torch::Tensor> kw, torch::Tensor cos,
+                  torch::Tensor sin, torch::Tensor qout, torch::Tensor kcache,
+                  torch::Tensor vcache, int64_t T, int64_t p0, double eps) {
+  const int64_t R = qout.size(0), nq = qout.size(1), D = qout.size(2);
+  const int64_t nkv = kcache.size(1), Smax = kcache.size(2);
+  for (const auto& t : {qkv, qout, kcache, vcache})
+    DNET_CHECK(t.scalar_type() == torch::kBFloat16 &&
+                   (uintptr_t)t.data_ptr() % 16 == 0, "bf16, 16 B");
+  DNET_CHECK(D % 16 == 0 && D <= 128, "head size");
+  DNET_CHECK(qkv.is_contiguous() && qkv.numel() == R * (nq + 2 * nkv) * D &&
+                 qout.is_contiguous(), "qkv rows");
+  DNET_CHECK(T > 0 && R % T == 0 && kcache.size(0) == R / T && p0 >= 0 &&
+                 p0 + T <= Smax, "rows and positions");
+  DNET_CHECK(kcache.size(3) == D && vcache.sizes() == kcache.sizes() &&
+                 kcache.stride(3) == 1 && kcache.stride(2) == D &&
+                 vcache.stride(3) == 1 && vcache.stride(2) == D &&
+                 kcache.stride(0) % 8 == 0 && kcache.stride(1) % 8 == 0 &&
+                 vcache.stride(0) % 8 == 0 && vcache.stride(1) % 8 == 0,
+             "cache rows");
+  for (const auto& t : {cos, sin})
+    DNET_CHECK(t.scalar_type() == torch::kFloat && t.is_contiguous() &&
+                   t.size(0) >= p0 + T && t.size(1) == D / 2, "cos, sin");
+  DNET_CHECK(qw.has_value() == kw.has_value(), "both norms or none");
+  if (qw.has_value())
+    for (const auto& t : {*qw, *kw})
+      DNET_CHECK(t.scalar_type() == torch::kBFloat16 && t.is_contiguous() &&
+                     t.numel() == D && (uintptr_t)t.data_ptr() % 16 == 0,
+                 "norm weights");
+  if (R == 0) return;
+  const int64_t items = R * (nq + 2 * nkv);
+  const dim3 grid((unsigned)cdiv(items, 32));
+#define LAUNCH_RP(NN, QW, KW)                                                 \
+  hipLaunchKernelGGL((rope_prefill_kernel<NN>), grid, dim3(256), 0,           \
+                     current_stream(), (const short*)qkv.data_ptr(), QW, KW,  \
+                     cos.data_ptr<float>(), sin.data_ptr<float>(),            \
+                     (short*)qout.data_ptr(), (short*)kcache.data_ptr(),      \
+                     (short*)vcache.data_ptr(), kcache.stride(0),             \
+                     kcache.stride(1), vcache.stride(0), vcache.stride(1),    \
+                     (int)T, (int)nq, (int)nkv, (int)D, (int)p0, (float)eps,  \
+                     items)
+  if (qw.has_value())
+    LAUNCH_RP(true, (const short*)qw->data_ptr(), (const short*)kw->data_ptr());
+  else
+    LAUNCH_RP(false, nullptr, nullptr);
+#undef LAUNCH_RP
+}
+
 }  // namespace dnet

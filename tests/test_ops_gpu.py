@@ -1009,3 +1009,43 @@ def test_attn_prefill_tile_edges(hq, hkv, d, dv, t, qoff, extra, window,
     assert got.shape == want.shape
     bound = (want.abs() + mass) * 2 ** -8 + mass * 2 ** -14
     assert ((got - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("d,norm", [(128, True), (64, False), (96, True),
+                                    (80, False), (16, True)])
+def test_rope_prefill(d, norm):
+    """Norm, rotation and append of a prompt in one kernel against the passes
+    it stands for, in fp32 with the same roundings to bf16: one unit of bf16
+    (2^-7) where the fp32 sums are taken in another order. Rows of the cache
+    outside the prompt stay as they are."""
+    torch.manual_seed(d)
+    B, T, nq, nkv, smax, p0, eps = 2, 5, 6, 2, 40, 9, 1e-6
+    dev = _dev()
+    qkv = torch.randn(B * T, (nq + 2 * nkv) * d, dtype=torch.bfloat16,
+                      device=dev)
+    qw, kw = ((1 + 0.2 * torch.randn(2, d, device=dev)).to(torch.bfloat16)
+              if norm else (None, None))
+    cos, sin = (t.to(dev) for t in ops.rope_tables(smax, d, 10000.0))
+    # a slot of a larger cache
+    full = torch.randn(2, 3, nkv, smax, d, dtype=torch.bfloat16, device=dev)
+    before = full.clone()
+    kc, vc = full[0, 1:], full[1, 1:]
+    q = ops.rope_prefill(qkv, qw, kw, cos, sin, kc, vc, nq, T, p0, eps)
+    x = qkv.view(B, T, nq + 2 * nkv, d)
+    wq, wk, wv = x.split([nq, nkv, nkv], dim=2)
+    pos = torch.arange(p0, p0 + T, device=dev)
+
+    def ref_of(t, w):
+        if w is not None:
+            t = ref.rmsnorm(t.reshape(-1, d), None, w, eps).view_as(t)
+        return ref.rope_apply(t, cos, sin, pos).float()
+    for got, want in ((q.view(B, T, nq, d), ref_of(wq, qw)),
+                      (kc[:, :, p0:p0 + T].transpose(1, 2), ref_of(wk, kw))):
+        # a rotated pair's error is relative to the pair
+        h = d // 2
+        pair = torch.maximum(want[..., :h].abs(), want[..., h:].abs())
+        bound = torch.cat([pair, pair], -1) * 2 ** -6 + 1e-6
+        assert ((got.float() - want).abs() <= bound).all()
+    assert torch.equal(vc[:, :, p0:p0 + T].transpose(1, 2), wv)
+    before[:, 1:, :, p0:p0 + T] = full[:, 1:, :, p0:p0 + T]
+    assert torch.equal(full, before)
