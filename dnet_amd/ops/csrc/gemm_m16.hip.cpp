@@ -1,22 +1,15 @@
 // MFMA decode GEMM: out[M,N] = x[M,K] @ W[N,K]^T (+bias), M <= 64 per pass.
 //
-// The scalar GEMV (gemv.hip.cpp) is VALU-bound at M>=4: every weight element
-// costs ~2 VALU ops per output row. Here one v_mfma_f32_16x16x32_bf16
-// covers a 16(M)x16(N)x32(K) tile; MT in {1,2,4} stacks up to 4 M-tiles per
-// wave so ONE weight read (and for int8 ONE in-register dequant) serves up
-// to 64 batch rows — decode batching at constant weight traffic. Fragment
-// layout for 16x16x32 (cdna_hip_programming.md §3): lane l holds
-// A[row=l&15][k=(l>>4)*8+j], B[col=l&15][k=(l>>4)*8+j],
-// C[col=l&15][row=(l>>4)*4+r].
+// A scalar GEMV is VALU-bound at M >= 4: every weight costs ~2 VALU ops per
+// output row. Here one v_mfma_f32_16x16x32_bf16 covers a 16(M)x16(N)x32(K) tile
+// and up to 4 M-tiles stack, so one weight read serves up to 64 batch rows.
+// Fragment layout: lane l holds A[row=l&15][k=(l>>4)*8+j],
+// B[col=l&15][k=(l>>4)*8+j], C[col=l&15][row=(l>>4)*4+r].
 //
-// x is staged tile-wise into LDS with coalesced full-line loads (direct
-// fragment-shaped x reads touch 16 scattered rows per instruction, up to
-// +45% — guide §5 M=256 GEMM row). int8 weights use the chunk-pair packed
-// layout (pack_int8_mfma) so each lane loads 16 B contiguous (full 64 B
-// HBM bursts).
-//
-// Wave tile: 16 N-columns; block = 4 waves = 64 columns; gridDim.y = SPLITK
-// K-splits (partials combined by f32 atomics + a convert/bias kernel).
+// x goes through LDS with coalesced full-line loads; bf16 weights are read in
+// fragment shape, int8 / int4 weights in the packed layouts that give each lane
+// 16 B of two (four) 32-wide steps. gridDim.y splits K (fp32 atomics into a
+// scratch, combined by the consumer or by a convert/bias kernel).
 #include "common.h"
 
 namespace dnet {
@@ -24,37 +17,15 @@ namespace dnet {
 using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
 using f32x4 = __attribute__((ext_vector_type(4))) float;
 
-__device__ __forceinline__ bf16x8 deq8(const int8_t* q, const float s) {
-  bf16x8 b;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) b[j] = (__bf16)((float)q[j] * s);
-  return b;
-}
-
-// 4 packed nibble-bytes (offset-8) -> 8 bf16 values * scale
-__device__ __forceinline__ bf16x8 deq4(const uint8_t* qb, const float s) {
-  bf16x8 b;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int byte = qb[j];
-    b[2 * j] = (__bf16)((float)((byte & 0xF) - 8) * s);
-    b[2 * j + 1] = (__bf16)((float)((byte >> 4) - 8) * s);
-  }
-  return b;
-}
-
-// QBITS: 16 = bf16 weights, 8 = packed int8 (pack_int8_mfma chunk-pair
-// layout), 4 = packed int4 (pack_int4_mfma chunk-quad layout).
-// MT: number of stacked 16-row A tiles (M <= 16*MT).
-template <int QBITS, int MT>
+// bf16 weights. MT: number of stacked 16-row A tiles (M <= 16*MT).
+template <int MT>
 __global__ void gemm_m16_kernel(const short* __restrict__ x,
-                                const void* __restrict__ w,
-                                const short* __restrict__ scales,
+                                const short* __restrict__ w,
                                 const short* __restrict__ bias,
                                 short* __restrict__ out,        // SPLITK==1
                                 float* __restrict__ out_f32,    // SPLITK>1
                                 const int M, const int K, const int N,
-                                const int G, const int splitk) {
+                                const int splitk) {
   constexpr int XT = 1024 / MT;        // k per x tile (LDS ~33 KB, 4 blocks/CU)
   constexpr int SE = XT + 8;           // row stride in bf16 elems (16B pad)
   __shared__ short x_lds[16 * MT * SE];
@@ -68,20 +39,9 @@ __global__ void gemm_m16_kernel(const short* __restrict__ x,
   const int n_w = min(n0 + row, N - 1);     // this lane's W row
 
   const int pairs = K / 64;
-  int p_begin, p_end;
-  if (QBITS == 4) {
-    // partition at quad (128-k) granularity so every split starts on an
-    // even pair (the int4 layout packs four chunks per lane load)
-    const int quads = K / 128;
-    const int qq = quads / splitk;
-    p_begin = blockIdx.y * qq * 2;
-    p_end = (blockIdx.y == splitk - 1) ? quads * 2 : p_begin + qq * 2;
-  } else {
-    const int pp = pairs / splitk;
-    p_begin = blockIdx.y * pp;
-    p_end = (blockIdx.y == splitk - 1) ? pairs : p_begin + pp;
-  }
-  const int woff = (lane >> 4) * 16;
+  const int pp = pairs / splitk;
+  const int p_begin = blockIdx.y * pp;
+  const int p_end = (blockIdx.y == splitk - 1) ? pairs : p_begin + pp;
 
   f32x4 acc[MT][2];
 #pragma unroll
@@ -89,17 +49,13 @@ __global__ void gemm_m16_kernel(const short* __restrict__ x,
 #pragma unroll
     for (int u = 0; u < 2; ++u) acc[t][u] = {0.f, 0.f, 0.f, 0.f};
 
-  const int8_t* wrow_q = (const int8_t*)w + (int64_t)n_w * K;
-  const uint8_t* wrow_q4 = (const uint8_t*)w + (int64_t)n_w * (K / 2);
-  const short* wrow_b = (const short*)w + (int64_t)n_w * K;
-  const short* srow = QBITS < 16 ? scales + (int64_t)n_w * (K / G) : nullptr;
+  const short* wrow = w + (int64_t)n_w * K;
 
   for (int k0 = p_begin * 64; k0 < p_end * 64; k0 += XT) {
     const int tk = min(XT, p_end * 64 - k0);
     // raw barrier (lgkmcnt only): __syncthreads() would wait vmcnt(0) and
     // drain the in-flight weight stream at EVERY x-tile boundary — at MT=4
     // (XT=256) that is a full memory-pipeline restart every 4 pairs
-    // (guide §6: counted waits, not vmcnt(0), across barriers)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     asm volatile("s_barrier" ::: "memory");
     for (int idx = threadIdx.x; idx < 16 * MT * (tk / 8); idx += 256) {
@@ -116,49 +72,15 @@ __global__ void gemm_m16_kernel(const short* __restrict__ x,
     int pl = 0;
     const int pl_end = tk / 64;
     for (; pl + 4 <= pl_end; pl += 4) {  // 4 pairs, all weight loads first
-      int4 wq8[4];
-      int4 wq4[2];
       bf16x8 wb[4][2];
-      float sv[4];
-      if (QBITS == 8) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int p = (k0 / 64) + pl + u;
-          wq8[u] = *reinterpret_cast<const int4*>(&wrow_q[p * 64 + woff]);
-          sv[u] = bits2f(srow[(p * 64) / G]);
-        }
-      } else if (QBITS == 4) {
-#pragma unroll
-        for (int v = 0; v < 2; ++v) {
-          const int quad = ((k0 / 64) + pl) / 2 + v;
-          wq4[v] = *reinterpret_cast<const int4*>(&wrow_q4[quad * 64 + woff]);
-          sv[v] = bits2f(srow[(quad * 128) / G]);
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int p = (k0 / 64) + pl + u;
-          wb[u][0] = *reinterpret_cast<const bf16x8*>(&wrow_b[p * 64 + ks]);
-          wb[u][1] = *reinterpret_cast<const bf16x8*>(
-              &wrow_b[p * 64 + 32 + ks]);
-        }
-      }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        bf16x8 b0, b1;
-        if (QBITS == 8) {
-          const int8_t* q8 = reinterpret_cast<const int8_t*>(&wq8[u]);
-          b0 = deq8(q8, sv[u]);
-          b1 = deq8(q8 + 8, sv[u]);
-        } else if (QBITS == 4) {
-          const uint8_t* q4 =
-              reinterpret_cast<const uint8_t*>(&wq4[u / 2]) + (u & 1) * 8;
-          b0 = deq4(q4, sv[u / 2]);
-          b1 = deq4(q4 + 4, sv[u / 2]);
-        } else {
-          b0 = wb[u][0];
-          b1 = wb[u][1];
-        }
+        const int p = (k0 / 64) + pl + u;
+        wb[u][0] = *reinterpret_cast<const bf16x8*>(&wrow[p * 64 + ks]);
+        wb[u][1] = *reinterpret_cast<const bf16x8*>(&wrow[p * 64 + 32 + ks]);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
           const short* at = arow + t * 16 * SE;
@@ -167,34 +89,17 @@ __global__ void gemm_m16_kernel(const short* __restrict__ x,
           const bf16x8 a1 =
               *reinterpret_cast<const bf16x8*>(&at[(pl + u) * 64 + 32 + ks]);
           acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              a0, b0, acc[t][0], 0, 0, 0);
+              a0, wb[u][0], acc[t][0], 0, 0, 0);
           acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              a1, b1, acc[t][1], 0, 0, 0);
+              a1, wb[u][1], acc[t][1], 0, 0, 0);
         }
-      }
     }
     for (; pl < pl_end; ++pl) {
       const int p = (k0 / 64) + pl;
-      bf16x8 b0, b1;
-      if (QBITS == 8) {
-        const int4 wq = *reinterpret_cast<const int4*>(&wrow_q[p * 64 + woff]);
-        const int8_t* q8 = reinterpret_cast<const int8_t*>(&wq);
-        const float sv = bits2f(srow[(p * 64) / G]);
-        b0 = deq8(q8, sv);
-        b1 = deq8(q8 + 8, sv);
-      } else if (QBITS == 4) {
-        const int quad = p / 2;
-        const int half = p & 1;
-        const int2 wq = *reinterpret_cast<const int2*>(
-            &wrow_q4[quad * 64 + woff + half * 8]);
-        const uint8_t* q4 = reinterpret_cast<const uint8_t*>(&wq);
-        const float sv = bits2f(srow[(quad * 128) / G]);
-        b0 = deq4(q4, sv);
-        b1 = deq4(q4 + 4, sv);
-      } else {
-        b0 = *reinterpret_cast<const bf16x8*>(&wrow_b[p * 64 + ks]);
-        b1 = *reinterpret_cast<const bf16x8*>(&wrow_b[p * 64 + 32 + ks]);
-      }
+      const bf16x8 b0 =
+          *reinterpret_cast<const bf16x8*>(&wrow[p * 64 + ks]);
+      const bf16x8 b1 =
+          *reinterpret_cast<const bf16x8*>(&wrow[p * 64 + 32 + ks]);
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
         const short* at = arow + t * 16 * SE;
@@ -231,406 +136,244 @@ __global__ void gemm_m16_kernel(const short* __restrict__ x,
 }
 
 // ---------------------------------------------------------------------------
-// Streamed int8/int4 schedule (round-2).
+// int8 / int4 weights (packed layouts), up to 64 rows.
 //
-// The generic kernel above is pair-rate bound on quantized weights: PMC
-// showed SQ_WAIT 69% with int8 wall time == bf16 wall time at every shape
-// (profiles/r01_gemm_ubench.md) — hipcc keeps only ~2 weight loads in
-// flight and serializes the x staging as load;vmcnt(0);ds_write per chunk
-// (one full round trip per 16-byte chunk). Per 256-k x-tile this schedule
-// instead takes ONE combined round trip:
-//
-//   raw s_barrier (lgkmcnt only — previous tile's consumers done)
-//   issue x staging as global_load_lds DMA (no VGPR round trip)
-//   ONE asm block: issue the tile's weight+scale loads, s_waitcnt vmcnt(0)
-//   raw s_barrier
-//   dequant + MFMA from registers (no VMEM waits at all)
-//
-// The weight loads and the staging DMA are all in flight together
-// (10-14 VMEM ops, 5-9 KB per lane-group), so their latencies overlap in
-// one drain; wave overlap (4 blocks x 4 waves / CU) covers the per-wave
-// consume phase. Every async VMEM value is produced AND waited for
-// INSIDE a single asm statement: hipcc models asm outputs as ready when
-// the statement ends, so an async result that escapes a statement before
-// its s_waitcnt can be copied/rematerialized from an in-flight register
-// (measured: garbage numerics and corrupted-address page faults from the
-// earlier cross-tile ping-pong prefetch). Outputs are early-clobber so
-// the in-flight destinations can never alias the address operands.
-//
-// glds writes LDS at (wave-uniform base + lane*16), so the LDS x image is
-// UNPADDED (16*MT rows x 32 16B-chunks); bank conflicts on the 16-lane
-// fragment reads are killed by an XOR swizzle applied on the SOURCE
-// address instead of row padding (guide §5 rule 21): source chunk c lands
-// at image chunk c ^ (row & 15) — the 16 reader lanes (rows 0..15, same
-// c) then touch 16 different 16B slots = all 64 LDS banks.
+// The weight stream bounds it; what has to stay out of its way are the
+// conversion to bf16, the reads of x from LDS and the barriers.
+//   * 4 waves, each with 16 NF columns of its own and all rows: a fragment of x
+//     read from LDS serves NF fragments of weights.
+//   * x goes through LDS in chunks of KC columns, two of them: the next chunk's
+//     x and weights are loaded into registers before the products of this one,
+//     x is written to the other buffer after them, one barrier per chunk. The
+//     barrier waits for LDS only, the weights stay in flight across it.
+//   * weights are multiplied as whole numbers (exact in bf16), their scale
+//     applies to the fp32 sums of one 16 B load's width (64 or 128 columns):
+//     one vector operation per four results instead of one per weight, and no
+//     rounding of scale x weight.
+//   * the inner dimension is split by chunks over gridDim.y where the columns
+//     alone leave CUs idle (fp32 atomics into the scratch).
+// Measured, MI355X, 5120 x 55296 / 27648 x 5120 / 5120 x 152064 (K x N):
+// int8, 8 rows 68 -> 67, 46 -> 38, 175 -> 174 us (4.2, 3.8, 4.5 TB/s); 64 rows
+// 108 -> 98, 66 -> 56, 267 -> 237 us; int4, 8 rows 56 -> 44, 40 -> 26, 134 ->
+// 116 us; 64 rows 91 -> 79, 57 -> 46, 230 -> 190 us. Before: one 16-column
+// fragment per wave, a drained round trip per chunk or two, weights rounded to
+// bf16 after scaling (error of the fp32 sums against 64 bits 1.6e-3, now 1e-7).
+// Reading a row's scales by one load per chunk instead of one per weight load
+// was a third of the time. What remains is a rate per CU and chunk that does
+// not depend on the number of waves.
+// Columns past the end of K repeat the last ones with a scale of zero: no
+// branch stands between products and the reads of their results.
 // ---------------------------------------------------------------------------
 
 using i32x4 = __attribute__((ext_vector_type(4))) int;
 
-// NSC = scales per 256-k tile = 256/G (G compile-time via dispatch; the
-// host streams only G in {64,128}, and requires the split start k to be
-// G-aligned so the in-tile scale index u*NSC/4 is exact).
-template <int QBITS, int NSC>
-struct WSet {
-  i32x4 w[QBITS == 8 ? 4 : 2];
-  unsigned s[NSC];
-};
-
-// Load one tile's weights+scales and drain: single asm statement (see
-// header comment). wb already includes the lane's row offset
-// (n_w*K + woff) plus the tile's k byte offset; sb points at the tile's
-// first scale.
-template <int QBITS, int NSC>
-__device__ __forceinline__ void wset_load(WSet<QBITS, NSC>& o,
-                                          const void* wb, const short* sb) {
-  if constexpr (QBITS == 8 && NSC == 2) {
-    asm volatile(
-        "global_load_dwordx4 %0, %6, off\n\t"
-        "global_load_dwordx4 %1, %6, off offset:64\n\t"
-        "global_load_dwordx4 %2, %6, off offset:128\n\t"
-        "global_load_dwordx4 %3, %6, off offset:192\n\t"
-        "global_load_ushort %4, %7, off\n\t"
-        "global_load_ushort %5, %7, off offset:2\n\t"
-        "s_waitcnt vmcnt(0)"
-        : "=&v"(o.w[0]), "=&v"(o.w[1]), "=&v"(o.w[2]), "=&v"(o.w[3]),
-          "=&v"(o.s[0]), "=&v"(o.s[1])
-        : "v"(wb), "v"(sb)
-        : "memory");
-  } else if constexpr (QBITS == 8 && NSC == 4) {
-    asm volatile(
-        "global_load_dwordx4 %0, %8, off\n\t"
-        "global_load_dwordx4 %1, %8, off offset:64\n\t"
-        "global_load_dwordx4 %2, %8, off offset:128\n\t"
-        "global_load_dwordx4 %3, %8, off offset:192\n\t"
-        "global_load_ushort %4, %9, off\n\t"
-        "global_load_ushort %5, %9, off offset:2\n\t"
-        "global_load_ushort %6, %9, off offset:4\n\t"
-        "global_load_ushort %7, %9, off offset:6\n\t"
-        "s_waitcnt vmcnt(0)"
-        : "=&v"(o.w[0]), "=&v"(o.w[1]), "=&v"(o.w[2]), "=&v"(o.w[3]),
-          "=&v"(o.s[0]), "=&v"(o.s[1]), "=&v"(o.s[2]), "=&v"(o.s[3])
-        : "v"(wb), "v"(sb)
-        : "memory");
-  } else {
-    static_assert(QBITS == 4 && NSC == 2, "unsupported stream variant");
-    asm volatile(
-        "global_load_dwordx4 %0, %4, off\n\t"
-        "global_load_dwordx4 %1, %4, off offset:64\n\t"
-        "global_load_ushort %2, %5, off\n\t"
-        "global_load_ushort %3, %5, off offset:2\n\t"
-        "s_waitcnt vmcnt(0)"
-        : "=&v"(o.w[0]), "=&v"(o.w[1]), "=&v"(o.s[0]), "=&v"(o.s[1])
-        : "v"(wb), "v"(sb)
-        : "memory");
-  }
-}
-
-// 2-tile weight batch: one statement issues BOTH tiles' weights (+ the
-// first tile's staging already in flight) and drains once — halves the
-// exposed weight round trips vs per-tile loads. Values are final at the
-// statement end, so holding tile B's registers across tile A's consume
-// and tile B's staging is safe (only IN-FLIGHT values must not escape).
-template <int QBITS, int NSC>
-struct WSet2 {
-  i32x4 w[QBITS == 8 ? 8 : 4];
-  unsigned s[2 * NSC];
-};
-
-template <int QBITS, int NSC>
-__device__ __forceinline__ void wset_load2(WSet2<QBITS, NSC>& o,
-                                           const void* wb, const short* sb) {
-  if constexpr (QBITS == 8 && NSC == 2) {
-    asm volatile(
-        "global_load_dwordx4 %0, %12, off\n\t"
-        "global_load_dwordx4 %1, %12, off offset:64\n\t"
-        "global_load_dwordx4 %2, %12, off offset:128\n\t"
-        "global_load_dwordx4 %3, %12, off offset:192\n\t"
-        "global_load_dwordx4 %4, %12, off offset:256\n\t"
-        "global_load_dwordx4 %5, %12, off offset:320\n\t"
-        "global_load_dwordx4 %6, %12, off offset:384\n\t"
-        "global_load_dwordx4 %7, %12, off offset:448\n\t"
-        "global_load_ushort %8, %13, off\n\t"
-        "global_load_ushort %9, %13, off offset:2\n\t"
-        "global_load_ushort %10, %13, off offset:4\n\t"
-        "global_load_ushort %11, %13, off offset:6\n\t"
-        "s_waitcnt vmcnt(0)"
-        : "=&v"(o.w[0]), "=&v"(o.w[1]), "=&v"(o.w[2]), "=&v"(o.w[3]),
-          "=&v"(o.w[4]), "=&v"(o.w[5]), "=&v"(o.w[6]), "=&v"(o.w[7]),
-          "=&v"(o.s[0]), "=&v"(o.s[1]), "=&v"(o.s[2]), "=&v"(o.s[3])
-        : "v"(wb), "v"(sb)
-        : "memory");
-  } else if constexpr (QBITS == 8 && NSC == 4) {
-    asm volatile(
-        "global_load_dwordx4 %0, %16, off\n\t"
-        "global_load_dwordx4 %1, %16, off offset:64\n\t"
-        "global_load_dwordx4 %2, %16, off offset:128\n\t"
-        "global_load_dwordx4 %3, %16, off offset:192\n\t"
-        "global_load_dwordx4 %4, %16, off offset:256\n\t"
-        "global_load_dwordx4 %5, %16, off offset:320\n\t"
-        "global_load_dwordx4 %6, %16, off offset:384\n\t"
-        "global_load_dwordx4 %7, %16, off offset:448\n\t"
-        "global_load_ushort %8, %17, off\n\t"
-        "global_load_ushort %9, %17, off offset:2\n\t"
-        "global_load_ushort %10, %17, off offset:4\n\t"
-        "global_load_ushort %11, %17, off offset:6\n\t"
-        "global_load_ushort %12, %17, off offset:8\n\t"
-        "global_load_ushort %13, %17, off offset:10\n\t"
-        "global_load_ushort %14, %17, off offset:12\n\t"
-        "global_load_ushort %15, %17, off offset:14\n\t"
-        "s_waitcnt vmcnt(0)"
-        : "=&v"(o.w[0]), "=&v"(o.w[1]), "=&v"(o.w[2]), "=&v"(o.w[3]),
-          "=&v"(o.w[4]), "=&v"(o.w[5]), "=&v"(o.w[6]), "=&v"(o.w[7]),
-          "=&v"(o.s[0]), "=&v"(o.s[1]), "=&v"(o.s[2]), "=&v"(o.s[3]),
-          "=&v"(o.s[4]), "=&v"(o.s[5]), "=&v"(o.s[6]), "=&v"(o.s[7])
-        : "v"(wb), "v"(sb)
-        : "memory");
-  } else {
-    static_assert(QBITS == 4 && NSC == 2, "unsupported stream variant");
-    asm volatile(
-        "global_load_dwordx4 %0, %8, off\n\t"
-        "global_load_dwordx4 %1, %8, off offset:64\n\t"
-        "global_load_dwordx4 %2, %8, off offset:128\n\t"
-        "global_load_dwordx4 %3, %8, off offset:192\n\t"
-        "global_load_ushort %4, %9, off\n\t"
-        "global_load_ushort %5, %9, off offset:2\n\t"
-        "global_load_ushort %6, %9, off offset:4\n\t"
-        "global_load_ushort %7, %9, off offset:6\n\t"
-        "s_waitcnt vmcnt(0)"
-        : "=&v"(o.w[0]), "=&v"(o.w[1]), "=&v"(o.w[2]), "=&v"(o.w[3]),
-          "=&v"(o.s[0]), "=&v"(o.s[1]), "=&v"(o.s[2]), "=&v"(o.s[3])
-        : "v"(wb), "v"(sb)
-        : "memory");
-  }
-}
-
-template <int MT, bool GLDS>
-__device__ __forceinline__ void stage_tile(const short* __restrict__ x,
-                                           short* x_lds, const int k0,
-                                           const int M, const int K) {
-  constexpr int NSG = MT * 2;  // glds per wave (1 KB each)
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  asm volatile("s_barrier" ::: "memory");
-  const int wavei = (int)threadIdx.x >> 6, lanei = (int)threadIdx.x & 63;
-  if constexpr (GLDS) {
-#pragma unroll
-    for (int g = 0; g < NSG; ++g) {
-      const int L = (wavei * NSG + g) * 64 + lanei;  // image chunk
-      const int r = L >> 5;
-      const int cs = (L & 31) ^ (r & 15);            // source chunk (swizzle)
-      const short* ga = &x[(int64_t)min(r, M - 1) * K + k0 + cs * 8];
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)ga,
-          (__attribute__((address_space(3))) void*)&x_lds[(wavei * NSG + g) *
-                                                          64 * 8],
-          16, 0, 0);
-    }
-  } else {
-    // debug/fallback: same swizzled image via plain loads + ds_write
-#pragma unroll
-    for (int g = 0; g < NSG; ++g) {
-      const int L = (wavei * NSG + g) * 64 + lanei;
-      const int r = L >> 5;
-      const int cs = (L & 31) ^ (r & 15);
-      *reinterpret_cast<short8*>(&x_lds[L * 8]) =
-          *reinterpret_cast<const short8*>(
-              &x[(int64_t)min(r, M - 1) * K + k0 + cs * 8]);
-    }
-  }
-}
-
-template <bool GLDS>
-__device__ __forceinline__ void end_stage() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  asm volatile("s_barrier" ::: "memory");
-  if constexpr (GLDS)  // DS ops bound-check against m0 on gfx9-family
-    asm volatile("s_mov_b32 m0, -1" ::: "memory");
-}
-
-// dequant + MFMA for one tile's 4 pairs from already-final registers
-template <int QBITS, int MT, int NSC>
-__device__ __forceinline__ void consume_tile(const i32x4* __restrict__ wv,
-                                             const unsigned* __restrict__ sc,
-                                             short* x_lds,
-                                             f32x4 (&acc)[MT][2],
-                                             const int row, const int ks) {
-  const int ln4 = ks >> 3;  // lane>>4
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    bf16x8 b0, b1;
-    if (QBITS == 8) {
-      const int8_t* q8 = reinterpret_cast<const int8_t*>(&wv[u]);
-      const float sv = bits2f((short)sc[u * NSC / 4]);
-      b0 = deq8(q8, sv);
-      b1 = deq8(q8 + 8, sv);
-    } else {
-      const uint8_t* q4 =
-          reinterpret_cast<const uint8_t*>(&wv[u / 2]) + (u & 1) * 8;
-      const float sv = bits2f((short)sc[(u / 2) * NSC / 2]);
-      b0 = deq4(q4, sv);
-      b1 = deq4(q4 + 4, sv);
-    }
-    const int c0 = (u * 8 + ln4) ^ row;      // swizzled image chunks
-    const int c1 = (u * 8 + 4 + ln4) ^ row;
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      const short* rb = &x_lds[(t * 16 + row) * 256];
-      const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(&rb[c0 * 8]);
-      const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(&rb[c1 * 8]);
-      acc[t][0] =
-          __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[t][0], 0, 0, 0);
-      acc[t][1] =
-          __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[t][1], 0, 0, 0);
-    }
-  }
-}
-
-// MINW: min waves per EU hint (occupancy/VGPR trade, see profiles/).
-template <int QBITS, int MT, int NSC, int MINW, bool GLDS = true>
-__global__ __launch_bounds__(256, MINW) void gemm_m16_stream_kernel(
+// NG: scales of a row and chunk, read by one load (groups of KC / NG columns, K
+// a multiple of KC); 0: one scale per 16 B load, any group.
+template <int BITS, int MT, int NF, int KC, int NG>
+__global__ __launch_bounds__(256, MT == 4 ? 2 : 3) void gemm_q_kernel(
     const short* __restrict__ x, const void* __restrict__ w,
     const short* __restrict__ scales, const short* __restrict__ bias,
     short* __restrict__ out, float* __restrict__ out_f32, const int M,
     const int K, const int N, const int G, const int splitk) {
-  constexpr int XT = 256;
-  __shared__ short x_lds[16 * MT * XT];  // unpadded (glds image, swizzled)
-  const int wave = threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int n0 = (blockIdx.x * 4 + wave) * 16;
-  const int row = lane & 15;
-  const int ks = (lane >> 4) * 8;
-  const int n_w = min(n0 + row, N - 1);
+  constexpr int SW = BITS == 8 ? 64 : 128;   // columns of a lane group's load
+  constexpr int NS = KC / SW;                // loads per row and chunk
+  constexpr int NJ = SW / 32;                // products per load
+  constexpr int R = 16 * MT;
+  constexpr int XP = KC + 8;                 // LDS pitch: 16 rows of a 16 B
+                                             // column fall into all banks
+  constexpr int XL = R * KC / 8 / 256;       // 16 B of x per thread and chunk
+  static_assert(XL * 256 * 8 == R * KC, "chunk");
+  __shared__ __attribute__((aligned(16))) short x_lds[2][R * XP];
+  const int wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int c = lane & 15, hi = lane >> 4;
+  const int n0 = (blockIdx.x * 4 + wave) * (16 * NF);
+  const int chunks = (K + KC - 1) / KC;
+  const int per = (chunks + splitk - 1) / splitk;
+  const int c0 = blockIdx.y * per, c1 = min(chunks, c0 + per);
+  if (c0 >= c1) return;
 
-  const int pairs = K / 64;
-  int p_begin, p_end;
-  if (QBITS == 4) {
-    const int quads = K / 128;
-    const int qq = quads / splitk;
-    p_begin = blockIdx.y * qq * 2;
-    p_end = (blockIdx.y == splitk - 1) ? quads * 2 : p_begin + qq * 2;
+  const int rb = BITS == 8 ? K : K / 2;      // bytes of a weight row
+  const int gs = G / SW;                     // loads per scale
+  const uint64_t ginv = ((1ull << 32) + gs - 1) / gs;
+  const char* wp[NF];
+  const short* sp[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    const int64_t row = min(n0 + f * 16 + c, N - 1);
+    wp[f] = (const char*)w + row * rb + hi * 16;
+    sp[f] = scales + row * (K / G);
+  }
+  f32x4 acc[MT][NF];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int f = 0; f < NF; ++f) acc[m][f] = {0.f, 0.f, 0.f, 0.f};
+
+  constexpr int NSC = NG ? NG : NS;          // scales of a chunk
+  constexpr int UG = NS / NSC;               // loads per scale
+  struct Weights {
+    i32x4 w[NS][NF];
+    unsigned s[NF][(NSC + 1) / 2];           // bf16 bits, two a word
+  };
+  const int loads = K / SW;                  // of a whole row
+  auto load_w = [&](Weights& q, const int ch) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+#pragma unroll
+      for (int u = 0; u < NS; ++u) {
+        const int at = NG ? ch * NS + u : min(ch * NS + u, loads - 1);
+        q.w[u][f] = *reinterpret_cast<const i32x4*>(wp[f] + at * 64);
+      }
+      if constexpr (NG == 4) {
+        const uint2 v = *reinterpret_cast<const uint2*>(sp[f] + ch * 4);
+        q.s[f][0] = v.x;
+        q.s[f][1] = v.y;
+      } else if constexpr (NG == 2) {
+        q.s[f][0] = *reinterpret_cast<const unsigned*>(sp[f] + ch * 2);
+      } else {
+#pragma unroll
+        for (int u = 0; u < NS; ++u) {
+          const int at = min(ch * NS + u, loads - 1);
+          const unsigned v =
+              ch * NS + u < loads
+                  ? (unsigned short)sp[f][((uint64_t)at * ginv) >> 32] : 0u;
+          q.s[f][u / 2] = u & 1 ? q.s[f][u / 2] | v << 16 : v;
+        }
+      }
+    }
+  };
+  i32x4 xr[XL];
+  auto load_x = [&](const int ch) {
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+      const int e = i * 256 + threadIdx.x;
+      const int k = min(ch * KC + e % (KC / 8) * 8, K - 8);
+      // rows >= M repeat the last one; their results are never stored
+      xr[i] = *reinterpret_cast<const i32x4*>(
+          &x[(int64_t)min(e / (KC / 8), M - 1) * K + k]);
+    }
+  };
+  auto store_x = [&](const int buf) {
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+      const int e = i * 256 + threadIdx.x;
+      *reinterpret_cast<i32x4*>(
+          &x_lds[buf][e / (KC / 8) * XP + e % (KC / 8) * 8]) = xr[i];
+    }
+    // LDS only: the weights in flight are waited for where they are used
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  auto mul = [&](const Weights& q, const int buf) {
+#pragma unroll
+    for (int g = 0; g < NSC; ++g) {
+      f32x4 p[MT][NF];
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) p[m][f] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int uu = 0; uu < UG; ++uu) {
+        const int u = g * UG + uu;
+        bf16x8 b[NF][NJ];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          // ties the conversions to this place: moved up to the load, a
+          // chunk's weights take four times the registers
+          i32x4 v = q.w[u][f];
+          asm volatile("" : "+v"(v));
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              if (BITS == 8)
+                b[f][j][e] = (__bf16)(float)(signed char)(
+                    v[2 * j + e / 4] >> (8 * (e & 3)));
+              else       // nibbles are stored offset by 8
+                b[f][j][e] = (__bf16)(float)(
+                    (int)((unsigned)(v[j] ^ 0x88888888) << (28 - 4 * e)) >>
+                    28);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) {
+            const bf16x8 a = *reinterpret_cast<const bf16x8*>(
+                &x_lds[buf][(m * 16 + c) * XP + u * SW + j * 32 + hi * 8]);
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+              p[m][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  a, b[f][j], p[m][f], 0, 0, 0);
+          }
+        // one load's conversions at a time
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        const float sc = __builtin_bit_cast(
+            float, g & 1 ? q.s[f][g / 2] & 0xffff0000u : q.s[f][g / 2] << 16);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            acc[m][f][r] = fmaf(sc, p[m][f][r], acc[m][f][r]);
+      }
+    }
+  };
+  // every workgroup starts at another chunk: in step they would all read the
+  // same columns of rows that lie a multiple of 256 B apart, a few channels
+  const int n_ch = c1 - c0;
+  const int turn = (int)((blockIdx.x * 5 + blockIdx.y * 3) % n_ch);
+  auto place = [&](int i) {
+    i += turn;
+    return c0 + (i < n_ch ? i : i - n_ch);
+  };
+  Weights q0, q1;
+  load_x(place(0));
+  load_w(q0, place(0));
+  store_x(0);
+  int i = 0;
+  for (; i + 2 < n_ch; i += 2) {
+    load_x(place(i + 1));
+    load_w(q1, place(i + 1));
+    __builtin_amdgcn_sched_barrier(0);
+    mul(q0, 0);
+    store_x(1);
+    load_x(place(i + 2));
+    load_w(q0, place(i + 2));
+    __builtin_amdgcn_sched_barrier(0);
+    mul(q1, 1);
+    store_x(0);
+  }
+  if (i + 1 < n_ch) {
+    load_x(place(i + 1));
+    load_w(q1, place(i + 1));
+    __builtin_amdgcn_sched_barrier(0);
+    mul(q0, 0);
+    store_x(1);
+    mul(q1, 1);
   } else {
-    const int pp = pairs / splitk;
-    p_begin = blockIdx.y * pp;
-    p_end = (blockIdx.y == splitk - 1) ? pairs : p_begin + pp;
+    mul(q0, 0);
   }
-  const int woff = (lane >> 4) * 16;
 
-  f32x4 acc[MT][2];
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
+  for (int f = 0; f < NF; ++f) {
+    const int n = n0 + f * 16 + c;
+    if (n >= N) continue;
+    const float bv =
+        splitk == 1 && bias != nullptr ? bits2f(bias[n]) : 0.f;
 #pragma unroll
-    for (int u = 0; u < 2; ++u) acc[t][u] = {0.f, 0.f, 0.f, 0.f};
-
-  const void* wrow =
-      QBITS == 8
-          ? (const void*)((const int8_t*)w + (int64_t)n_w * K + woff)
-          : (const void*)((const uint8_t*)w + (int64_t)n_w * (K / 2) + woff);
-  const short* srow = scales + (int64_t)n_w * (K / G);
-
-  const int kbeg = p_begin * 64, kend = p_end * 64;
-  const int kfull = kbeg + ((kend - kbeg) / XT) * XT;
-  constexpr int GS = 256 / NSC;
-  int k0 = kbeg;
-  // 2-tile groups: one weight statement serves both tiles (one exposed
-  // round trip instead of two); tile B's staging waits alone
-  for (; k0 + 2 * XT <= kfull; k0 += 2 * XT) {
-    WSet2<QBITS, NSC> w2;
-    stage_tile<MT, GLDS>(x, x_lds, k0, M, K);
-    if (QBITS == 8)
-      wset_load2<QBITS, NSC>(w2, (const int8_t*)wrow + k0, srow + k0 / GS);
-    else
-      wset_load2<QBITS, NSC>(w2, (const uint8_t*)wrow + k0 / 2,
-                             srow + k0 / GS);
-    end_stage<GLDS>();
-    consume_tile<QBITS, MT, NSC>(&w2.w[0], &w2.s[0], x_lds, acc, row, ks);
-    stage_tile<MT, GLDS>(x, x_lds, k0 + XT, M, K);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // staging only
-    end_stage<GLDS>();
-    consume_tile<QBITS, MT, NSC>(&w2.w[QBITS == 8 ? 4 : 2], &w2.s[NSC],
-                                 x_lds, acc, row, ks);
-  }
-  for (; k0 < kfull; k0 += XT) {
-    WSet<QBITS, NSC> w1;
-    stage_tile<MT, GLDS>(x, x_lds, k0, M, K);
-    if (QBITS == 8)
-      wset_load<QBITS, NSC>(w1, (const int8_t*)wrow + k0, srow + k0 / GS);
-    else
-      wset_load<QBITS, NSC>(w1, (const uint8_t*)wrow + k0 / 2,
-                            srow + k0 / GS);
-    end_stage<GLDS>();
-    consume_tile<QBITS, MT, NSC>(&w1.w[0], &w1.s[0], x_lds, acc, row, ks);
-  }
-
-  // tail (< XT k): generic serial staging + pair loop, executed by the
-  // whole block (condition uniform)
-  const int ln4 = ks >> 3;
-  for (; k0 < kend; k0 += XT) {
-    const int tk = kend - k0;  // < XT, multiple of 64
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");
-    for (int idx = threadIdx.x; idx < 16 * MT * (tk / 8); idx += 256) {
-      const int r = idx / (tk / 8);
-      const int vec = idx % (tk / 8);
-      // same swizzled image as the glds path (rows are full 32-chunk
-      // strides even when tk < XT)
-      *reinterpret_cast<short8*>(&x_lds[(r * 32 + (vec ^ (r & 15))) * 8]) =
-          *reinterpret_cast<const short8*>(
-              &x[(int64_t)min(r, M - 1) * K + k0 + vec * 8]);
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");
-    for (int pl = 0; pl < tk / 64; ++pl) {
-      const int p = (k0 / 64) + pl;
-      bf16x8 b0, b1;
-      if (QBITS == 8) {
-        const int8_t* wq = (const int8_t*)wrow;
-        const int4 wv = *reinterpret_cast<const int4*>(&wq[p * 64]);
-        const int8_t* q8 = reinterpret_cast<const int8_t*>(&wv);
-        const float sv = bits2f(srow[(p * 64) / G]);
-        b0 = deq8(q8, sv);
-        b1 = deq8(q8 + 8, sv);
-      } else {
-        const int quad = p / 2;
-        const int half = p & 1;
-        const uint8_t* wq = (const uint8_t*)wrow;
-        const int2 wv =
-            *reinterpret_cast<const int2*>(&wq[quad * 64 + half * 8]);
-        const uint8_t* q4 = reinterpret_cast<const uint8_t*>(&wv);
-        const float sv = bits2f(srow[(quad * 128) / G]);
-        b0 = deq4(q4, sv);
-        b1 = deq4(q4 + 4, sv);
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = m * 16 + hi * 4 + r;
+        if (row >= M) continue;
+        if (splitk > 1)
+          atomicAdd(out_f32 + (int64_t)row * N + n, acc[m][f][r]);
+        else
+          out[(int64_t)row * N + n] = f2bits(acc[m][f][r] + bv);
       }
-      const int c0 = (pl * 8 + ln4) ^ row;
-      const int c1 = (pl * 8 + 4 + ln4) ^ row;
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        const short* rb = &x_lds[(t * 16 + row) * 256];
-        const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(&rb[c0 * 8]);
-        const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(&rb[c1 * 8]);
-        acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[t][0],
-                                                            0, 0, 0);
-        acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[t][1],
-                                                            0, 0, 0);
-      }
-    }
-  }
-
-  const int n = n0 + (lane & 15);
-  if (n >= N) return;
-#pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const f32x4 a2 = acc[t][0] + acc[t][1];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = t * 16 + (lane >> 4) * 4 + r;
-      if (m >= M) continue;
-      if (splitk > 1) {
-        atomicAdd(out_f32 + (int64_t)m * N + n, a2[r]);
-      } else {
-        float v = a2[r];
-        if (bias != nullptr) v += bits2f(bias[n]);
-        out[(int64_t)m * N + n] = f2bits(v);
-      }
-    }
   }
 }
 
@@ -690,10 +433,11 @@ void scratch_clean(torch::Tensor scratch) {
   g_scratch_dirty_elems = 0;
 }
 
-static int pick_splitk(int64_t N, int64_t K, int64_t M, int64_t scratch_elems,
-                       int min_pairs, int g_align) {
-  // Target ~1024 blocks (~4 blocks / 16 waves per CU) so HBM latency is
-  // covered by wave overlap; each split keeps >= 8 K-chunk-pairs of work.
+// Splits of the inner dimension for the bf16 kernel: ~1024 workgroups (4 per CU)
+// so that wave overlap covers the memory's latency; each split keeps 8 x 64
+// columns.
+static int pick_splitk(int64_t N, int64_t K, int64_t M,
+                       int64_t scratch_elems) {
   static const int forced = []() {
     const char* e = getenv("DNET_GEMM_SPLITK");  // debug/bench override
     return e ? atoi(e) : 0;
@@ -702,26 +446,64 @@ static int pick_splitk(int64_t N, int64_t K, int64_t M, int64_t scratch_elems,
   if (forced > 0)
     return (M * N > scratch_elems || (K / 64) < forced) ? 1 : forced;
   int sk = 1;
-  while (sk < 32 && blocks * sk < 1024 &&
-         (K / 64) / (sk * 2) >= min_pairs &&
-         ((K / 64) / (sk * 2)) * 64 % g_align == 0)  // split starts G-aligned
-    sk *= 2;
-  // Measured (profiles/r02, sk sweep): a split span that is not a
-  // multiple of 256 pushes its remainder through the serial tail path;
-  // on SHORT spans that tail dominates (qkv K=5120 sk=8: span 640,
-  // 20% tail, 27.7us vs 23.6us at sk=4). Halve sk when the tail is
-  // >=15% of the span, the halved span is tail-free, and the halved
-  // grid still covers the chip (o N=5120 shows 320 blocks is too few).
+  while (sk < 32 && blocks * sk < 1024 && (K / 64) / (sk * 2) >= 8) sk *= 2;
+  // a span that is no multiple of 256 ends in single steps: half as many splits
+  // where that rest is >= 15 % of the span, twice the span has none and the
+  // grid still covers the chip
   if (sk > 1) {
     const int64_t span = ((K / 64) / sk) * 64;
     const int64_t span2 = ((K / 64) / (sk / 2)) * 64;
     if (span % 256 != 0 && (double)(span % 256) / span >= 0.15 &&
-        span2 % 256 == 0 && span2 % g_align == 0 &&
-        blocks * (sk / 2) >= 440)
+        span2 % 256 == 0 && blocks * (sk / 2) >= 440)
       sk /= 2;
   }
   if (sk > 1 && M * N > scratch_elems) sk = 1;
   return sk;
+}
+
+constexpr int kQChunk = 256, kQCols = 128;   // of gemm_q_kernel
+
+// Splits of the inner dimension for the int8 / int4 kernel, by a model of what
+// was measured over 4096 to 55296 columns, 4096 to 27648 deep, 8 to 64 rows: a
+// CU gets through its workgroups' chunks at a constant rate, whether one or
+// three of them share it, so the fullest CU counts (56 column tiles, 20 chunks,
+// 8 rows: 4 splits, 224 workgroups, 11.9 us; 5 splits, 280 workgroups, 15.7);
+// one workgroup alone is a tenth slower, filling the pipeline costs about 0.6
+// of a chunk per workgroup, and of the splits' atomics, 1.8 TB/s, a quarter
+// shows, more where they exceed 0.4 of the rest (432 tiles, 64 rows: 1 split
+// 94 us, 5 splits 101, 10 splits 141).
+static int pick_splits_q(int64_t N, int64_t K, int64_t M,
+                         int64_t scratch_elems, int bits) {
+  static const int forced = []() {
+    const char* e = getenv("DNET_GEMM_SPLITK");  // debug/bench override
+    return e ? atoi(e) : 0;
+  }();
+  const int chunks = cdiv(K, kQChunk), tiles = cdiv(N, kQCols);
+  if (M * N > scratch_elems) return 1;
+  if (forced > 0) return std::min(forced, chunks);
+  const double chunk_us =
+      (M <= 16 ? 1.5 : M <= 32 ? 1.9 : 2.6) * (bits == 8 ? 1.0 : 0.8);
+  int best = 1;
+  double best_us = 1e30;
+  for (int sk = 1; sk <= std::min(chunks, 32); ++sk) {
+    const int per = cdiv(chunks, sk);
+    if (cdiv(chunks, per) != sk) continue;      // the last ones would be empty
+    const int full = cdiv((int64_t)tiles * sk, 256);
+    const double base = chunk_us * (full == 1 ? 1.1 : full) * (per + 0.6);
+    const double atom = sk > 1 ? (double)sk * M * N * 4 / 1.8e6 : 0.0;
+    const double us = base + std::max(0.25 * atom, atom - 0.4 * base);
+    if (us < best_us) {
+      best_us = us;
+      best = sk;
+    }
+  }
+  return best;
+}
+
+static int pick_splits(int64_t N, int64_t K, int64_t M, int64_t scratch_elems,
+                       int bits) {
+  return bits < 16 ? pick_splits_q(N, K, M, scratch_elems, bits)
+                   : pick_splitk(N, K, M, scratch_elems);
 }
 
 static bool launch_m16(torch::Tensor x, torch::Tensor w,
@@ -732,11 +514,7 @@ static bool launch_m16(torch::Tensor x, torch::Tensor w,
   const int64_t K = x.size(1), N = w.size(0);
   auto stream = current_stream();
   const int64_t scratch_elems = scratch.has_value() ? scratch->numel() : 0;
-  // the streamed schedule tolerates short splits (one combined round
-  // trip per 4-pair tile), so quantized paths split deeper to fill the
-  // 256 CUs on small-N shapes (qkv/o run at <2 blocks/CU otherwise)
-  const int sk = pick_splitk(N, K, M, scratch_elems, bits < 16 ? 4 : 8,
-                             bits < 16 ? std::max<int>((int)group, 64) : 64);
+  const int sk = pick_splits(N, K, M, scratch_elems, bits);
   const short* bptr = bias.has_value() ? (const short*)bias->data_ptr() : nullptr;
   const dim3 grid((unsigned)((N + 63) / 64), sk);
   const short* xp = (const short*)x.data_ptr() + m0 * K;
@@ -763,72 +541,38 @@ static bool launch_m16(torch::Tensor x, torch::Tensor w,
   }
   const short* sp = bits < 16 ? (const short*)scales->data_ptr() : nullptr;
   const short* bp1 = sk > 1 ? nullptr : bptr;
-#define LAUNCH(QQ, TT)                                                      \
-  hipLaunchKernelGGL((gemm_m16_kernel<QQ, TT>), grid, dim3(256), 0, stream, \
-                     xp, w.data_ptr(), sp, bp1, op, fp, M, (int)K, (int)N,  \
-                     group, sk)
-  static const bool mt4occ3 = []() {
-    const char* e = getenv("DNET_GEMM_MT4OCC");
-    return e == nullptr || e[0] == '3';  // default: spill-free 3-wave MT4
-  }();
-  static const bool noglds = getenv("DNET_GEMM_NOGLDS") != nullptr;
-#define LAUNCH_STREAM(QQ, TT, NSC, MW)                                      \
+#define LAUNCH(TT)                                                          \
+  hipLaunchKernelGGL((gemm_m16_kernel<TT>), grid, dim3(256), 0, stream, xp, \
+                     (const short*)w.data_ptr(), bp1, op, fp, M, (int)K,    \
+                     (int)N, sk)
+#define LAUNCH_QN(QQ, TT, FF, KK, GG)                                       \
+  hipLaunchKernelGGL((gemm_q_kernel<QQ, TT, FF, KK, GG>),                   \
+                     dim3((unsigned)cdiv(N, 64 * FF), sk), dim3(256), 0,    \
+                     stream, xp, w.data_ptr(), sp, bp1, op, fp, M, (int)K,  \
+                     (int)N, group, sk)
+#define LAUNCH_Q(QQ, TT, FF, KK)                                            \
   do {                                                                      \
-    if (noglds)                                                             \
-      hipLaunchKernelGGL((gemm_m16_stream_kernel<QQ, TT, NSC, MW, false>), \
-                         grid, dim3(256), 0, stream, xp, w.data_ptr(), sp,  \
-                         bp1, op, fp, M, (int)K, (int)N, group, sk);        \
-    else                                                                    \
-      hipLaunchKernelGGL((gemm_m16_stream_kernel<QQ, TT, NSC, MW, true>),   \
-                         grid, dim3(256), 0, stream, xp, w.data_ptr(), sp,  \
-                         bp1, op, fp, M, (int)K, (int)N, group, sk);        \
+    if (K % 256 == 0 && group == 128) LAUNCH_QN(QQ, TT, FF, KK, 2);         \
+    else if (QQ == 8 && K % 256 == 0 && group == 64)                        \
+      LAUNCH_QN(QQ, TT, FF, KK, QQ == 8 ? 4 : 0);                           \
+    else LAUNCH_QN(QQ, TT, FF, KK, 0);                                      \
   } while (0)
-#define LAUNCH_STREAM_G8(TT)                                            \
-  do {                                                                    \
-    if (TT == 4 && mt4occ3) {                                             \
-      if (group == 64) LAUNCH_STREAM(8, TT, 4, 3);                        \
-      else LAUNCH_STREAM(8, TT, 2, 3);                                    \
-    } else {                                                              \
-      if (group == 64) LAUNCH_STREAM(8, TT, 4, 4);                        \
-      else LAUNCH_STREAM(8, TT, 2, 4);                                    \
-    }                                                                     \
+#define LAUNCH_QB(QQ)                                                       \
+  do {                                                                      \
+    if (M > 32) LAUNCH_Q(QQ, 4, 2, 256);                                    \
+    else if (M > 16) LAUNCH_Q(QQ, 2, 2, 256);                               \
+    else LAUNCH_Q(QQ, 1, 2, 256);                                           \
   } while (0)
-#define LAUNCH_STREAM_G4(TT)                                              \
-  do {                                                                    \
-    if (TT == 4 && mt4occ3) LAUNCH_STREAM(4, TT, 2, 3);                   \
-    else LAUNCH_STREAM(4, TT, 2, 4);                                      \
-  } while (0)
-  // the streamed counted-vmcnt schedule needs a compile-time scale count
-  // per 256-k tile; other group sizes fall back to the generic kernel
-  // G must divide every tile start (k0 is any multiple of 64 under
-  // split-k partitioning, and the in-tile scale index u*NSC/4 assumes
-  // k0 % G == 0), so only G <= 128 streams; G=256 falls back
-  // additionally every split start kbeg = by*(pairs/sk)*64 must be
-  // G-aligned (the in-tile scale index assumes k0 % G == 0)
-  const bool split_aligned =
-      group > 0 && (sk == 1 || ((K / 64 / sk) * 64) % group == 0);
-  const bool can_stream =
-      split_aligned && ((bits == 8 && (group == 64 || group == 128)) ||
-                        (bits == 4 && group == 128));
-  static const bool nostream = getenv("DNET_GEMM_NOSTREAM") != nullptr;
-  const bool use_stream = can_stream && !nostream;
-  if (bits == 8) {
-    if (M > 32) { if (use_stream) LAUNCH_STREAM_G8(4); else LAUNCH(8, 4); }
-    else if (M > 16) { if (use_stream) LAUNCH_STREAM_G8(2); else LAUNCH(8, 2); }
-    else { if (use_stream) LAUNCH_STREAM_G8(1); else LAUNCH(8, 1); }
-  } else if (bits == 4) {
-    if (M > 32) { if (use_stream) LAUNCH_STREAM_G4(4); else LAUNCH(4, 4); }
-    else if (M > 16) { if (use_stream) LAUNCH_STREAM_G4(2); else LAUNCH(4, 2); }
-    else { if (use_stream) LAUNCH_STREAM_G4(1); else LAUNCH(4, 1); }
-  } else {
-    if (M > 32) LAUNCH(16, 4);
-    else if (M > 16) LAUNCH(16, 2);
-    else LAUNCH(16, 1);
+  if (bits == 8) LAUNCH_QB(8);
+  else if (bits == 4) LAUNCH_QB(4);
+  else {
+    if (M > 32) LAUNCH(4);
+    else if (M > 16) LAUNCH(2);
+    else LAUNCH(1);
   }
 #undef LAUNCH
-#undef LAUNCH_STREAM
-#undef LAUNCH_STREAM_G8
-#undef LAUNCH_STREAM_G4
+#undef LAUNCH_Q
+#undef LAUNCH_QB
   if (sk > 1) {
     // defer_combine: the caller's next kernel reads (and re-zeroes) the
     // f32 scratch itself — skip the convert/bias pass
@@ -849,8 +593,7 @@ static bool launch_m16(torch::Tensor x, torch::Tensor w,
 bool gemm_m16_will_defer(int64_t M, int64_t N, int64_t K, int64_t group,
                          int64_t bits, int64_t scratch_elems) {
   if (M > 64 || M <= 2) return false;
-  const int sk = pick_splitk(N, K, M, scratch_elems, bits < 16 ? 4 : 8,
-                             bits < 16 ? std::max<int>((int)group, 64) : 64);
+  const int sk = pick_splits(N, K, M, scratch_elems, bits);
   return sk > 1;
 }
 

@@ -1049,3 +1049,45 @@ def test_rope_prefill(d, norm):
     assert torch.equal(vc[:, :, p0:p0 + T].transpose(1, 2), wv)
     before[:, 1:, :, p0:p0 + T] = full[:, 1:, :, p0:p0 + T]
     assert torch.equal(full, before)
+
+
+@pytest.mark.parametrize("M", [3, 16, 17, 33, 64])
+@pytest.mark.parametrize("bits,N,K,G", [
+    (8, 200, 320, 64),       # columns end inside a tile, a chunk inside K
+    (8, 136, 64, 64),        # one load per row
+    (8, 256, 1024, 64),      # four scales per chunk, splits
+    (8, 1000, 2560, 128),
+    (8, 72, 768, 192),       # groups that no chunk divides into
+    (8, 64, 1024, 256),
+    (4, 200, 384, 128),
+    (4, 136, 128, 128),
+    (4, 1000, 2560, 128),
+    (4, 72, 768, 256),
+])
+def test_gemm_quant_chunk_edges(bits, N, K, G, M):
+    """Packed int8 / int4 weights, with and without splits and bias. Whole
+    numbers are exact, the sums fp32: within (K + 8) 2^-24 of sum |x w|, then
+    bf16 (2^-8)."""
+    torch.manual_seed(N + M)
+    dev = _dev()
+    x = torch.randn(M, K, dtype=torch.bfloat16)
+    w = (torch.randn(N, K) / K ** 0.5).to(torch.bfloat16)
+    bias = torch.randn(N, dtype=torch.bfloat16)
+    if bits == 8:
+        q, s = ops.quantize_int8(w, G)
+        codes, packed, f = q, ops.pack_int8_mfma(q), ops.gemv_int8
+    else:
+        q, s = ops.quantize_int4(w, G)
+        codes, packed, f = ref.unpack_int4(q), ops.pack_int4_mfma(q), \
+            ops.gemv_int4
+    w64 = (codes.double().view(N, K // G, G)
+           * s.double().unsqueeze(-1)).view(N, K)
+    want = x.double() @ w64.t()
+    mass = x.double().abs() @ w64.abs().t()
+    for b in (None, bias):
+        ref64 = want if b is None else want + b.double()
+        got = f(x.to(dev), packed.to(dev), s.to(dev), G,
+                None if b is None else b.to(dev), True).double().cpu()
+        bound = mass * (K + 8) * 2 ** -24 + ref64.abs() * 2 ** -8 \
+            + (0 if b is None else b.double().abs() * 2 ** -22)
+        assert ((got - ref64).abs() <= bound).all()
