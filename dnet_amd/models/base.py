@@ -119,6 +119,16 @@ class Linear:
                                     self.packed)
         return self.w
 
+    def small_m(self, x: torch.Tensor) -> bool:
+        """x's rows go through the small-M GPU product in its packed or bf16
+        form, whose split sums a fused consumer can read (ops.gemv_*)."""
+        m = x.shape[0]
+        if not x.is_cuda or m > GEMV_MAX_M or x.dtype != torch.bfloat16:
+            return False
+        if self.is_quant:
+            return self.packed and not self.mxfp4 and m > 2
+        return self.w.dtype == torch.bfloat16 and self.in_features % 64 == 0
+
     _wd = None   # transient dequantized weights (prefill side-stream
                  # prefetch; consumed once by the next big-M call)
 
@@ -800,20 +810,21 @@ class RingModel:
             ql = lw.qkv
             wpos = ((kv.pos - self.cp_rank * self.cp_cap).int()
                     if self.cp_size > 1 else None)
-            if (y.is_cuda and ql.is_quant and not ql.mxfp4 and ql.packed
-                    and not c.qk_norm and 2 < B <= 64
-                    and self.cp_size == 1):
+            if (ql.small_m(y) and self.cp_size == 1
+                    and (not c.qk_norm or d <= 128)):
                 # (CP excluded: the wpos-offset variant of the fused
                 # kernel has no single-GPU test path — the unfused
                 # chain is the gloo-verified one)
-                # decode fast path: qkv split-k combine fused into
-                # RoPE+append (bias applied there, k/v go straight to
-                # the cache)
+                # decode fast path: qkv split-k combine and per-head norms
+                # fused into RoPE+append (bias applied there, k/v go
+                # straight to the cache)
                 q = ops.gemv_qkv_rope(
                     y, ql.w, ql.scales, ql.group, ql.bits, ql.bias, nq,
                     nkv, d, kv.k[li], kv.v[li], kv.pos, self.cos, self.sin,
                     kv.kscale[li] if kv.quantized else None,
-                    kv.vscale[li] if kv.quantized else None, wpos)
+                    kv.vscale[li] if kv.quantized else None, wpos,
+                    lw.q_norm if c.qk_norm else None,
+                    lw.k_norm if c.qk_norm else None, c.rms_eps)
             else:
                 qkv = lw.qkv(y)
                 q = qkv[:, :nq * d].view(B, nq, d)
@@ -850,18 +861,7 @@ class RingModel:
                                        window, sinks,
                                        kv.kscale[li] if kv.quantized else None,
                                        kv.vscale[li] if kv.quantized else None)
-            ol = lw.o
-            if (y.is_cuda and ol.is_quant and not ol.mxfp4 and ol.packed
-                    and ol.bias is None and self.tp_size == 1
-                    and 2 < B <= 64):
-                # decode fast path: o split-k combine fused into the
-                # residual RMSNorm
-                y2 = ops.gemv_rmsnorm(attn.view(B, nq * d), ol.w, ol.scales,
-                                      ol.group, ol.bits, h, lw.mlp_norm,
-                                      c.rms_eps)
-            else:
-                o = self._tp_reduce(lw.o(attn.view(B, nq * d)))
-                y2 = ops.rmsnorm(o, h, lw.mlp_norm, c.rms_eps)
+            y2 = self._o_norm(attn.view(B, nq * d), h, lw)
             delta = self._mlp(y2, lw)
             if delta is not ops.DEFERRED:
                 delta = self._tp_reduce(delta)
@@ -898,19 +898,29 @@ class RingModel:
                     (now - last) * 1e3)
         self._obs_t0 = time.perf_counter()
 
+    def _o_norm(self, attn: torch.Tensor, h: torch.Tensor,
+                lw: LayerWeights) -> torch.Tensor:
+        """Output projection of the attention's rows, added to the residual
+        rows ``h``, and the feed-forward's norm of the sum."""
+        c, ol = self.cfg, lw.o
+        if self.tp_size == 1 and ol.small_m(attn):
+            # split-k combine (and bias) fused into the residual RMSNorm
+            return ops.gemv_rmsnorm(attn, ol.w, ol.scales, ol.group, ol.bits,
+                                    h, lw.mlp_norm, c.rms_eps, ol.bias)
+        return ops.rmsnorm(self._tp_reduce(ol(attn)), h, lw.mlp_norm,
+                           c.rms_eps)
+
     def _mlp(self, y: torch.Tensor, lw: LayerWeights) -> torch.Tensor:
         g = lw.gateup
-        if (y.is_cuda and g.is_quant and not g.mxfp4 and g.packed
-                and g.bias is None and 2 < y.shape[0] <= 64):
-            # decode fast path: split-k combine fused into SwiGLU
+        if g.bias is None and g.small_m(y):
+            # decode fast path: split-k combine fused into SwiGLU, or SwiGLU
+            # into the product
             a = ops.gemv_swiglu(y, g.w, g.scales, g.group, g.bits)
         else:
             a = ops.swiglu(g(y))
         dl = lw.down
-        if (getattr(self, "_mlp_defer_ok", False) and a.is_cuda
-                and dl.is_quant and not dl.mxfp4 and dl.packed
-                and dl.bias is None and self.tp_size == 1
-                and 2 < a.shape[0] <= 64
+        if (getattr(self, "_mlp_defer_ok", False) and dl.bias is None
+                and self.tp_size == 1 and dl.small_m(a)
                 and ops.linear_will_defer(a, dl.w, dl.group, dl.bits)):
             # leave the down projection un-combined in the f32 scratch;
             # the decode loop's next RMSNorm (or the final residual add)
@@ -919,11 +929,12 @@ class RingModel:
             return ops.DEFERRED
         return dl(a)
 
-    def _dequant_prefetch(self, layer_ids: Sequence[int], i: int):
+    def _dequant_prefetch(self, layer_ids: Sequence[int], i: int, rows: int):
         """Side-stream dequant of layer i+1's dense weights while layer i
         computes (prefill only; ~65 ms of the 64x128 TTFT was serial
-        dequant). Returns an event the consumer waits on, or None."""
-        if (self.device.type != "cuda" or i + 1 >= len(layer_ids)
+        dequant). Returns an event the consumer waits on, or None: also for
+        few rows, whose products read the quantized weights."""
+        if (rows <= GEMV_MAX_M or self.device.type != "cuda" or i + 1 >= len(layer_ids)
                 or self.weight_provider is not None):  # offload streams
             return None
         nxt = self.layers.get(layer_ids[i + 1])
@@ -954,27 +965,36 @@ class RingModel:
         nq, nkv, d = self.nq_local, self.nkv_local, c.head_dim
         positions = torch.arange(p0, p0 + T, device=h.device)
         layer_ids = list(layer_ids)
-        dq_ev = self._dequant_prefetch(layer_ids, -1)  # prefetch layer 0
+        dq_ev = self._dequant_prefetch(layer_ids, -1, B * T)  # layer 0
         delta = None     # the previous layer's output, not yet in the residual
+        self._mlp_defer_ok = True   # short prompts: as in decode_window
         for i, lid in enumerate(layer_ids):
             lw = self._layer(lid)
             if dq_ev is not None:
                 torch.cuda.current_stream().wait_event(dq_ev)
-            dq_ev = self._dequant_prefetch(layer_ids, i)
+            dq_ev = self._dequant_prefetch(layer_ids, i, B * T)
             flat = h.view(B * T, H)
-            y = ops.rmsnorm(delta if delta is not None else flat,
-                            flat if delta is not None else None,
-                            lw.attn_norm, c.rms_eps)
-            qkv = lw.qkv(y)
+            if delta is ops.DEFERRED:
+                y = ops.rmsnorm_f32_scratch(flat, lw.attn_norm, c.rms_eps)
+            else:
+                y = ops.rmsnorm(delta if delta is not None else flat,
+                                flat if delta is not None else None,
+                                lw.attn_norm, c.rms_eps)
             li = kv.local[lid]
             if (self.cp_size == 1 and not kv.quantized
                     and ops.rope_prefill_supported(d, kv.k[li])):
                 # norms, rotation and append in one pass; attention reads
                 # q and the cache in place
-                q = ops.rope_prefill(
-                    qkv, lw.q_norm if c.qk_norm else None,
-                    lw.k_norm if c.qk_norm else None, self.cos, self.sin,
-                    kv.k[li], kv.v[li], nq, T, p0, c.rms_eps)
+                ql = lw.qkv
+                rest = (lw.q_norm if c.qk_norm else None,
+                        lw.k_norm if c.qk_norm else None, self.cos, self.sin,
+                        kv.k[li], kv.v[li], nq, T, p0, c.rms_eps)
+                if ql.small_m(y) and ops.linear_will_defer(y, ql.w, ql.group,
+                                                           ql.bits):
+                    q = ops.gemv_rope_prefill(y, ql.w, ql.scales, ql.group,
+                                              ql.bits, ql.bias, *rest)
+                else:
+                    q = ops.rope_prefill(ql(y), *rest)
                 window, sinks = self._attn_params(lid, lw)
                 attn = _chunked_causal_attention(
                     q.view(B, T, nq, d).transpose(1, 2),
@@ -982,6 +1002,7 @@ class RingModel:
                     d ** -0.5, p0, window, sinks)
                 delta = self._prefill_rest(attn, flat, lw)
                 continue
+            qkv = lw.qkv(y)
             q = qkv[:, :nq * d].view(B, T, nq, d)
             k = qkv[:, nq * d:(nq + nkv) * d].view(B, T, nkv, d)
             v = qkv[:, (nq + nkv) * d:].view(B, T, nkv, d)
@@ -1041,18 +1062,23 @@ class RingModel:
                     q.transpose(1, 2), kv.k_deq(li)[:, :, :p0 + T],
                     kv.v_deq(li)[:, :, :p0 + T], d ** -0.5, p0, window, sinks)
             delta = self._prefill_rest(attn, flat, lw)
-        flat.add_(delta)
+        self._mlp_defer_ok = False
+        if delta is ops.DEFERRED:
+            ops.resid_add_scratch(flat)
+        else:
+            flat.add_(delta)
         return h
 
     def _prefill_rest(self, attn: torch.Tensor, flat: torch.Tensor,
-                      lw: LayerWeights) -> torch.Tensor:
+                      lw: LayerWeights):
         """Output projection and feed-forward of a prompt: ``attn``
         [B, heads, T, d], the residual rows ``flat`` get the attention's part.
         Returns the feed-forward's, which the next norm adds."""
-        o = self._tp_reduce(
-            lw.o(attn.transpose(1, 2).reshape(flat.shape[0], -1).contiguous()))
-        y2 = ops.rmsnorm(o, flat, lw.mlp_norm, self.cfg.rms_eps)
-        return self._tp_reduce(self._mlp(y2, lw))
+        y2 = self._o_norm(
+            attn.transpose(1, 2).reshape(flat.shape[0], -1).contiguous(),
+            flat, lw)
+        delta = self._mlp(y2, lw)
+        return delta if delta is ops.DEFERRED else self._tp_reduce(delta)
 
     def normalize_project(self, h: torch.Tensor) -> torch.Tensor:
         """Final RMSNorm + lm head -> logits [B, V] (last shard only)."""

@@ -240,17 +240,36 @@ def rope_prefill(qkv: torch.Tensor, q_norm, k_norm, cos, sin, kcache, vcache,
     q [B*T, nq, d]. GPU only, callers gate on rope_prefill_supported."""
     q = torch.empty(qkv.shape[0], nq, kcache.shape[3], dtype=qkv.dtype,
                     device=qkv.device)
-    _native().rope_prefill(qkv, q_norm, k_norm, cos, sin, q, kcache, vcache,
-                           T, p0, eps)
+    _native().rope_prefill(qkv, None, q_norm, k_norm, cos, sin, q, kcache,
+                           vcache, T, p0, eps)
+    return q
+
+
+def gemv_rope_prefill(y: torch.Tensor, w: torch.Tensor, scales, group: int,
+                      bits: int, bias, q_norm, k_norm, cos, sin, kcache,
+                      vcache, nq: int, T: int, p0: int,
+                      eps: float) -> torch.Tensor:
+    """A short prompt's fused projection (up to 64 rows, linear_will_defer)
+    and rope_prefill on its sums in the split-k scratch: the combine kernel
+    disappears from the chain."""
+    gemv_defer(y, w, scales, group, bits)
+    q = torch.empty(y.shape[0], nq, kcache.shape[3], dtype=y.dtype,
+                    device=y.device)
+    _native().rope_prefill(_get_scratch(y.device), bias, q_norm, k_norm, cos,
+                           sin, q, kcache, vcache, T, p0, eps)
     return q
 
 
 def rope_append(q, k, v, kcache, vcache, pos, cos, sin,
-                kscale=None, vscale=None, wpos=None) -> None:
+                kscale=None, vscale=None, wpos=None, q_norm=None, k_norm=None,
+                eps: float = 0.0) -> None:
+    """Rotate q and k in place (after per-head norms, GPU only) and write k, v
+    to the cache."""
     if q.is_cuda:
         _native().rope_append(q, k, v, kcache, vcache, pos, cos, sin,
-                              kscale, vscale, wpos)
+                              kscale, vscale, wpos, q_norm, k_norm, eps)
         return
+    assert q_norm is None and k_norm is None
     ref.rope_append(q, k, v, kcache, vcache, pos, cos, sin, kscale, vscale,
                     wpos)
 
@@ -268,34 +287,39 @@ def _will_defer(M: int, N: int, K: int, group: int, bits: int,
     return v
 
 
-def gemv_qkv_rope(y: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
+def _gemv(x: torch.Tensor, w: torch.Tensor, scales, group: int, bits: int,
+          bias) -> torch.Tensor:
+    if bits == 16:
+        return gemv_bf16(x, w, bias)
+    return (gemv_int8 if bits == 8 else gemv_int4)(x, w, scales, group, bias,
+                                                   True)
+
+
+def gemv_qkv_rope(y: torch.Tensor, w: torch.Tensor, scales,
                   group: int, bits: int, bias, nq: int, nkv: int, d: int,
                   kcache, vcache, pos, cos, sin, kscale=None, vscale=None,
-                  wpos=None):
-    """Fused qkv GEMM + RoPE + KV append for the decode path: when the
+                  wpos=None, q_norm=None, k_norm=None, eps: float = 0.0):
+    """Fused qkv GEMM + per-head norms + RoPE + KV append for the decode path
+    (``bits`` 16: bf16 weights, no scales): when the
     GEMM runs split-k, RoPE reads (and re-zeroes) the f32 scratch
     directly, applies the qkv bias itself, writes the rotated q to a
     dedicated buffer and k/v straight to the cache — the combine kernel
     and the bf16 k/v round trip disappear from the dependency chain.
     Returns the rotated q [B, nq, d]."""
     B = y.shape[0]
-    scratch = _get_scratch(y.device)
-    if _will_defer(B, w.shape[0], y.shape[1], group, bits, scratch.numel()):
-        out = torch.empty(B, w.shape[0], dtype=y.dtype, device=y.device)
-        deferred = _native().gemm_m16(y, w, scales, None, out, scratch,
-                                      group, True, bits, True)
-        assert deferred, "will_defer disagreed with gemm_m16"
+    if linear_will_defer(y, w, group, bits):
+        gemv_defer(y, w, scales, group, bits)
         q = torch.empty(B, nq, d, dtype=y.dtype, device=y.device)
-        _native().rope_append_f32(scratch, bias, q, nkv, kcache, vcache,
-                                  pos, cos, sin, kscale, vscale, wpos)
+        _native().rope_append_f32(_get_scratch(y.device), bias, q, nkv, kcache,
+                                  vcache, pos, cos, sin, kscale, vscale, wpos,
+                                  q_norm, k_norm, eps)
         return q
-    gemv = gemv_int8 if bits == 8 else gemv_int4
-    qkv = gemv(y, w, scales, group, bias, True)
+    qkv = _gemv(y, w, scales, group, bits, bias)
     q = qkv[:, :nq * d].view(B, nq, d)
     k = qkv[:, nq * d:(nq + nkv) * d].view(B, nkv, d)
     v = qkv[:, (nq + nkv) * d:].view(B, nkv, d)
     rope_append(q, k, v, kcache, vcache, pos, cos, sin, kscale, vscale,
-                wpos=wpos)
+                wpos=wpos, q_norm=q_norm, k_norm=k_norm, eps=eps)
     return q
 
 
@@ -307,10 +331,10 @@ class _Deferred:
 DEFERRED = _Deferred()
 
 
-def gemv_defer(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
+def gemv_defer(x: torch.Tensor, w: torch.Tensor, scales,
                group: int, bits: int) -> bool:
     """Launch the GEMM leaving the f32 split-k result in the scratch
-    (caller checked _will_defer). Returns True."""
+    (caller checked linear_will_defer). Returns True."""
     out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
     d = _native().gemm_m16(x, w, scales, None, out, _get_scratch(x.device),
                            group, True, bits, True)
@@ -319,11 +343,12 @@ def gemv_defer(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
 
 
 def rmsnorm_f32_scratch(residual: torch.Tensor, wn: torch.Tensor,
-                        eps: float) -> torch.Tensor:
-    """RMSNorm(+residual) whose x input is the deferred f32 scratch."""
+                        eps: float, bias=None) -> torch.Tensor:
+    """RMSNorm(+residual) whose x input is the deferred f32 scratch (plus the
+    projection's bias)."""
     y = torch.empty_like(residual)
     _native().rmsnorm_f32(_get_scratch(residual.device), residual, wn, y,
-                          eps)
+                          eps, bias)
     return y
 
 
@@ -337,48 +362,38 @@ def linear_will_defer(x: torch.Tensor, w: torch.Tensor, group: int,
                        _get_scratch(x.device).numel())
 
 
-def gemv_rmsnorm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
+def gemv_rmsnorm(x: torch.Tensor, w: torch.Tensor, scales,
                  group: int, bits: int, residual: torch.Tensor,
-                 wn: torch.Tensor, eps: float) -> torch.Tensor:
+                 wn: torch.Tensor, eps: float, bias=None) -> torch.Tensor:
     """Fused projection GEMM + RMSNorm(+residual) for the decode path:
     when the GEMM runs split-k, the norm reads (and re-zeroes) the f32
     scratch directly — the combine kernel disappears from the chain.
     Updates `residual` in place (residual += proj) like ops.rmsnorm."""
-    scratch = _get_scratch(x.device)
-    if _will_defer(x.shape[0], w.shape[0], x.shape[1], group, bits,
-                   scratch.numel()):
-        out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
-                          device=x.device)
-        _native().gemm_m16(x, w, scales, None, out, scratch, group, True,
-                           bits, True)
-        y = torch.empty_like(residual)
-        _native().rmsnorm_f32(scratch, residual, wn, y, eps)
-        return y
-    gemv = gemv_int8 if bits == 8 else gemv_int4
-    o = gemv(x, w, scales, group, None, True)
-    return rmsnorm(o, residual, wn, eps)
+    if linear_will_defer(x, w, group, bits):
+        gemv_defer(x, w, scales, group, bits)
+        return rmsnorm_f32_scratch(residual, wn, eps, bias)
+    return rmsnorm(_gemv(x, w, scales, group, bits, bias), residual, wn, eps)
 
 
-def gemv_swiglu(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
+def gemv_swiglu(x: torch.Tensor, w: torch.Tensor, scales,
                 group: int, bits: int = 8,
                 packed: bool = True) -> torch.Tensor:
     """Fused gate/up GEMM + SwiGLU for the decode path: when the GEMM
     runs split-k, SwiGLU reads (and re-zeroes) the f32 scratch directly
-    instead of going through the f32->bf16 combine kernel — one fewer
-    dependent ~5 us kernel per layer per step."""
-    if not (x.is_cuda and packed and 2 < x.shape[0] <= 64):
+    instead of going through the f32->bf16 combine kernel; when it does not,
+    the activation is part of the product."""
+    if not (x.is_cuda and x.shape[0] <= 64 and (
+            x.shape[1] % 64 == 0 if bits == 16 else
+            packed and 2 < x.shape[0])):
+        if bits == 16:
+            return swiglu(gemv_bf16(x, w))
         gemv = gemv_int8 if bits == 8 else gemv_int4
         return swiglu(gemv(x, w, scales, group, None, packed))
-    M, N = x.shape[0], w.shape[0]
-    out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    y = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
+                    device=x.device)
     scratch = _get_scratch(x.device)
-    deferred = _native().gemm_m16(x, w, scales, None, out, scratch, group,
-                                  True, bits, True)
-    y = torch.empty(M, N // 2, dtype=x.dtype, device=x.device)
-    if deferred:
-        _native().swiglu_f32(scratch, y, N)
-    else:
-        _native().swiglu(out, y)
+    if _native().gemm_swiglu(x, w, scales, y, scratch, group, bits):
+        _native().swiglu_f32(scratch, y, w.shape[0])
     return y
 
 

@@ -4,7 +4,8 @@ namespace py = pybind11;
 
 namespace dnet {
 void rmsnorm_f32(torch::Tensor xf, torch::Tensor residual, torch::Tensor w,
-                 torch::Tensor y, double eps);
+                 torch::Tensor y, double eps,
+                 c10::optional<torch::Tensor> bias);
 void resid_add_f32(torch::Tensor h, torch::Tensor xf);
 void rmsnorm(torch::Tensor x, c10::optional<torch::Tensor> residual,
              torch::Tensor w, torch::Tensor y, double eps);
@@ -31,8 +32,11 @@ void rope_append_f32(torch::Tensor src, c10::optional<torch::Tensor> bias,
                      torch::Tensor cos_table, torch::Tensor sin_table,
                      c10::optional<torch::Tensor> kscale,
                      c10::optional<torch::Tensor> vscale,
-                     c10::optional<torch::Tensor> wpos);
-void rope_prefill(torch::Tensor qkv, c10::optional<torch::Tensor> qw,
+                     c10::optional<torch::Tensor> wpos,
+                 c10::optional<torch::Tensor> q_norm,
+                 c10::optional<torch::Tensor> k_norm, double eps);
+void rope_prefill(torch::Tensor qkv, c10::optional<torch::Tensor> bias,
+                  c10::optional<torch::Tensor> qw,
                   c10::optional<torch::Tensor> kw, torch::Tensor cos,
                   torch::Tensor sin, torch::Tensor qout, torch::Tensor kcache,
                   torch::Tensor vcache, int64_t T, int64_t p0, double eps);
@@ -41,7 +45,9 @@ void rope_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                  torch::Tensor cos_table, torch::Tensor sin_table,
                  c10::optional<torch::Tensor> kscale,
                  c10::optional<torch::Tensor> vscale,
-                 c10::optional<torch::Tensor> wpos);
+                 c10::optional<torch::Tensor> wpos,
+                 c10::optional<torch::Tensor> q_norm,
+                 c10::optional<torch::Tensor> k_norm, double eps);
 void swiglu(torch::Tensor gu, torch::Tensor y);
 void swiglu_f32(torch::Tensor gu_f32, torch::Tensor y, int64_t N);
 void dequant_int8(torch::Tensor w, torch::Tensor scales, torch::Tensor out,
@@ -50,6 +56,9 @@ void dequant_int4(torch::Tensor w, torch::Tensor scales, torch::Tensor out,
                   int64_t group);
 void dequant_mxfp4(torch::Tensor w, torch::Tensor scales, torch::Tensor out);
 void scratch_clean(torch::Tensor scratch);
+bool gemm_swiglu(torch::Tensor x, torch::Tensor w,
+                 c10::optional<torch::Tensor> scales, torch::Tensor out,
+                 torch::Tensor scratch, int64_t group, int64_t bits);
 bool gemm_m16_will_defer(int64_t M, int64_t N, int64_t K, int64_t group,
                          int64_t bits, int64_t scratch_elems);
 bool gemm_m16(torch::Tensor x, torch::Tensor w,
@@ -285,10 +294,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("kcache"),
         py::arg("vcache"), py::arg("pos"), py::arg("cos_table"),
         py::arg("sin_table"), py::arg("kscale"), py::arg("vscale"),
-        py::arg("wpos") = c10::nullopt);
+        py::arg("wpos") = c10::nullopt, py::arg("q_norm") = c10::nullopt,
+        py::arg("k_norm") = c10::nullopt, py::arg("eps") = 0.0);
   m.def("swiglu", &dnet::swiglu, "fused SwiGLU");
   m.def("scratch_clean", &dnet::scratch_clean,
         "zero the split-k scratch region that plain combines left dirty");
+  m.def("gemm_swiglu", &dnet::gemm_swiglu,
+        "gate/up product with SwiGLU, or its sums left in the scratch");
   m.def("gemm_m16_will_defer", &dnet::gemm_m16_will_defer,
         "would gemm_m16(defer_combine=true) defer for this shape");
   m.def("rope_append_f32", &dnet::rope_append_f32,

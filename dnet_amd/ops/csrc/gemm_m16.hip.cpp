@@ -17,8 +17,16 @@ namespace dnet {
 using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
 using f32x4 = __attribute__((ext_vector_type(4))) float;
 
-// bf16 weights. MT: number of stacked 16-row A tiles (M <= 16*MT).
-template <int MT>
+// silu(g) * u
+__device__ __forceinline__ float swiglu_of(const float g, const float u) {
+  return g / (1.f + __expf(-g)) * u;
+}
+
+// bf16 weights. MT: number of stacked 16-row A tiles (M <= 16*MT). GLU: w holds
+// N gate rows and N up rows, a wave computes 16 columns of both and stores
+// silu(gate) * up (no splits): the activation as a kernel of its own, and its
+// launch, are gone.
+template <int MT, bool GLU>
 __global__ void gemm_m16_kernel(const short* __restrict__ x,
                                 const short* __restrict__ w,
                                 const short* __restrict__ bias,
@@ -43,13 +51,18 @@ __global__ void gemm_m16_kernel(const short* __restrict__ x,
   const int p_begin = blockIdx.y * pp;
   const int p_end = (blockIdx.y == splitk - 1) ? pairs : p_begin + pp;
 
-  f32x4 acc[MT][2];
+  constexpr int NW = GLU ? 2 : 1;
+  f32x4 acc[NW][MT][2];
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
+  for (int g = 0; g < NW; ++g)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) acc[t][u] = {0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) acc[g][t][u] = {0.f, 0.f, 0.f, 0.f};
 
-  const short* wrow = w + (int64_t)n_w * K;
+  const short* wrow[NW];
+#pragma unroll
+  for (int g = 0; g < NW; ++g) wrow[g] = w + ((int64_t)g * N + n_w) * K;
 
   for (int k0 = p_begin * 64; k0 < p_end * 64; k0 += XT) {
     const int tk = min(XT, p_end * 64 - k0);
@@ -72,13 +85,17 @@ __global__ void gemm_m16_kernel(const short* __restrict__ x,
     int pl = 0;
     const int pl_end = tk / 64;
     for (; pl + 4 <= pl_end; pl += 4) {  // 4 pairs, all weight loads first
-      bf16x8 wb[4][2];
+      bf16x8 wb[NW][4][2];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int p = (k0 / 64) + pl + u;
-        wb[u][0] = *reinterpret_cast<const bf16x8*>(&wrow[p * 64 + ks]);
-        wb[u][1] = *reinterpret_cast<const bf16x8*>(&wrow[p * 64 + 32 + ks]);
-      }
+      for (int g = 0; g < NW; ++g)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int p = (k0 / 64) + pl + u;
+          wb[g][u][0] =
+              *reinterpret_cast<const bf16x8*>(&wrow[g][p * 64 + ks]);
+          wb[g][u][1] =
+              *reinterpret_cast<const bf16x8*>(&wrow[g][p * 64 + 32 + ks]);
+        }
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -88,30 +105,41 @@ __global__ void gemm_m16_kernel(const short* __restrict__ x,
               *reinterpret_cast<const bf16x8*>(&at[(pl + u) * 64 + ks]);
           const bf16x8 a1 =
               *reinterpret_cast<const bf16x8*>(&at[(pl + u) * 64 + 32 + ks]);
-          acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              a0, wb[u][0], acc[t][0], 0, 0, 0);
-          acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              a1, wb[u][1], acc[t][1], 0, 0, 0);
+#pragma unroll
+          for (int g = 0; g < NW; ++g) {
+            acc[g][t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                a0, wb[g][u][0], acc[g][t][0], 0, 0, 0);
+            acc[g][t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                a1, wb[g][u][1], acc[g][t][1], 0, 0, 0);
+          }
         }
     }
     for (; pl < pl_end; ++pl) {
       const int p = (k0 / 64) + pl;
-      const bf16x8 b0 =
-          *reinterpret_cast<const bf16x8*>(&wrow[p * 64 + ks]);
-      const bf16x8 b1 =
-          *reinterpret_cast<const bf16x8*>(&wrow[p * 64 + 32 + ks]);
+      bf16x8 b0[NW], b1[NW];
+#pragma unroll
+      for (int g = 0; g < NW; ++g) {
+        b0[g] = *reinterpret_cast<const bf16x8*>(&wrow[g][p * 64 + ks]);
+        b1[g] = *reinterpret_cast<const bf16x8*>(&wrow[g][p * 64 + 32 + ks]);
+      }
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
         const short* at = arow + t * 16 * SE;
         const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(&at[pl * 64 + ks]);
         const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(&at[pl * 64 + 32 + ks]);
-        acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[t][0],
-                                                            0, 0, 0);
-        acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[t][1],
-                                                            0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < NW; ++g) {
+          acc[g][t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a0, b0[g], acc[g][t][0], 0, 0, 0);
+          acc[g][t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a1, b1[g], acc[g][t][1], 0, 0, 0);
+        }
       }
     }
   }
+  // the last products' results are read below, behind a branch: past their
+  // latency in any case
+  asm volatile("s_nop 15" ::: "memory");
 
   // C write: lane covers col = n0 + (lane&15), rows (lane>>4)*4 + 0..3 of
   // each stacked tile.
@@ -119,12 +147,16 @@ __global__ void gemm_m16_kernel(const short* __restrict__ x,
   if (n >= N) return;
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    const f32x4 a2 = acc[t][0] + acc[t][1];
+    const f32x4 a2 = acc[0][t][0] + acc[0][t][1];
+    f32x4 up = {0.f, 0.f, 0.f, 0.f};
+    if (GLU) up = acc[NW - 1][t][0] + acc[NW - 1][t][1];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int m = t * 16 + (lane >> 4) * 4 + r;
       if (m >= M) continue;
-      if (splitk > 1) {
+      if (GLU) {
+        out[(int64_t)m * N + n] = f2bits(swiglu_of(a2[r], up[r]));
+      } else if (splitk > 1) {
         atomicAdd(out_f32 + (int64_t)m * N + n, a2[r]);
       } else {
         float v = a2[r];
@@ -133,6 +165,187 @@ __global__ void gemm_m16_kernel(const short* __restrict__ x,
       }
     }
   }
+}
+
+// bf16 weights for few rows or little work: a workgroup owns 16 NC columns and
+// its NW waves divide the inner dimension (the kernel above divides columns and
+// needs atomics to divide the rest). No staging and no barrier before the one
+// fold at the end: weights go from memory to registers, U neighbouring 64 B
+// pieces of each row, x in fragment shape from L2; the next group of pieces is
+// in flight while one is multiplied. Products start from zero and the vector
+// unit adds them up (the matrix core's own running sum rounds less exactly).
+// GLU as above (NF = 2 NC: gate columns, then up columns).
+// Bound by the weight stream, below 10 MB by latency and launch. Measured,
+// MI355X, one row, with the zeroing and combining kernels that the splits
+// needed -> here:
+// 6144 x 4096 15.7 us -> 13.1 (3.8 TB/s), 4096 x 14336 28.6 -> 24.0 (4.9 TB/s),
+// 2 x 14336 x 4096 with swiglu 51.5 -> 42.7 (5.5 TB/s), 768 x 768 5.4 -> 2.7.
+template <int MT, int NF, int NW, int U, bool GLU>
+__global__ __launch_bounds__(NW * 64) void gemm_b16_kernel(
+    const short* __restrict__ x, const short* __restrict__ w,
+    const short* __restrict__ bias, short* __restrict__ out, const int M,
+    const int K, const int N) {
+  constexpr int NC = GLU ? NF / 2 : NF;
+  __shared__ f32x4 part[NW - 1][MT * NF][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int c = lane & 15, hi = lane >> 4;
+  const int n0 = blockIdx.x * (16 * NC);
+  const short* wp[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+    wp[f] = w + ((int64_t)(f / NC) * N + min(n0 + (f % NC) * 16 + c, N - 1)) *
+                    K + hi * 8;
+  const short* xp[MT];      // rows >= M repeat the last one, never stored
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+    xp[m] = x + (int64_t)min(m * 16 + c, M - 1) * K + hi * 8;
+  f32x4 acc[MT][NF];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int f = 0; f < NF; ++f) acc[m][f] = {0.f, 0.f, 0.f, 0.f};
+  struct Batch { bf16x8 w[U][NF], x[U][MT]; };
+  auto load = [&](Batch& q, const int s) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        q.w[u][f] = *reinterpret_cast<const bf16x8*>(wp[f] + (s + u) * 32);
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        q.x[u][m] = *reinterpret_cast<const bf16x8*>(xp[m] + (s + u) * 32);
+  };
+  auto mul = [&](const Batch& q) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        f32x4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q.x[u][m], q.w[u][f], p,
+                                                      0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[m][f][r] += p[r];
+      }
+  };
+  const int total = K / 32;
+  const int groups = total / (NW * U);
+  auto place = [&](int g) { return (g * NW + wave) * U; };
+  if (groups > 0) {
+    Batch q0, q1;
+    load(q0, place(0));
+    int g = 0;
+    for (; g + 2 < groups; g += 2) {
+      load(q1, place(g + 1));
+      __builtin_amdgcn_sched_barrier(0);
+      mul(q0);
+      load(q0, place(g + 2));
+      __builtin_amdgcn_sched_barrier(0);
+      mul(q1);
+    }
+    if (g + 1 < groups) {
+      load(q1, place(g + 1));
+      __builtin_amdgcn_sched_barrier(0);
+      mul(q0);
+      mul(q1);
+    } else {
+      mul(q0);
+    }
+  }
+  for (int s = groups * NW * U + wave; s < total; s += NW) {
+    bf16x8 xv[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+      xv[m] = *reinterpret_cast<const bf16x8*>(xp[m] + s * 32);
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const bf16x8 wv = *reinterpret_cast<const bf16x8*>(wp[f] + s * 32);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        f32x4 p = {0.f, 0.f, 0.f, 0.f};
+        p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv[m], wv, p, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[m][f][r] += p[r];
+      }
+    }
+  }
+  if (wave != 0)
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+        part[wave - 1][m * NF + f][lane] = acc[m][f];
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int v = 0; v < NW - 1; ++v) {
+        const f32x4 p = part[v][m * NF + f][lane];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[m][f][r] += p[r];
+      }
+#pragma unroll
+    for (int f = 0; f < NC; ++f) {
+      const int n = n0 + f * 16 + c;
+      if (n >= N) continue;
+      const float bv = bias != nullptr ? bits2f(bias[n]) : 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = m * 16 + hi * 4 + r;
+        if (row >= M) continue;
+        out[(int64_t)row * N + n] =
+            f2bits(GLU ? swiglu_of(acc[m][f][r], acc[m][NC + f][r])
+                       : acc[m][f][r] + bv);
+      }
+    }
+  }
+}
+
+// Whether gemm_b16_kernel takes the product (`rows` weight rows, 2 N with glu).
+// Its x comes from L2 once per 16 columns, so its line is where x outweighs
+// what it saves (us, the staged kernel with its extra launches -> this one):
+// 1 row 28672 x 4096 with swiglu 51.5 -> 42.7, 6144 x 4096 15.7 -> 13.1,
+// 4096 x 14336 28.6 -> 24.0, 2304 x 768 5.8 -> 3.5; 16 rows 4096 x 4096 14.6 ->
+// 11.5, but 6144 x 4096 17.5 -> 18.3 and 4096 x 14336 30.9 -> 34.7; 32 rows
+// 768 x 3072 12.0 -> 10.3; 64 rows 768 x 768 11.3 -> 5.9, but 768 x 3072 15.5 ->
+// 16.1. Many columns alone fill the chip without splits: 1 row 128256 x 4096
+// 193 -> 199.
+static bool on_b16(int64_t M, int64_t rows, int64_t K, bool glu) {
+  if (rows > 16 * 1024) return glu && M <= 16;
+  if (M <= 8) return true;
+  if (M <= 16) return rows * K <= 20 * 1024 * 1024;
+  return rows * K <= 6 * 1024 * 1024 && K <= (M <= 32 ? 4096 : 2048);
+}
+
+static void launch_b16(const short* x, const short* w, const short* bias,
+                       short* out, int M, int K, int N, bool glu,
+                       hipStream_t st) {
+#define LB(MM, FF, WW, UU, GL)                                              \
+  hipLaunchKernelGGL((gemm_b16_kernel<MM, FF, WW, UU, GL>),                 \
+                     dim3((unsigned)cdiv(N, 16 * (GL ? FF / 2 : FF))),      \
+                     dim3(WW * 64), 0, st, x, w, bias, out, M, K, N)
+  // 8 waves per workgroup where the inner dimension has work for them (from 2
+  // groups of pieces each) and the columns alone leave compute units idle
+  const bool deep = K >= 2048;
+  if (glu) {
+    if (M > 32) LB(4, 2, 4, 2, true);
+    else if (M > 16) LB(2, 2, 4, 2, true);
+    else if (deep) LB(1, 2, 8, 4, true);
+    else LB(1, 2, 4, 4, true);
+  } else {
+    if (M > 32) LB(4, 1, 4, 4, false);
+    else if (M > 16) LB(2, 1, 4, 4, false);
+    else if (deep) LB(1, 1, 8, 4, false);
+    else LB(1, 1, 4, 4, false);
+  }
+#undef LB
 }
 
 // ---------------------------------------------------------------------------
@@ -169,7 +382,9 @@ using i32x4 = __attribute__((ext_vector_type(4))) int;
 
 // NG: scales of a row and chunk, read by one load (groups of KC / NG columns, K
 // a multiple of KC); 0: one scale per 16 B load, any group.
-template <int BITS, int MT, int NF, int KC, int NG>
+// GLU: as in gemm_m16_kernel, the two fragments of a wave are 16 gate columns
+// and the 16 up columns beside them.
+template <int BITS, int MT, int NF, int KC, int NG, bool GLU>
 __global__ __launch_bounds__(256, MT == 4 ? 2 : 3) void gemm_q_kernel(
     const short* __restrict__ x, const void* __restrict__ w,
     const short* __restrict__ scales, const short* __restrict__ bias,
@@ -187,7 +402,8 @@ __global__ __launch_bounds__(256, MT == 4 ? 2 : 3) void gemm_q_kernel(
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
   const int c = lane & 15, hi = lane >> 4;
-  const int n0 = (blockIdx.x * 4 + wave) * (16 * NF);
+  static_assert(!GLU || NF == 2, "gate and up");
+  const int n0 = (blockIdx.x * 4 + wave) * (GLU ? 16 : 16 * NF);
   const int chunks = (K + KC - 1) / KC;
   const int per = (chunks + splitk - 1) / splitk;
   const int c0 = blockIdx.y * per, c1 = min(chunks, c0 + per);
@@ -200,7 +416,8 @@ __global__ __launch_bounds__(256, MT == 4 ? 2 : 3) void gemm_q_kernel(
   const short* sp[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f) {
-    const int64_t row = min(n0 + f * 16 + c, N - 1);
+    const int64_t row = GLU ? (int64_t)f * N + min(n0 + c, N - 1)
+                            : min(n0 + f * 16 + c, N - 1);
     wp[f] = (const char*)w + row * rb + hi * 16;
     sp[f] = scales + row * (K / G);
   }
@@ -357,6 +574,19 @@ __global__ __launch_bounds__(256, MT == 4 ? 2 : 3) void gemm_q_kernel(
     mul(q0, 0);
   }
 
+  if constexpr (GLU) {
+    if (n0 + c >= N) return;
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = m * 16 + hi * 4 + r;
+        if (row < M)
+          out[(int64_t)row * N + n0 + c] =
+              f2bits(swiglu_of(acc[m][0][r], acc[m][1][r]));
+      }
+    return;
+  }
 #pragma unroll
   for (int f = 0; f < NF; ++f) {
     const int n = n0 + f * 16 + c;
@@ -502,19 +732,20 @@ static int pick_splits_q(int64_t N, int64_t K, int64_t M,
 
 static int pick_splits(int64_t N, int64_t K, int64_t M, int64_t scratch_elems,
                        int bits) {
-  return bits < 16 ? pick_splits_q(N, K, M, scratch_elems, bits)
-                   : pick_splitk(N, K, M, scratch_elems);
+  if (bits < 16) return pick_splits_q(N, K, M, scratch_elems, bits);
+  return on_b16(M, N, K, false) ? 1 : pick_splitk(N, K, M, scratch_elems);
 }
 
 static bool launch_m16(torch::Tensor x, torch::Tensor w,
                        c10::optional<torch::Tensor> scales,
                        c10::optional<torch::Tensor> bias, torch::Tensor out,
                        c10::optional<torch::Tensor> scratch, int group,
-                       int64_t m0, int M, int bits, bool defer_combine) {
-  const int64_t K = x.size(1), N = w.size(0);
+                       int64_t m0, int M, int bits, bool defer_combine,
+                       bool glu = false) {
+  const int64_t K = x.size(1), N = glu ? w.size(0) / 2 : w.size(0);
   auto stream = current_stream();
   const int64_t scratch_elems = scratch.has_value() ? scratch->numel() : 0;
-  const int sk = pick_splits(N, K, M, scratch_elems, bits);
+  const int sk = glu ? 1 : pick_splits(N, K, M, scratch_elems, bits);
   const short* bptr = bias.has_value() ? (const short*)bias->data_ptr() : nullptr;
   const dim3 grid((unsigned)((N + 63) / 64), sk);
   const short* xp = (const short*)x.data_ptr() + m0 * K;
@@ -539,37 +770,49 @@ static bool launch_m16(torch::Tensor x, torch::Tensor w,
       g_scratch_dirty_elems = 0;
     }
   }
+  if (bits == 16 && on_b16(M, glu ? 2 * N : N, K, glu)) {
+    launch_b16(xp, (const short*)w.data_ptr(), bptr, op, M, (int)K, (int)N,
+               glu, stream);
+    return false;
+  }
   const short* sp = bits < 16 ? (const short*)scales->data_ptr() : nullptr;
   const short* bp1 = sk > 1 ? nullptr : bptr;
-#define LAUNCH(TT)                                                          \
-  hipLaunchKernelGGL((gemm_m16_kernel<TT>), grid, dim3(256), 0, stream, xp, \
-                     (const short*)w.data_ptr(), bp1, op, fp, M, (int)K,    \
-                     (int)N, sk)
-#define LAUNCH_QN(QQ, TT, FF, KK, GG)                                       \
-  hipLaunchKernelGGL((gemm_q_kernel<QQ, TT, FF, KK, GG>),                   \
-                     dim3((unsigned)cdiv(N, 64 * FF), sk), dim3(256), 0,    \
-                     stream, xp, w.data_ptr(), sp, bp1, op, fp, M, (int)K,  \
-                     (int)N, group, sk)
-#define LAUNCH_Q(QQ, TT, FF, KK)                                            \
+#define LAUNCH(TT, GL)                                                      \
+  hipLaunchKernelGGL((gemm_m16_kernel<TT, GL>), grid, dim3(256), 0, stream, \
+                     xp, (const short*)w.data_ptr(), bp1, op, fp, M,        \
+                     (int)K, (int)N, sk)
+#define LAUNCH_QN(QQ, TT, GG, GL)                                           \
+  hipLaunchKernelGGL((gemm_q_kernel<QQ, TT, 2, kQChunk, GG, GL>),           \
+                     dim3((unsigned)cdiv(N, GL ? 64 : kQCols), sk),         \
+                     dim3(256), 0, stream, xp, w.data_ptr(), sp, bp1, op,   \
+                     fp, M, (int)K, (int)N, group, sk)
+#define LAUNCH_Q(QQ, TT, GL)                                                \
   do {                                                                      \
-    if (K % 256 == 0 && group == 128) LAUNCH_QN(QQ, TT, FF, KK, 2);         \
-    else if (QQ == 8 && K % 256 == 0 && group == 64)                        \
-      LAUNCH_QN(QQ, TT, FF, KK, QQ == 8 ? 4 : 0);                           \
-    else LAUNCH_QN(QQ, TT, FF, KK, 0);                                      \
+    if (K % kQChunk == 0 && group == 128) LAUNCH_QN(QQ, TT, 2, GL);         \
+    else if (QQ == 8 && K % kQChunk == 0 && group == 64)                    \
+      LAUNCH_QN(QQ, TT, QQ == 8 ? 4 : 0, GL);                               \
+    else LAUNCH_QN(QQ, TT, 0, GL);                                          \
   } while (0)
-#define LAUNCH_QB(QQ)                                                       \
+#define LAUNCH_M(GL)                                                        \
   do {                                                                      \
-    if (M > 32) LAUNCH_Q(QQ, 4, 2, 256);                                    \
-    else if (M > 16) LAUNCH_Q(QQ, 2, 2, 256);                               \
-    else LAUNCH_Q(QQ, 1, 2, 256);                                           \
+    if (bits == 8) {                                                        \
+      if (M > 32) LAUNCH_Q(8, 4, GL);                                       \
+      else if (M > 16) LAUNCH_Q(8, 2, GL);                                  \
+      else LAUNCH_Q(8, 1, GL);                                              \
+    } else if (bits == 4) {                                                 \
+      if (M > 32) LAUNCH_Q(4, 4, GL);                                       \
+      else if (M > 16) LAUNCH_Q(4, 2, GL);                                  \
+      else LAUNCH_Q(4, 1, GL);                                              \
+    } else {                                                                \
+      if (M > 32) LAUNCH(4, GL);                                            \
+      else if (M > 16) LAUNCH(2, GL);                                       \
+      else LAUNCH(1, GL);                                                   \
+    }                                                                       \
   } while (0)
-  if (bits == 8) LAUNCH_QB(8);
-  else if (bits == 4) LAUNCH_QB(4);
-  else {
-    if (M > 32) LAUNCH(4);
-    else if (M > 16) LAUNCH(2);
-    else LAUNCH(1);
-  }
+  if (glu) LAUNCH_M(true);
+  else LAUNCH_M(false);
+#undef LAUNCH_M
+#undef LAUNCH_QN
 #undef LAUNCH
 #undef LAUNCH_Q
 #undef LAUNCH_QB
@@ -592,20 +835,17 @@ static bool launch_m16(torch::Tensor x, torch::Tensor w,
 // bias-in-combine paths BEFORE launching.)
 bool gemm_m16_will_defer(int64_t M, int64_t N, int64_t K, int64_t group,
                          int64_t bits, int64_t scratch_elems) {
-  if (M > 64 || M <= 2) return false;
+  if (M > 64 || (bits < 16 && M <= 2)) return false;
   const int sk = pick_splits(N, K, M, scratch_elems, bits);
   return sk > 1;
 }
 
-bool gemm_m16(torch::Tensor x, torch::Tensor w,
-              c10::optional<torch::Tensor> scales,
-              c10::optional<torch::Tensor> bias, torch::Tensor out,
-              c10::optional<torch::Tensor> scratch, int64_t group,
-              bool packed, int64_t bits, bool defer_combine) {
-  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+static void check_m16(const torch::Tensor& x, const torch::Tensor& w,
+                      const c10::optional<torch::Tensor>& scales,
+                      int64_t group, bool packed, int64_t bits) {
+  const int64_t K = x.size(1);
   DNET_CHECK(K % 64 == 0, "K % 64 == 0 required for the MFMA path");
-  DNET_CHECK(out.size(0) == M && out.size(1) == N, "shape");
-  DNET_CHECK(x.is_contiguous() && w.is_contiguous() && out.is_contiguous(), "contig");
+  DNET_CHECK(x.is_contiguous() && w.is_contiguous(), "contig");
   if (bits == 16) {
     DNET_CHECK(w.size(1) == K, "w shape");
   } else {
@@ -618,6 +858,17 @@ bool gemm_m16(torch::Tensor x, torch::Tensor w,
                  "w shape / align (int4)");
     }
   }
+}
+
+bool gemm_m16(torch::Tensor x, torch::Tensor w,
+              c10::optional<torch::Tensor> scales,
+              c10::optional<torch::Tensor> bias, torch::Tensor out,
+              c10::optional<torch::Tensor> scratch, int64_t group,
+              bool packed, int64_t bits, bool defer_combine) {
+  const int64_t M = x.size(0), N = w.size(0);
+  check_m16(x, w, scales, group, packed, bits);
+  DNET_CHECK(out.size(0) == M && out.size(1) == N && out.is_contiguous(),
+             "shape");
   // defer only meaningful for the single-chunk (M <= 64) decode path:
   // multiple chunks could pick different sk and leave a mixed state
   const bool defer = defer_combine && M <= 64 && !bias.has_value();
@@ -630,6 +881,24 @@ bool gemm_m16(torch::Tensor x, torch::Tensor w,
     m0 += mt;
   }
   return deferred;
+}
+
+// out[M, I] = silu(x @ Wg^T) * (x @ Wu^T), w the gate rows and the up rows
+// [2 I, K] without bias, M <= 64. Where the splits of the inner dimension pay
+// (pick_splits), the fp32 sums stay in the scratch (returns true: the caller's
+// swiglu_f32 reads and clears them), else the activation is part of the product.
+bool gemm_swiglu(torch::Tensor x, torch::Tensor w,
+                 c10::optional<torch::Tensor> scales, torch::Tensor out,
+                 torch::Tensor scratch, int64_t group, int64_t bits) {
+  const int64_t M = x.size(0), K = x.size(1), I = out.size(1);
+  check_m16(x, w, scales, group, true, bits);
+  DNET_CHECK(M <= 64 && out.size(0) == M && w.size(0) == 2 * I &&
+                 out.is_contiguous(), "gemm_swiglu shape");
+  const bool split =
+      !(bits == 16 && on_b16(M, 2 * I, K, true)) &&
+      pick_splits(2 * I, K, M, scratch.numel(), (int)bits) > 1;
+  return launch_m16(x, w, scales, c10::nullopt, out, scratch, (int)group, 0,
+                    (int)M, (int)bits, true, !split);
 }
 
 }  // namespace dnet

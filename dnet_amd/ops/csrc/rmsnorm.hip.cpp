@@ -19,7 +19,8 @@ __global__ void rmsnorm_kernel(const short* __restrict__ x,
                                const short* __restrict__ w,
                                short* __restrict__ y,
                                const int H, const float eps, const int T,
-                               float* __restrict__ xf = nullptr) {
+                               float* __restrict__ xf = nullptr,
+                               const short* __restrict__ xb = nullptr) {
   __shared__ float scratch[16];
   const int vecs = H / 8;  // H % 8 == 0 enforced on host
   for (int row = blockIdx.x; row < T; row += gridDim.x) {
@@ -35,7 +36,9 @@ __global__ void rmsnorm_kernel(const short* __restrict__ x,
         xr[1] = make_float4(0.f, 0.f, 0.f, 0.f);
         const float av[8] = {a.x, a.y, a.z, a.w, bq.x, bq.y, bq.z, bq.w};
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v.x[j] = f2bits(av[j]);
+        for (int j = 0; j < 8; ++j)
+          v.x[j] = f2bits(xb != nullptr ? av[j] + bits2f(xb[i * 8 + j])
+                                        : av[j]);
       } else {
         v = xv[i];
       }
@@ -96,12 +99,16 @@ void resid_add_f32(torch::Tensor h, torch::Tensor xf) {
                      (short*)h.data_ptr(), (float*)xf.data_ptr(), total);
 }
 
-// Split-k-fused variant: x read (and re-zeroed) from the f32 scratch.
+// Split-k-fused variant: x read (and re-zeroed) from the f32 scratch, the
+// projection's bias (optional) added.
 void rmsnorm_f32(torch::Tensor xf, torch::Tensor residual, torch::Tensor w,
-                 torch::Tensor y, double eps) {
+                 torch::Tensor y, double eps,
+                 c10::optional<torch::Tensor> bias) {
   const int64_t H = residual.size(-1);
   const int64_t T = residual.numel() / H;
   DNET_CHECK(H % 8 == 0, "H % 8");
+  DNET_CHECK(!bias.has_value() || (bias->is_contiguous() &&
+                                   bias->numel() == H), "bias");
   DNET_CHECK(xf.numel() >= T * H, "scratch too small");
   DNET_CHECK(residual.is_contiguous() && y.is_contiguous() &&
                  w.is_contiguous() && xf.is_contiguous(), "contig");
@@ -110,7 +117,9 @@ void rmsnorm_f32(torch::Tensor xf, torch::Tensor residual, torch::Tensor w,
   hipLaunchKernelGGL((rmsnorm_kernel<true, true>), dim3(grid), dim3(256), 0,
                      stream, nullptr, (short*)residual.data_ptr(),
                      (const short*)w.data_ptr(), (short*)y.data_ptr(),
-                     (int)H, (float)eps, (int)T, (float*)xf.data_ptr());
+                     (int)H, (float)eps, (int)T, (float*)xf.data_ptr(),
+                     bias.has_value() ? (const short*)bias->data_ptr()
+                                      : nullptr);
 }
 
 // y = rmsnorm(x) * w ; if residual is given: residual += x (in place), then

@@ -38,7 +38,10 @@ __global__ void rope_append_kernel(short* __restrict__ q,
                                    const int ldv,
                                    float* __restrict__ src = nullptr,
                                    const short* __restrict__ biasv = nullptr,
-                                   short* __restrict__ qout = nullptr) {
+                                   short* __restrict__ qout = nullptr,
+                                   const short* __restrict__ qn = nullptr,
+                                   const short* __restrict__ kn = nullptr,
+                                   const float eps = 0.f) {
   const int b = blockIdx.x;
   const int h = blockIdx.y;
   const int i = threadIdx.x;  // 0 .. max(D/2,64)-1; lanes >= D/2 idle
@@ -47,24 +50,44 @@ __global__ void rope_append_kernel(short* __restrict__ q,
   const bool act = i < half;
   const float c = act ? cost[(int64_t)p * half + i] : 0.f;
   const float s = act ? sint[(int64_t)p * half + i] : 0.f;
+  // per-head RMS norm of the row (x1, x2 of the block's one wave), optional
+  auto head_norm = [&](const short* w, float& x1, float& x2) {
+    if (w == nullptr) return;
+    float ss = act ? x1 * x1 + x2 * x2 : 0.f;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    const float sc = rsqrtf(ss / (float)D + eps);
+    if (act) {
+      x1 *= sc * bits2f(w[i]);
+      x2 *= sc * bits2f(w[i + half]);
+    }
+  };
   if (h < Hq) {
-    if (!act) return;
     if (F32) {
       float* row = src + (int64_t)b * ldq + h * D;
-      float x1 = row[i], x2 = row[i + half];
-      if (biasv != nullptr) {
-        x1 += bits2f(biasv[h * D + i]);
-        x2 += bits2f(biasv[h * D + i + half]);
+      float x1 = 0.f, x2 = 0.f;
+      if (act) {
+        x1 = row[i];
+        x2 = row[i + half];
+        if (biasv != nullptr) {
+          x1 += bits2f(biasv[h * D + i]);
+          x2 += bits2f(biasv[h * D + i + half]);
+        }
+        row[i] = 0.f;
+        row[i + half] = 0.f;
       }
-      row[i] = 0.f;
-      row[i + half] = 0.f;
+      head_norm(qn, x1, x2);
+      if (!act) return;
       short* qrow = qout + (int64_t)b * Hq * D + h * D;
       qrow[i] = f2bits(x1 * c - x2 * s);
       qrow[i + half] = f2bits(x2 * c + x1 * s);
       return;
     }
     short* row = q + (int64_t)b * ldq + h * D;
-    const float x1 = bits2f(row[i]), x2 = bits2f(row[i + half]);
+    float x1 = act ? bits2f(row[i]) : 0.f;
+    float x2 = act ? bits2f(row[i + half]) : 0.f;
+    head_norm(qn, x1, x2);
+    if (!act) return;
     row[i] = f2bits(x1 * c - x2 * s);
     row[i + half] = f2bits(x2 * c + x1 * s);
     return;
@@ -72,11 +95,13 @@ __global__ void rope_append_kernel(short* __restrict__ q,
   const int hk = h - Hq;
   short* krow = k + (int64_t)b * ldk + hk * D;
   float k1 = 0.f, k2 = 0.f, v1 = 0.f, v2 = 0.f;
+  float x1 = 0.f, x2 = 0.f;
   if (act && F32) {
     const int kcol = (Hq + hk) * D, vcol = (Hq + Hkv + hk) * D;
     float* krowf = src + (int64_t)b * ldq + kcol;
     float* vrowf = src + (int64_t)b * ldq + vcol;
-    float x1 = krowf[i], x2 = krowf[i + half];
+    x1 = krowf[i];
+    x2 = krowf[i + half];
     v1 = vrowf[i];
     v2 = vrowf[i + half];
     if (biasv != nullptr) {
@@ -89,12 +114,14 @@ __global__ void rope_append_kernel(short* __restrict__ q,
     krowf[i + half] = 0.f;
     vrowf[i] = 0.f;
     vrowf[i + half] = 0.f;
-    k1 = x1 * c - x2 * s;
-    k2 = x2 * c + x1 * s;
   } else if (act) {
-    const float x1 = bits2f(krow[i]), x2 = bits2f(krow[i + half]);
-    k1 = x1 * c - x2 * s;
-    k2 = x2 * c + x1 * s;
+    x1 = bits2f(krow[i]);
+    x2 = bits2f(krow[i + half]);
+  }
+  head_norm(kn, x1, x2);
+  k1 = x1 * c - x2 * s;
+  k2 = x2 * c + x1 * s;
+  if (act && !F32) {
     krow[i] = f2bits(k1);
     krow[i + half] = f2bits(k2);
     const short* vrow = v + (int64_t)b * ldv + hk * D;
@@ -159,6 +186,14 @@ __global__ void rope_append_kernel(short* __restrict__ q,
   }
 }
 
+// weights of a per-head norm: the kernel's block is then one wave per head
+static const short* norm_of(const c10::optional<torch::Tensor>& w, int64_t D) {
+  if (!w.has_value()) return nullptr;
+  DNET_CHECK(D <= 128 && w->scalar_type() == torch::kBFloat16 &&
+                 w->is_contiguous() && w->numel() == D, "norm weights");
+  return (const short*)w->data_ptr();
+}
+
 // Fused qkv-split-k-combine + RoPE + append: src = f32 scratch of the
 // qkv GEMM (un-combined), qout receives the rotated+biased q rows.
 void rope_append_f32(torch::Tensor src, c10::optional<torch::Tensor> bias,
@@ -167,8 +202,12 @@ void rope_append_f32(torch::Tensor src, c10::optional<torch::Tensor> bias,
                      torch::Tensor cos_table, torch::Tensor sin_table,
                      c10::optional<torch::Tensor> kscale,
                      c10::optional<torch::Tensor> vscale,
-                     c10::optional<torch::Tensor> wpos) {
+                     c10::optional<torch::Tensor> wpos,
+                     c10::optional<torch::Tensor> q_norm,
+                     c10::optional<torch::Tensor> k_norm, double eps) {
   const int64_t B = qout.size(0), Hq = qout.size(1), D = qout.size(2);
+  const short* qn = norm_of(q_norm, D);
+  const short* kn = norm_of(k_norm, D);
   const int64_t Smax = kcache.size(2);
   const int64_t N = (Hq + 2 * Hkv) * D;
   DNET_CHECK(D % 2 == 0 && D / 2 <= 1024, "head_dim");
@@ -180,7 +219,7 @@ void rope_append_f32(torch::Tensor src, c10::optional<torch::Tensor> bias,
   const int* wpp = wpos.has_value() ? (const int*)wpos->data_ptr() : nullptr;
   const short* bp = bias.has_value() ? (const short*)bias->data_ptr()
                                      : nullptr;
-  const unsigned thr = q8 ? 64u : (unsigned)(D / 2);
+  const unsigned thr = q8 || qn || kn ? 64u : (unsigned)(D / 2);
   if (q8)
     hipLaunchKernelGGL((rope_append_kernel<true, true>),
                        dim3((unsigned)B, (unsigned)(Hq + Hkv)), dim3(thr), 0,
@@ -191,7 +230,8 @@ void rope_append_f32(torch::Tensor src, c10::optional<torch::Tensor> bias,
                        (const float*)cos_table.data_ptr(),
                        (const float*)sin_table.data_ptr(), (int)Hq, (int)Hkv,
                        (int)Smax, (int)D, (int)N, 0, 0,
-                       (float*)src.data_ptr(), bp, (short*)qout.data_ptr());
+                       (float*)src.data_ptr(), bp, (short*)qout.data_ptr(),
+                       qn, kn, (float)eps);
   else
     hipLaunchKernelGGL((rope_append_kernel<false, true>),
                        dim3((unsigned)B, (unsigned)(Hq + Hkv)), dim3(thr), 0,
@@ -201,7 +241,8 @@ void rope_append_f32(torch::Tensor src, c10::optional<torch::Tensor> bias,
                        (const float*)cos_table.data_ptr(),
                        (const float*)sin_table.data_ptr(), (int)Hq, (int)Hkv,
                        (int)Smax, (int)D, (int)N, 0, 0,
-                       (float*)src.data_ptr(), bp, (short*)qout.data_ptr());
+                       (float*)src.data_ptr(), bp, (short*)qout.data_ptr(),
+                       qn, kn, (float)eps);
 }
 
 void rope_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
@@ -209,8 +250,12 @@ void rope_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                  torch::Tensor cos_table, torch::Tensor sin_table,
                  c10::optional<torch::Tensor> kscale,
                  c10::optional<torch::Tensor> vscale,
-                 c10::optional<torch::Tensor> wpos) {
+                 c10::optional<torch::Tensor> wpos,
+                 c10::optional<torch::Tensor> q_norm,
+                 c10::optional<torch::Tensor> k_norm, double eps) {
   const int64_t B = q.size(0), Hq = q.size(1), D = q.size(2);
+  const short* qn = norm_of(q_norm, D);
+  const short* kn = norm_of(k_norm, D);
   const int64_t Hkv = k.size(1), Smax = kcache.size(2);
   DNET_CHECK(D % 2 == 0 && D / 2 <= 1024, "head_dim");
   DNET_CHECK(cos_table.dtype() == torch::kFloat32, "cos table f32");
@@ -234,18 +279,21 @@ void rope_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                        (const float*)cos_table.data_ptr(),
                        (const float*)sin_table.data_ptr(), (int)Hq, (int)Hkv,
                        (int)Smax, (int)D, (int)q.stride(0), (int)k.stride(0),
-                       (int)v.stride(0));
+                       (int)v.stride(0), nullptr, nullptr, nullptr, qn, kn,
+                       (float)eps);
   } else {
     hipLaunchKernelGGL(rope_append_kernel<false>,
                        dim3((unsigned)B, (unsigned)(Hq + Hkv)),
-                       dim3((unsigned)(D / 2)), 0, stream, (short*)q.data_ptr(),
+                       dim3(qn || kn ? 64u : (unsigned)(D / 2)), 0, stream,
+                       (short*)q.data_ptr(),
                        (short*)k.data_ptr(), (const short*)v.data_ptr(),
                        kcache.data_ptr(), vcache.data_ptr(), nullptr, nullptr,
                        (const int*)pos.data_ptr(), wpp,
                        (const float*)cos_table.data_ptr(),
                        (const float*)sin_table.data_ptr(), (int)Hq, (int)Hkv,
                        (int)Smax, (int)D, (int)q.stride(0), (int)k.stride(0),
-                       (int)v.stride(0));
+                       (int)v.stride(0), nullptr, nullptr, nullptr, qn, kn,
+                       (float)eps);
   }
 }
 
@@ -258,9 +306,12 @@ void rope_append(torch::Tensor q, torch::Tensor k, torch::Tensor v,
 // Measured, MI355X: a 37-token prompt through 4 layers of 4096 wide, with the
 // residual sum inside the next norm, 1310 -> 948 us; 64 x 128 tokens through 2
 // layers of 5120 wide 16290 -> 14960 us.
-template <bool NORM>
+// F32: the rows are the un-combined sums of a split product (cleared here for
+// the next one), the projection's bias is added.
+template <bool NORM, bool F32>
 __global__ __launch_bounds__(256) void rope_prefill_kernel(
-    const short* __restrict__ qkv, const short* __restrict__ qw,
+    void* __restrict__ qkv, const short* __restrict__ bias,
+    const short* __restrict__ qw,
     const short* __restrict__ kw, const float* __restrict__ cost,
     const float* __restrict__ sint, short* __restrict__ qout,
     short* __restrict__ kc, short* __restrict__ vc, const int64_t kb,
@@ -277,11 +328,29 @@ __global__ __launch_bounds__(256) void rope_prefill_kernel(
   const bool act = d < half;      // lanes past the half only join the norm
   const int64_t b = row / T;
   const int p = p0 + (int)(row % T);
-  const short* src = qkv + (row * heads + h) * D + d;
+  const int64_t at = (row * heads + h) * D + d;
   short8 x1 = {}, x2 = {};
   if (act) {
-    x1 = *reinterpret_cast<const short8*>(src);
-    x2 = *reinterpret_cast<const short8*>(src + half);
+    if (F32) {
+      const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        float4* fp = reinterpret_cast<float4*>((float*)qkv + at + s * half);
+        const float4 a = fp[0], c = fp[1];
+        fp[0] = z;
+        fp[1] = z;
+        const float f[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+        short8& x = s ? x2 : x1;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          x.x[j] = f2bits(bias != nullptr
+                              ? f[j] + bits2f(bias[h * D + s * half + d + j])
+                              : f[j]);
+      }
+    } else {
+      x1 = *reinterpret_cast<const short8*>((const short*)qkv + at);
+      x2 = *reinterpret_cast<const short8*>((const short*)qkv + at + half);
+    }
   }
   short* dst;
   if (h < nq) dst = qout + (row * nq + h) * D;
@@ -333,18 +402,27 @@ __global__ __launch_bounds__(256) void rope_prefill_kernel(
   }
 }
 
-void rope_prefill(torch::Tensor qkv, c10::optional<torch::Tensor> qw,
+// qkv: bf16 rows, or the fp32 scratch of the split product (its leading values)
+void rope_prefill(torch::Tensor qkv, c10::optional<torch::Tensor> bias,
+                  c10::optional<torch::Tensor> qw,
                   c10::optional<torch::Tensor> kw, torch::Tensor cos,
                   torch::Tensor sin, torch::Tensor qout, torch::Tensor kcache,
                   torch::Tensor vcache, int64_t T, int64_t p0, double eps) {
   const int64_t R = qout.size(0), nq = qout.size(1), D = qout.size(2);
   const int64_t nkv = kcache.size(1), Smax = kcache.size(2);
-  for (const auto& t : {qkv, qout, kcache, vcache})
+  const bool f32 = qkv.scalar_type() == torch::kFloat;
+  for (const auto& t : {qout, kcache, vcache})
     DNET_CHECK(t.scalar_type() == torch::kBFloat16 &&
                    (uintptr_t)t.data_ptr() % 16 == 0, "bf16, 16 B");
   DNET_CHECK(D % 16 == 0 && D <= 128, "head size");
-  DNET_CHECK(qkv.is_contiguous() && qkv.numel() == R * (nq + 2 * nkv) * D &&
+  DNET_CHECK((f32 || qkv.scalar_type() == torch::kBFloat16) &&
+                 qkv.is_contiguous() && (uintptr_t)qkv.data_ptr() % 16 == 0 &&
+                 (f32 ? qkv.numel() >= R * (nq + 2 * nkv) * D
+                      : qkv.numel() == R * (nq + 2 * nkv) * D) &&
                  qout.is_contiguous(), "qkv rows");
+  DNET_CHECK(!bias.has_value() || (f32 && bias->is_contiguous() &&
+                                   bias->numel() == (nq + 2 * nkv) * D),
+             "bias");
   DNET_CHECK(T > 0 && R % T == 0 && kcache.size(0) == R / T && p0 >= 0 &&
                  p0 + T <= Smax, "rows and positions");
   DNET_CHECK(kcache.size(3) == D && vcache.sizes() == kcache.sizes() &&
@@ -365,19 +443,22 @@ void rope_prefill(torch::Tensor qkv, c10::optional<torch::Tensor> qw,
   if (R == 0) return;
   const int64_t items = R * (nq + 2 * nkv);
   const dim3 grid((unsigned)cdiv(items, 32));
-#define LAUNCH_RP(NN, QW, KW)                                                 \
-  hipLaunchKernelGGL((rope_prefill_kernel<NN>), grid, dim3(256), 0,           \
-                     current_stream(), (const short*)qkv.data_ptr(), QW, KW,  \
-                     cos.data_ptr<float>(), sin.data_ptr<float>(),            \
-                     (short*)qout.data_ptr(), (short*)kcache.data_ptr(),      \
-                     (short*)vcache.data_ptr(), kcache.stride(0),             \
-                     kcache.stride(1), vcache.stride(0), vcache.stride(1),    \
-                     (int)T, (int)nq, (int)nkv, (int)D, (int)p0, (float)eps,  \
-                     items)
-  if (qw.has_value())
-    LAUNCH_RP(true, (const short*)qw->data_ptr(), (const short*)kw->data_ptr());
-  else
-    LAUNCH_RP(false, nullptr, nullptr);
+#define LAUNCH_RP(NN, FF)                                                     \
+  hipLaunchKernelGGL(                                                         \
+      (rope_prefill_kernel<NN, FF>), grid, dim3(256), 0, current_stream(),    \
+      qkv.data_ptr(),                                                         \
+      bias.has_value() ? (const short*)bias->data_ptr() : nullptr,            \
+      NN ? (const short*)qw->data_ptr() : nullptr,                            \
+      NN ? (const short*)kw->data_ptr() : nullptr, cos.data_ptr<float>(),     \
+      sin.data_ptr<float>(), (short*)qout.data_ptr(),                         \
+      (short*)kcache.data_ptr(), (short*)vcache.data_ptr(),                   \
+      kcache.stride(0), kcache.stride(1), vcache.stride(0),                   \
+      vcache.stride(1), (int)T, (int)nq, (int)nkv, (int)D, (int)p0,           \
+      (float)eps, items)
+  if (qw.has_value() && f32) LAUNCH_RP(true, true);
+  else if (qw.has_value()) LAUNCH_RP(true, false);
+  else if (f32) LAUNCH_RP(false, true);
+  else LAUNCH_RP(false, false);
 #undef LAUNCH_RP
 }
 

@@ -1091,3 +1091,129 @@ def test_gemm_quant_chunk_edges(bits, N, K, G, M):
         bound = mass * (K + 8) * 2 ** -24 + ref64.abs() * 2 ** -8 \
             + (0 if b is None else b.double().abs() * 2 ** -22)
         assert ((got - ref64).abs() <= bound).all()
+
+
+def _small_weights(bits, N, K, G):
+    """(weights on the device, scales or None, the same in fp64)"""
+    w = (torch.randn(N, K) / K ** 0.5).to(torch.bfloat16)
+    if bits == 16:
+        return w.to(_dev()), None, w.double()
+    if bits == 8:
+        q, s = ops.quantize_int8(w, G)
+        codes, packed = q, ops.pack_int8_mfma(q)
+    else:
+        q, s = ops.quantize_int4(w, G)
+        codes, packed = ref.unpack_int4(q), ops.pack_int4_mfma(q)
+    w64 = (codes.double().view(N, K // G, G)
+           * s.double().unsqueeze(-1)).view(N, K)
+    return packed.to(_dev()), s.to(_dev()), w64
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 17, 33, 64])
+@pytest.mark.parametrize("N,K", [(72, 64), (200, 320), (24, 2112),
+                                 (768, 1024), (4096, 4160), (16400, 128)])
+def test_gemm_bf16_small_edges(M, N, K):
+    """bf16 weights on both sides of the rule that divides K between waves:
+    columns that end inside a tile, pieces that no group of waves divides
+    into, with and without bias. fp32 sums within (K + 8) 2^-24 of sum |x w|,
+    then bf16 (2^-8)."""
+    torch.manual_seed(N + M)
+    x = torch.randn(M, K, dtype=torch.bfloat16)
+    w, _, w64 = _small_weights(16, N, K, 0)
+    want, mass = x.double() @ w64.t(), x.double().abs() @ w64.abs().t()
+    bias = torch.randn(N, dtype=torch.bfloat16)
+    for b in (None, bias):
+        ref64 = want if b is None else want + b.double()
+        got = ops.gemv_bf16(x.to(_dev()), w,
+                            None if b is None else b.to(_dev()))
+        bound = mass * (K + 8) * 2 ** -24 + ref64.abs() * 2 ** -8 \
+            + (0 if b is None else b.double().abs() * 2 ** -22)
+        assert ((got.double().cpu() - ref64).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M", [3, 16, 20, 64])
+@pytest.mark.parametrize("bits,I,K,G", [
+    (16, 40, 64, 0), (16, 1536, 2112, 0), (16, 8256, 192, 0),
+    (8, 40, 64, 64), (8, 264, 1024, 128), (8, 8200, 128, 64),
+    (4, 40, 128, 128), (4, 264, 1024, 128), (4, 8200, 256, 256),
+])
+def test_gemv_swiglu_edges(bits, I, K, G, M):
+    """The activation as part of the product and on split sums. With an error
+    e_g, e_u of the sums (as above) |silu'| < 1.1 and |silu(g)| <= |g| bound
+    the product's; bf16 sums are allowed twice 2^-8 of themselves, since the
+    gate and up values may be rounded between the two steps."""
+    torch.manual_seed(I + M)
+    x = torch.randn(M, K, dtype=torch.bfloat16)
+    w, s, w64 = _small_weights(bits, 2 * I, K, G)
+    got = ops.gemv_swiglu(x.to(_dev()), w, s, G, bits).double().cpu()
+    z, mass = x.double() @ w64.t(), x.double().abs() @ w64.abs().t()
+    err = mass * (K + 8) * 2 ** -24 + z.abs() * 2 ** -8
+    (g, u), (eg, eu) = z.split(I, 1), err.split(I, 1)
+    want = torch.nn.functional.silu(g) * u
+    bound = 1.1 * eg * (u.abs() + eu) + (g.abs() + eg) * eu \
+        + want.abs() * 2 ** -8 + 1e-30
+    assert ((got - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M,bits,K,G", [(1, 16, 512, 0), (20, 16, 4096, 0),
+                                        (64, 16, 4096, 0), (5, 8, 4096, 128),
+                                        (33, 4, 4096, 128)])
+def test_gemv_fused_consumers(M, bits, K, G):
+    """Projection + norm, and projection + per-head norms + rotation + append
+    (a decode step's and a prompt's), against the same consumers on the
+    projection's own bf16 output: sums left in the scratch skip that rounding
+    (2^-8 of a value, carried through norm and rotation: 2^-6 of the row's
+    largest). Twice, for the scratch must be left clean."""
+    torch.manual_seed(K + M)
+    dev, d, nq, nkv, smax, eps = _dev(), 128, 8, 2, 96, 1e-6
+    x = torch.randn(M, K, dtype=torch.bfloat16, device=dev)
+    bf = lambda *n: torch.randn(*n, dtype=torch.bfloat16, device=dev)
+    N = (nq + 2 * nkv) * d
+    w, s, w64 = _small_weights(bits, N, K, G)
+    bias, wn = 0.1 * bf(N), 1 + 0.1 * bf(N)
+    qw, kw = 1 + 0.1 * bf(d), 1 + 0.1 * bf(d)
+    cos, sin = (t.to(dev) for t in ops.rope_tables(smax, d, 10000.0))
+    proj = (x.double() @ w64.to(dev).t().contiguous() + bias.double()
+            ).to(torch.bfloat16)
+
+    def close(a, b):
+        a, b = a.float().reshape(M, -1, d), b.float().reshape(M, -1, d)
+        return ((a - b).abs() <= b.abs().amax(-1, keepdim=True)
+                * 2 ** -6).all()
+    for _ in range(2):
+        r0 = bf(M, N)
+        r1 = r0.clone()
+        got = ops.gemv_rmsnorm(x, w, s, G, bits, r0, wn, eps, bias)
+        want = ops.rmsnorm(proj, r1, wn, eps)
+        assert close(got, want) and close(r0, r1)
+        # a decode step
+        kv = [bf(M, nkv, smax, d) for _ in range(2)]
+        kv2 = [t.clone() for t in kv]
+        pos = torch.randint(0, smax, (M,), dtype=torch.int32, device=dev)
+        q = ops.gemv_qkv_rope(x, w, s, G, bits, bias, nq, nkv, d, *kv, pos,
+                              cos, sin, q_norm=qw, k_norm=kw, eps=eps)
+        at = torch.arange(M, device=dev)
+        px = proj.view(M, nq + 2 * nkv, d)
+        norm = lambda t, g: ops.rmsnorm(t.reshape(-1, d), None, g,
+                                        eps).view(t.shape)
+        q2, k2 = norm(px[:, :nq], qw), norm(px[:, nq:nq + nkv], kw)
+        ops.rope_append(q2, k2, px[:, nq + nkv:].contiguous(), *kv2, pos, cos,
+                        sin)
+        assert close(q, q2)
+        for a, b in zip(kv, kv2):
+            assert close(a[at, :, pos.long()], b[at, :, pos.long()])
+            a[at, :, pos.long()] = b[at, :, pos.long()]
+            assert torch.equal(a, b)
+        # a prompt of M tokens
+        if ops.linear_will_defer(x, w, G, bits):
+            kv = [bf(1, nkv, smax, d) for _ in range(2)]
+            kv2 = [t.clone() for t in kv]
+            q = ops.gemv_rope_prefill(x, w, s, G, bits, bias, qw, kw, cos, sin,
+                                      *kv, nq, M, 3, eps)
+            q2 = ops.rope_prefill(proj, qw, kw, cos, sin, *kv2, nq, M, 3, eps)
+            assert close(q, q2)
+            for a, b in zip(kv, kv2):
+                assert close(a[0, :, 3:3 + M].transpose(0, 1).contiguous(),
+                             b[0, :, 3:3 + M].transpose(0, 1).contiguous())
+                a[:, :, 3:3 + M] = b[:, :, 3:3 + M]
+                assert torch.equal(a, b)
