@@ -1,9 +1,8 @@
 """Mixtral-style MoE ring model (top-k routed experts, SwiGLU experts).
 
 Reference counterpart: src/dnet/core/models/gpt_oss.py (MoE layer pattern);
-this is the dense-correct implementation — per-expert token gather + the
-same fused SwiGLU/GEMV kernels. Expert-parallel execution across ranks is a
-later milestone.
+decode batches and prompts run all experts in two launches, what those do not
+hold runs one expert after the other. Experts are divided over TP ranks.
 """
 from __future__ import annotations
 
@@ -268,6 +267,20 @@ class MoERingModel(RingModel):
             if getattr(lw, "shared_gateup", None) is not None:
                 out = out + self._shared_expert(y, lw)
             return out.to(y.dtype)
+        own = [e for e in range(c.num_experts)
+               if self.tp_size <= 1 or e % self.tp_size == self.tp_rank]
+        gus, dns = ([bank[e] for e in own]
+                    for bank in (lw.experts_gateup, lw.experts_down))
+        if own and ops.moe_prompt_supported(y, idx.numel(), gus, dns):
+            if self.tp_size > 1:      # places in `own`, -1 elsewhere
+                idx = torch.where(idx % self.tp_size == self.tp_rank,
+                                  idx // self.tp_size, -1)
+            shared = gate = None
+            if getattr(lw, "shared_gateup", None) is not None:
+                shared = lw.shared_down(ops.swiglu(lw.shared_gateup(y)))
+                gate = torch.sigmoid(lw.shared_gate(y).float()).view(-1)
+            return ops.moe_prompt(y, idx, weights, gus, dns, self.GLU,
+                                  self.GLU_ALPHA, self.GLU_LIMIT, shared, gate)
         out = torch.zeros_like(y, dtype=torch.float32)
         for e in range(c.num_experts):
             if self.tp_size > 1 and e % self.tp_size != self.tp_rank:

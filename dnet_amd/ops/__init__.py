@@ -1055,6 +1055,81 @@ def moe_plan(idx, E: int):
     return ref.moe_plan(idx, E)
 
 
+def moe_prompt_supported(x, entries: int, gateup: list, down: list) -> bool:
+    """Whether ``moe_prompt`` takes this many (row, choice) entries through
+    these experts: bf16 x on the GPU, up to 128 experts, all bf16 or all packed
+    int8, inner widths in whole steps.
+
+    Up to 5e11 operations per expert: beyond, a library product per expert
+    makes up for its dequantized weights and its waits for the host. us, one
+    expert after the other -> here: 8 int8 experts of 4096 x 14336, 700 rows
+    (2 choices each) 2916 -> 896, 6000 rows (5.3e11 per expert) 6194 -> 5574,
+    8000 rows 6984 -> 7248; bf16 4000 rows (3.5e11) 3945 -> 3655, 8000 rows 6152
+    -> 6772; 32 bf16 experts of 2880 x 2880, 100 rows (4 choices) 5804 -> 356,
+    24000 rows (1.5e11) 16403 -> 8389. Up to 4 GiB of activations and results,
+    which the loop holds for one expert at a time."""
+    if not (x.is_cuda and x.dtype == torch.bfloat16
+            and 1 <= len(gateup) <= 128):
+        return False
+    h, inter = x.shape[1], gateup[0].w.shape[0] // 2
+    if (6.0 * entries * h * inter > 5e11 * len(gateup)
+            or 2 * entries * (h + inter) > 1 << 32):
+        return False
+    for bank in (gateup, down):
+        l0 = bank[0]
+        if l0.mxfp4 or l0.bits not in (8, 16):
+            return False
+        k = l0.w.shape[1]
+        if l0.bits == 16:
+            if k % 64:
+                return False
+        elif not (l0.packed and k % 128 == 0
+                  and (l0.group == 64 or l0.group % 128 == 0)):
+            return False
+        if l0.w.numel() * l0.w.element_size() >= 1 << 32:
+            return False
+        if any(l.bits != l0.bits or l.group != l0.group
+               or l.packed != l0.packed or l.w.shape != l0.w.shape
+               or (l.bias is None) != (l0.bias is None)
+               or not l.w.is_contiguous() for l in bank):
+            return False
+    return True
+
+
+def moe_prompt(x: torch.Tensor, idx: torch.Tensor, val: torch.Tensor,
+               gateup: list, down: list, glu: int, alpha: float, limit: float,
+               shared=None, gate=None) -> torch.Tensor:
+    """out[t] = sum_k val[t, k] * down_e(act(gateup_e(x[t]))) with e = idx[t,
+    k] the place in the banks or -1 (not in them), plus gate * shared. All
+    experts in two products, no host sync (moe_prompt_supported)."""
+    T, top = idx.shape
+    E, n = len(gateup), T * top
+    idx = idx.to(torch.int32).contiguous()
+    val = val.float().contiguous()
+    order = torch.empty(n, dtype=torch.int32, device=x.device)
+    at = torch.full_like(idx, -1)
+    counts = torch.empty(E, dtype=torch.int32, device=x.device)
+    # rows of a tile: what the narrower of the two products takes
+    tile = 96 if 8 in (gateup[0].bits, down[0].bits) else 128
+    tab = torch.empty(8 * (1 + n // tile + E), dtype=torch.int32,
+                      device=x.device)
+    lib = _native()
+    lib.moe_plan(idx, order, at, counts)
+    lib.moe_tiles(counts, tab, n, tile)
+
+    def product(a, bank, width, kind):
+        out = torch.empty(n, width, dtype=x.dtype, device=x.device)
+        l0 = bank[0]
+        lib.moe_prompt(a, order, val, tab, [l.w for l in bank],
+                       [l.scales for l in bank] if l0.bits == 8 else [],
+                       [l.bias for l in bank] if l0.bias is not None else [],
+                       out, l0.group, tile, kind, alpha, limit)
+        return out
+    act = product(x.contiguous(), gateup, gateup[0].w.shape[0] // 2, glu)
+    y = product(act, down, down[0].w.shape[0], 2)
+    return moe_merge(y, at, shared, gate, x.dtype)
+
+
 def moe_gather(x, order, val):
     """Rows of x [T, W] and scales val [T, top] of the sorted entries
     ``order``: (xs [T*top, W], scale fp32 [T*top])."""

@@ -256,6 +256,14 @@ void moe_clamped_rows(torch::Tensor x, torch::Tensor w, torch::Tensor we,
                       torch::Tensor act, double alpha, double limit);
 void moe_plan(torch::Tensor idx, torch::Tensor order, torch::Tensor at,
               torch::Tensor counts);
+void moe_tiles(torch::Tensor counts, torch::Tensor tab, int64_t n,
+               int64_t tile);
+void moe_prompt(torch::Tensor x, torch::Tensor order, torch::Tensor val,
+                torch::Tensor tab, std::vector<torch::Tensor> w,
+                std::vector<torch::Tensor> scales,
+                std::vector<torch::Tensor> bias, torch::Tensor out,
+                int64_t group, int64_t tile, int64_t kind, double alpha,
+                double limit);
 void moe_gather(torch::Tensor x, torch::Tensor order, torch::Tensor val,
                 torch::Tensor xs, torch::Tensor scale);
 void moe_gateup_rows(torch::Tensor x, torch::Tensor w, torch::Tensor we,
@@ -404,6 +412,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "sigmoid router: top-k scores times a constant, optional correction, "
         "expert groups and shared-expert gate");
   m.def("moe_plan", &dnet::moe_plan, "routed entries sorted by expert");
+  m.def("moe_tiles", &dnet::moe_tiles, "row tiles of sorted entries");
+  m.def("moe_prompt", &dnet::moe_prompt,
+        "one product of all experts on a prompt's sorted entries");
   m.def("moe_gather", &dnet::moe_gather, "rows and scales of sorted entries");
   m.def("moe_gateup_rows", &dnet::moe_gateup_rows,
         "gated experts on a decode batch, inputs scaled (matrix cores)");

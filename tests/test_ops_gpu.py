@@ -1217,3 +1217,94 @@ def test_gemv_fused_consumers(M, bits, K, G):
                              b[0, :, 3:3 + M].transpose(0, 1).contiguous())
                 a[:, :, 3:3 + M] = b[:, :, 3:3 + M]
                 assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,H,I,E,top,bits,G,glu,bias", [
+    (65, 320, 192, 4, 2, 16, 0, 0, False),      # columns end inside a tile
+    (300, 192, 448, 3, 1, 16, 0, 1, True),      # one expert fills two tiles
+    (100, 2880, 320, 32, 4, 16, 0, 1, True),    # tiles of a few rows
+    (97, 256, 384, 2, 2, 8, 64, 0, False),      # 97 rows: one over a tile
+    (200, 640, 128, 8, 2, 8, 128, 0, False),    # an odd number of steps
+    (1000, 128, 1152, 5, 3, 8, 64, 1, True),
+    (70, 128, 128, 128, 8, 8, 128, 0, False),   # the most experts
+])
+def test_moe_prompt_edges(T, H, I, E, top, bits, G, glu, bias):
+    """A prompt through routed experts in two products, against fp64. Entries
+    out of the bank (-1) count nothing; one expert stays without rows. Sums in
+    fp32; weights of int8 experts, act and each entry's result are rounded to
+    bf16 (2^-8 of the sums of magnitudes at most)."""
+    from dnet_amd.models.base import Linear
+    from dnet_amd.models.config import QuantConfig
+    torch.manual_seed(T + I)
+    dev = _dev()
+    quant = QuantConfig(8, G) if bits == 8 else None
+
+    def bank(n, k):
+        return [Linear.make(
+            (torch.randn(n, k, device=dev) / k ** 0.5).to(torch.bfloat16),
+            torch.randn(n, device=dev).to(torch.bfloat16) if bias else None,
+            quant) for _ in range(E)]
+    gu, dn = bank(2 * I, H), bank(H, I)
+    x = torch.randn(T, H, device=dev).to(torch.bfloat16)
+    score = torch.randn(T, E, device=dev)
+    if E > top:
+        score[:, E // 2] = -100.0
+    val, idx = torch.topk(score, top, -1)
+    val = torch.softmax(val, -1)
+    idx = torch.where(torch.rand(T, top, device=dev) < 0.1, -1, idx)
+    shared = torch.randn(T, H, device=dev).to(torch.bfloat16)
+    gate = torch.rand(T, device=dev)
+    assert ops.moe_prompt_supported(x, T * top, gu, dn)
+    got = ops.moe_prompt(x, idx, val, gu, dn, glu, 1.702, 7.0, shared, gate)
+
+    def prod(a, lin):          # value and sum of magnitudes, on the CPU
+        w = lin.dequant().double().cpu()
+        b = lin.bias.double().cpu() if bias else torch.zeros(len(w))
+        return a @ w.t() + b, a.abs() @ w.t().abs() + b.abs()
+    x64, idx, val = x.double().cpu(), idx.cpu(), val.double().cpu()
+    want = (gate.double().view(-1, 1) * shared.double()).cpu()
+    bound = want.abs() * 2 ** -22
+    for e in range(E):
+        r, k = (idx == e).nonzero(as_tuple=True)
+        if len(r) == 0:
+            continue
+        (g, u), mass = prod(x64[r], gu[e])[0].split(I, 1), \
+            prod(x64[r], gu[e])[1]
+        eg, eu = (mass * (H + 8) * 2 ** -23).split(I, 1)
+        if glu:
+            g, u = g.clamp(max=7.0), u.clamp(-7.0, 7.0)
+            act, f = (u + 1) * g * torch.sigmoid(1.702 * g), u.abs() + 1
+        else:
+            act, f = torch.nn.functional.silu(g) * u, u.abs()
+        err = act.abs() * 2 ** -8 + 1.2 * eg * (f + eu) + (g.abs() + eg) * eu
+        d, m = prod(act, dn[e])
+        w = dn[e].dequant().double().cpu().abs()
+        v = val[r, k].unsqueeze(1)
+        want[r] += v * d
+        bound[r] += v * (err @ w.t() + m * (I + 8) * 2 ** -23
+                         + d.abs() * 2 ** -8)
+    bound += (want.abs() + bound) * 2 ** -8
+    assert ((got.double().cpu() - want).abs() <= bound).all()
+
+
+def test_moe_prompt_takes_only_what_it_holds():
+    """Forms that the two products do not hold go one expert after the
+    other."""
+    from dnet_amd.models.base import Linear
+    from dnet_amd.models.config import QuantConfig
+    dev = _dev()
+
+    def takes(h=256, i=256, e=2, entries=200, quant=None, dtype=torch.bfloat16):
+        mk = lambda n, k: [Linear.make(torch.zeros(
+            n, k, dtype=torch.bfloat16, device=dev), None, quant)] * e
+        return ops.moe_prompt_supported(torch.zeros(2, h, dtype=dtype,
+                                                    device=dev),
+                                        entries, mk(2 * i, h), mk(h, i))
+    assert takes() and takes(quant=QuantConfig(8, 64))
+    assert not takes(dtype=torch.float32)
+    assert not takes(h=96)
+    assert not takes(h=192, quant=QuantConfig(8, 64))
+    assert not takes(h=384, i=384, quant=QuantConfig(8, 192))
+    assert not takes(e=129)
+    assert not takes(quant=QuantConfig(4, 128))
+    assert not takes(entries=10 ** 7)
