@@ -43,7 +43,9 @@
 //    one key per lane, accumulate phase = output dims across lanes with the
 //    weight broadcast from a per-wave LDS slab. Used for decode, for fp32,
 //    and for head sizes the MFMA kernel does not cover.
-//  * attn_mod_mfma<DC,NV>: bf16 prefill on v_mfma_f32_16x16x32_bf16 — QK^T
+//  * attn_mod_mfma<DC,NV>: bf16 prefill of what the prompt kernel of
+//    attn_prefill does not take (other head sizes, shared values, pooled
+//    entries, chunks, gates ...) on v_mfma_f32_16x16x32_bf16 — QK^T
 //    and PV on the matrix cores, modifiers + online softmax in the fp32 C
 //    fragments. Head sizes are zero-padded in LDS to DC*32 / NV*16.
 //  * attn_mod_mfma_heads<DC,NV>: bf16 decode with >= 16 query heads per kv
@@ -52,6 +54,14 @@
 #include "common.h"
 
 namespace dnet {
+
+// attn_prefill.hip.cpp
+bool attn_prompt_mod(const short* q, const short* k, const short* v, short* out,
+                     const int* pos, const int* lens, const int* slots,
+                     const float* temp, const float* r1, const float* r2,
+                     const float* sinks, float scale, float softcap, int B,
+                     int T, int Bc, int Hq, int Hkv, int Smax, int D, int DV,
+                     int window, int64_t out_ld);
 
 using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
 using bf16x2 = __attribute__((ext_vector_type(2))) __bf16;
@@ -1095,7 +1105,21 @@ void attn_mod(torch::Tensor q, torch::Tensor kcache,
                        0, P);
     return;
   }
-  // bf16 prompts: matrix-core kernel (head sizes padded to its tile classes)
+  // bf16 prompts with their own values, a softmax and at most a window: the
+  // prompt kernel of attn_prefill, faster at every size (cap, penalty and sinks,
+  // us, attn_mod_mfma -> there: 5 prompts of 1023 tokens, 32 heads of 128, 773
+  // -> 129, one of 16 tokens 10.3 -> 8.0, 64 tokens behind 1000 160 -> 50; 4 of
+  // 500, 16 heads of 64, 79 -> 24; 2000 with a window of 256 133 -> 33)
+  if (!f32 && T >= 16 && !vshare && pool == 0 && !sig && P.chunk == 0 &&
+      P.keep == 0 && P.gate == nullptr && !wide && T <= INT_MAX / G &&
+      attn_prompt_mod((const short*)q.data_ptr(),
+                      (const short*)kcache.data_ptr(),
+                      (const short*)vcache.data_ptr(), (short*)out.data_ptr(),
+                      P.pos, P.lens, P.slots, P.temp, P.r1, P.r2, P.sinks,
+                      P.scale, P.softcap, (int)B, (int)T, Bc, Hq, Hkv, Smax, D,
+                      DV, std::max(0, P.window), P.out_ld))
+    return;
+  // other bf16 prompts: matrix-core kernel (head sizes padded to its tile classes)
   if (!f32 && T >= 16 && D % 8 == 0 && DV % 8 == 0) {
     const dim3 mgrid((unsigned)((T + 63) / 64), (unsigned)Hq, (unsigned)B);
 #define AM_W(DCC, NVV, WW)                                                   \

@@ -29,6 +29,8 @@
 // us; 1500 tokens x 64 heads of 64 201 -> 47 us. Before: 16x16 tiles, weights
 // and transposed V through LDS, one query head per workgroup, loads not
 // overlapped. Error against 64 bits unchanged (weights are bf16 in both).
+// With changed scores (MOD; 3 more transcendental functions per score): 5
+// prompts of 1023 tokens x 32 heads of 128 773 -> 129 us.
 #include "common.h"
 
 namespace dnet {
@@ -46,14 +48,23 @@ struct Strides {             // elements; the last axis is contiguous
   int64_t b, h, t;
 };
 
-template <int D, int DV, bool WINDOW>
+// Scores changed before the softmax (MOD): factor per head, tanh cap,
+// logarithmic distance penalty; rows at their own positions, slots and lengths
+struct Mod {
+  const int *pos, *lens, *slots;             // [B]; lens, slots or null
+  const float *temp, *r1, *r2, *sinks;       // [Hq] or null
+  float scale, softcap;
+  int Bc;
+};
+
+template <int D, int DV, bool WINDOW, bool MOD>
 __global__ __launch_bounds__(256, D == 192 ? 1 : 2) void attn_prefill_kernel(
     const short* __restrict__ q, const short* __restrict__ k,
     const short* __restrict__ v, const short* __restrict__ sinks,
     short* __restrict__ out, const Strides qs, const Strides ks,
     const Strides vs, const Strides os, const int G, const int Hkv,
-    const int T, const int S, const int tiles, const int q_off,
-    const int window, const float scale2, const bool flip) {
+    const int T, const int S, const int tiles, const int q_off0,
+    const int window, const float scale2, const bool flip, const Mod md) {
   constexpr int NC = D / 16;                 // contraction steps of the scores
   constexpr int NV = DV / 32;                // 32-dim blocks of the values
   constexpr int KP = D + 8;
@@ -70,8 +81,11 @@ __global__ __launch_bounds__(256, D == 192 ? 1 : 2) void attn_prefill_kernel(
   const int lane = threadIdx.x & 63;
   const int c = lane & 31;
   const int hi = lane >> 5;
-  const int rows = T * G;
+  const int rows = (MOD && md.lens != nullptr ? min(md.lens[b], T) : T) * G;
   const int r0 = tile * kRows;
+  const int slot = MOD && md.slots != nullptr ? md.slots[b] : b;
+  if (MOD && (r0 >= rows || slot < 0 || slot >= md.Bc)) return;
+  const int q_off = MOD ? md.pos[b] : q_off0;
   const int row = min(r0 + wave * 32 + c, rows - 1);
   const int t = row / G, g = row % G;
   const int qpos = q_off + t;
@@ -92,8 +106,19 @@ __global__ __launch_bounds__(256, D == 192 ? 1 : 2) void attn_prefill_kernel(
   for (int i = 0; i < NC; ++i)
     qf[i] = *reinterpret_cast<const bf16x8*>(&qp[i * 16 + hi * 8]);
 
-  const short* kb = k + b * ks.b + hkv * ks.h;
-  const short* vb = v + b * vs.b + hkv * vs.h;
+  const short* kb = k + slot * ks.b + hkv * ks.h;
+  const short* vb = v + slot * vs.b + hkv * vs.h;
+  // this lane's head; the cap's exponential takes 2 log2(e) x / cap
+  float factor = 0.f, r1 = 0.f, r2 = 0.f, cap_in = 0.f;
+  if constexpr (MOD) {
+    const int h = hkv * G + g;
+    factor = md.scale * (md.temp != nullptr ? md.temp[h] : 1.f);
+    if (md.softcap > 0.f) cap_in = factor * (2.f * 1.44269504f) / md.softcap;
+    if (md.r1 != nullptr) {
+      r1 = md.r1[h] * 0.69314718f;           // of a base 2 logarithm
+      r2 = md.r2[h];
+    }
+  }
   u32x4 kr[KL], vr[VL];
   // positions past the end repeat the last one: in range and finite, masked
   auto load = [&](const int kt) {
@@ -150,13 +175,41 @@ __global__ __launch_bounds__(256, D == 192 ? 1 : 2) void attn_prefill_kernel(
     // the branch below stands between the products and the first read of
     // their results: past the products' latency in any case
     asm volatile("s_nop 15\n\ts_nop 3" : "+v"(s[0]), "+v"(s[1]));
-    if (flip) {
+    if (!MOD && flip) {
       s[0] = -s[0];
       s[1] = -s[1];
     }
     // position of result r of half h: kt * 64 + h * 32 + r / 4 * 8 + hi * 4 +
     // r % 4
     const int k0 = kt * kKeys;
+    if constexpr (MOD) {
+      if (md.softcap > 0.f) {
+        // cap * tanh(x / cap) = cap - 2 cap / (e^(2 x / cap) + 1)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            s[h][r] = fmaf(-2.f * md.softcap,
+                           __builtin_amdgcn_rcpf(
+                               __builtin_amdgcn_exp2f(s[h][r] * cap_in) + 1.f),
+                           md.softcap);
+      } else {
+        s[0] *= factor;
+        s[1] *= factor;
+      }
+      if (md.r1 != nullptr) {
+        const float back = (float)(qpos - k0 - hi * 4);   // exact
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            s[h][r] = fmaf(-r1,
+                           __builtin_amdgcn_logf(fmaf(
+                               r2, fmaxf(back - (h * 32 + r / 4 * 8 + r % 4),
+                                         0.f), 1.f)),
+                           s[h][r]);
+      }
+    }
     const bool whole = k0 + kKeys - 1 <= whole_end && k0 + kKeys <= S &&
                        (!WINDOW || k0 > last - window);
     if (!whole) {
@@ -220,9 +273,10 @@ __global__ __launch_bounds__(256, D == 192 ? 1 : 2) void attn_prefill_kernel(
   l += __shfl_xor(l, 32, 64);
   if (r0 + wave * 32 + c >= rows) return;
   float f = 1.f;
-  if (sinks != nullptr) {
+  if (MOD ? md.sinks != nullptr : sinks != nullptr) {
     // one extra logit per head whose mass has no value
-    const float sk = bits2f(sinks[hkv * G + g]) * 1.44269504f;
+    const float sk = 1.44269504f * (MOD ? md.sinks[hkv * G + g]
+                                        : bits2f(sinks[hkv * G + g]));
     const float m2 = fmaxf(m, sk);
     f = __builtin_amdgcn_exp2f(m - m2);
     l = l * f + __builtin_amdgcn_exp2f(sk - m2);
@@ -279,11 +333,13 @@ void attn_prefill(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   const float scale2 =
       (float)(std::max(std::abs(scale), 1e-30) * 1.4426950408889634);
 #define LAUNCH_AP(DD, DDV, WW)                                               \
-  hipLaunchKernelGGL((attn_prefill_kernel<DD, DDV, WW>), grid, dim3(256), 0, \
-                     current_stream(), (const short*)q.data_ptr(),           \
+  hipLaunchKernelGGL((attn_prefill_kernel<DD, DDV, WW, false>), grid,        \
+                     dim3(256), 0, current_stream(),                         \
+                     (const short*)q.data_ptr(),                             \
                      (const short*)k.data_ptr(), (const short*)v.data_ptr(), \
                      sp, (short*)out.data_ptr(), qs, ks, vs, os, G, Hkv, T,  \
-                     S, tiles, (int)q_off, (int)window, scale2, scale < 0)
+                     S, tiles, (int)q_off, (int)window, scale2, scale < 0,   \
+                     Mod{})
 #define LAUNCH_AP_W(DD, DDV)                \
   do {                                      \
     if (window > 0) LAUNCH_AP(DD, DDV, true); \
@@ -296,6 +352,45 @@ void attn_prefill(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   else DNET_CHECK(false, "attn_prefill: unsupported head dims");
 #undef LAUNCH_AP
 #undef LAUNCH_AP_W
+}
+
+// The prompts of attn_mod that have only the modifiers of Mod and a window: q
+// [B T, Hq D], caches [Bc, Hkv, Smax, D], out rows out_ld apart. Returns false
+// (nothing launched) for other head sizes and for rows off 16 B boundaries.
+bool attn_prompt_mod(const short* q, const short* k, const short* v, short* out,
+                     const int* pos, const int* lens, const int* slots,
+                     const float* temp, const float* r1, const float* r2,
+                     const float* sinks, float scale, float softcap, int B,
+                     int T, int Bc, int Hq, int Hkv, int Smax, int D, int DV,
+                     int window, int64_t out_ld) {
+  const int G = Hq / Hkv;
+  if (D != DV || (D != 64 && D != 96 && D != 128) || Smax < 1 ||
+      (uintptr_t)q % 16 || (uintptr_t)k % 16 || (uintptr_t)v % 16 ||
+      (uintptr_t)out % 8 || out_ld % 4 || (int64_t)T * G >= (1ll << 30))
+    return false;
+  const int tiles = cdiv((int64_t)T * G, kRows);
+  if ((int64_t)tiles * Hkv * B >= (1ll << 31)) return false;
+  const Strides qs{(int64_t)T * Hq * D, D, (int64_t)Hq * D};
+  const Strides cs{(int64_t)Hkv * Smax * D, (int64_t)Smax * D, D};
+  const Strides os{(int64_t)T * out_ld, DV, out_ld};
+  const Mod md{pos, lens, slots, temp, r1, r2, sinks, scale, softcap, Bc};
+#define LAUNCH_PM(DD, WW)                                                    \
+  hipLaunchKernelGGL((attn_prefill_kernel<DD, DD, WW, true>),                \
+                     dim3((unsigned)(tiles * Hkv * B)), dim3(256), 0,        \
+                     current_stream(), q, k, v, (const short*)nullptr, out,  \
+                     qs, cs, cs, os, G, Hkv, T, Smax, tiles, 0, window,      \
+                     1.44269504f, false, md)
+#define LAUNCH_PM_W(DD)               \
+  do {                                \
+    if (window > 0) LAUNCH_PM(DD, true); \
+    else LAUNCH_PM(DD, false);        \
+  } while (0)
+  if (D == 128) LAUNCH_PM_W(128);
+  else if (D == 96) LAUNCH_PM_W(96);
+  else LAUNCH_PM_W(64);
+#undef LAUNCH_PM
+#undef LAUNCH_PM_W
+  return true;
 }
 
 }  // namespace dnet

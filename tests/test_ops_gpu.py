@@ -1308,3 +1308,64 @@ def test_moe_prompt_takes_only_what_it_holds():
     assert not takes(e=129)
     assert not takes(quant=QuantConfig(4, 128))
     assert not takes(entries=10 ** 7)
+
+
+@pytest.mark.parametrize("d,G,T,window,mods,ld", [
+    (128, 4, 16, 0, True, 0),       # fewer rows than a tile
+    (128, 1, 129, 0, True, 0),      # one row over a tile
+    (128, 3, 97, 40, True, 64),     # out is a column range, heads not a power
+    (64, 2, 200, 0, False, 0),
+    (64, 8, 70, 65, True, 0),
+    (96, 4, 33, 0, True, 4),
+])
+def test_attn_mod_prompt(d, G, T, window, mods, ld):
+    """Prompts with changed scores on the prompt kernel, against fp64: ragged
+    and empty rows, a row without a slot, positions up to the cache's end.
+    Weights are rounded to bf16 as is the result (2^-8 each); a score's fp32
+    sum and its modifiers are within 2^-13 here (|score| below 16), which moves
+    a weight and the total by twice that."""
+    torch.manual_seed(T + d)
+    dev, hkv, smax, ns = _dev(), 2, 300, 5
+    hq, scale, cap = hkv * G, d ** -0.5, 4.0 if mods else 0.0
+    pos0, lens = [0, 37, smax - T, 5], [T, T // 2, T, 0]
+    slots = [3, 0, 4, -1]
+    B = 4
+    bf = lambda *n: torch.randn(*n, device=dev).to(torch.bfloat16)
+    q, kc, vc = bf(B * T, hq * d), bf(ns, hkv, smax, d), bf(ns, hkv, smax, d)
+    f = lambda lo, hi: (lo + (hi - lo) * torch.rand(hq, device=dev)
+                        if mods else None)
+    temp, r1, r2, sinks = f(0.5, 1.5), f(0.0, 1.0), f(0.0, 0.2), f(-1.0, 2.0)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    wide = torch.full((B * T, hq * d + ld), 7.0, dtype=torch.bfloat16,
+                      device=dev)
+    got = ops.attn_mod(q, kc, vc, i32(pos0), T, scale, i32(lens), i32(slots),
+                       temp=temp, softcap=cap, dist_r1=r1, dist_r2=r2,
+                       sinks=sinks, window=window, out=wide[:, :hq * d])
+    assert (wide[:, hq * d:] == 7).all()
+    got = got.double().cpu().view(B, T, hq, d)
+    c = lambda t: t.double().cpu().view(-1, 1, 1)
+    for b in range(B):
+        n = lens[b] if slots[b] >= 0 else 0
+        assert (got[b, n:] == 7).all()
+        if n == 0:
+            continue
+        qq = q.double().cpu().view(B, T, hq, d)[b, :n].transpose(0, 1)
+        k, v = (t[slots[b]].double().cpu().repeat_interleave(G, 0)
+                for t in (kc, vc))
+        s = qq @ k.transpose(1, 2) * scale * (c(temp) if mods else 1.0)
+        i = torch.arange(pos0[b], pos0[b] + n).view(-1, 1)
+        j = torch.arange(smax).view(1, -1)
+        if mods:
+            s = cap * torch.tanh(s / cap)
+            s = s - c(r1) * torch.log(1 + c(r2) * (i - j).clamp(min=0))
+        dead = (j > i) | ((j <= i - window) if window else (j < 0))
+        s = s.masked_fill(dead, float("-inf"))
+        if mods:
+            p = torch.softmax(torch.cat(
+                [s, c(sinks).expand(hq, n, 1)], -1), -1)[..., :-1]
+        else:
+            p = torch.softmax(s, -1)
+        want, mass = p @ v, p @ v.abs()
+        bound = (want.abs() + mass) * 2 ** -8 + mass * 2 ** -11
+        err = (got[b, :n].transpose(0, 1) - want).abs()
+        assert (err <= bound).all()
